@@ -229,12 +229,72 @@ void pack_device_profile(const std::vector<double> &hp, int n, std::vector<doubl
 {
     static const int rows[mt::PR_N] = {FWI3D_P_ESIG, FWI3D_P_MSIG, FWI3D_P_BE, FWI3D_P_BH,
                                        FWI3D_P_CE,   FWI3D_P_CH,   FWI3D_P_KED, FWI3D_P_KHD};
-    dp.assign((size_t)mt::PR_N * n, 0.0);
+    // rows, then the records of the per-cell kernels (CQ_N doubles per index);
+    // the range flags (axis_flags) take the rest
+    dp.assign((size_t)(mt::PR_N + mt::CQ_N) * n + (n + 1) / 2, 0.0);
     for (int r = 0; r < mt::PR_N; ++r)
         std::memcpy(&dp[(size_t)r * n], &hp[(size_t)rows[r] * n], sizeof(double) * n);
+    static const int rec[mt::CQ_N] = {FWI3D_P_ESIG, FWI3D_P_KED, FWI3D_P_BE, FWI3D_P_CE,
+                                      FWI3D_P_MSIG, FWI3D_P_KHD, FWI3D_P_BH, FWI3D_P_CH};
+    for (int i = 0; i < n; ++i)
+        for (int q = 0; q < mt::CQ_N; ++q)
+            dp[(size_t)mt::PR_N * n + (size_t)i * mt::CQ_N + q] = hp[(size_t)rec[q] * n + i];
+}
+
+// Range flags (mt::FL_*) of index r on axis a of n cells: the condition on this
+// axis of every update and CPML range of the C reference
+// (satan_i/fwi3d_cpu_function_v1.4.c:1195-1290, fwi3d_cpu_cpmlabc_v1.4.c:402-679).
+int axis_flags(int a, int r, int n, int nc)
+{
+    int f = 0;
+    for (int d = 0; d < 3; ++d) {   // component d updates; face of axis d
+        const bool own = a == d;
+        if (own ? r >= 1 && r < n - 1 : r >= 2 && r < n - 1)
+            f |= mt::FL_UEX << d;
+        if (own ? r >= 1 && r < n - 1 : r >= 1 && r < n - 2)
+            f |= mt::FL_UHX << d;
+        const int e1 = d == 0 ? nc - 1 : nc;
+        if (own ? (r >= 2 && r < e1) || (r >= n - nc + 1 && r < n - 2) : r < n - 1)
+            f |= mt::FL_PEX << d;
+        if (own ? (r >= 1 && r < nc - 1) || (r >= n - nc && r < n - 2) : r < n - 1)
+            f |= mt::FL_PHX << d;
+    }
+    if (r >= nc && r < n - nc)
+        f |= mt::FL_IN;
+    return f;
+}
+
+// q / d as (q * mul) >> sh for q < 2^31: mul = ceil(2^sh / d), sh = 31 +
+// ceil(log2 d), so mul < 2^32 and mul d - 2^sh < d <= 2^(sh - 31)
+void magic_div(unsigned d, unsigned &mul, int &sh)
+{
+    int l = 0;
+    while ((1ull << l) < d)
+        ++l;
+    sh = 31 + l;
+    mul = (unsigned)(((1ull << sh) + d - 1) / d);
 }
 
 int tiles(int n, int t) { return (n + t - 1) / t; }
+
+// Tile w x h of the per-cell kernels on planes of ix x iy cells: the shape with
+// the fewest idle lanes and halo loads (6 (w + h) values per tile), rows of at
+// least 16 cells (128 B).
+void cell_tile(int ix, int iy, int &w, int &h)
+{
+    double best = 0.0;
+    for (int cw = 16; cw <= mt::PT_WH - 4; ++cw) {
+        const int ch = std::min(mt::PT / cw, mt::PT_WH - cw);
+        if ((cw + 3) * (ch + 3) > mt::PT_TILE)
+            continue;
+        const double cost = (double)tiles(ix, cw) * tiles(iy, ch) * (mt::PT + (cw + ch));
+        if (best == 0.0 || cost < best) {
+            best = cost;
+            w = cw;
+            h = ch;
+        }
+    }
+}
 
 // Tiles {x0, y0, k, yend} of the per-cell kernels around an LDS region [lo, hi):
 // planes outside the region and rows of 32 x 8 tiles not inside it in y get
@@ -512,8 +572,8 @@ int launch_eh(const Fam &f, const ShotDev *d, int ns, int j, bool h, hipStream_t
         e = h ? mt::launch_hfield_p(d, ns, f.pre, f.nblocks, j, 1, st)
               : mt::launch_efield_p(d, ns, f.pre, f.nblocks, j, 1, st);
     else
-        e = h ? mt::launch_hfield_f(d, ns, f.pre, f.nblocks, j, 1, st, f.fused, f.nt)
-              : mt::launch_efield_f(d, ns, f.pre, f.nblocks, j, 1, st, rec_prev, f.fused, f.nt);
+        e = h ? mt::launch_hfield_f(d, ns, f.pre, f.nblocks, j, st, f.fused, f.nt)
+              : mt::launch_efield_f(d, ns, f.pre, f.nblocks, j, st, rec_prev, f.fused, f.nt);
     HIP_TRY(e);
     if (f.kind == 3 && f.fused) {
         if (!h)
@@ -656,6 +716,9 @@ int fwi3d_model_create_variant(const fwi3d_grid_params *p, int variant, void *st
         std::vector<double> dp;
         const int n = axis_len(*p, a);
         pack_device_profile(m->prof[a], n, dp);
+        int *fl = reinterpret_cast<int *>(&dp[(size_t)(mt::PR_N + mt::CQ_N) * n]);
+        for (int r = 0; r < n; ++r)
+            fl[r] = axis_flags(a, r, n, p->ncpml);
         if (dalloc(&m->d_prof[a], dp.size()) != hipSuccess ||
             hcopy(m->d_prof[a], dp.data(), sizeof(double) * dp.size()) !=
                 hipSuccess) {
@@ -909,10 +972,26 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.iz = p.iz;
     d.nc = p.ncpml;
     d.n = (int)N;
-    d.nbx = tiles(p.ix, mt::TX);
-    d.nby = tiles(p.iy, mt::TY);
+    d.row = 8u * (unsigned)p.ix;
+    d.pb = 8u * (unsigned)(p.ix * p.iy);
+    cell_tile(p.ix, p.iy, d.tw, d.th);
+    d.ttx = tiles(p.ix, d.tw);
+    d.tpp = d.ttx * tiles(p.iy, d.th);
+    magic_div((unsigned)d.ttx, d.xmul, d.xsh);
+    magic_div((unsigned)d.tpp, d.tmul, d.tsh);
+    d.opp = tiles(p.ix * p.iy, mt::PT);
+    magic_div((unsigned)d.opp, d.omul, d.osh);
+    magic_div((unsigned)p.ix, d.imul, d.ish);
+    d.op_pad = tiles(d.opp * p.iz, 8) * 8;
+    d.src_k = -1;
+    d.src_o = 0;
+    if (s->src_cell >= 0) {
+        d.src_k = sp->src_k;
+        d.src_o = 8u * (unsigned)(sp->src_j * p.ix + sp->src_i);
+    }
     d.it = sp->it;
     d.dt = p.dt;
+    d.dtm = p.dt / p.mu0;
     d.omega0 = p.omega0;
     d.mu0 = p.mu0;
     d.c1 = p.c1;
@@ -921,7 +1000,10 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.dl[1] = p.dy;
     d.dl[2] = p.dz;
     for (int a = 0; a < 3; ++a) {
+        const size_t na = (size_t)axis_len(p, a);
         d.prof[a] = m->d_prof[a];
+        d.cq[a] = m->d_prof[a] + mt::PR_N * na;
+        d.fl[a] = reinterpret_cast<const int *>(d.cq[a] + mt::CQ_N * na);
         d.psi[a] = s->d_psi[a];
         d.slab[a] = (long long)slab[a];
     }
@@ -938,7 +1020,7 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.pair = (p.ix % 2 == 0 && env_pad("MITTET_FDTD_PAIR", 0)) ? 1 : 0;
     d.ftx = d.pair ? tiles(p.ix, 32) : tiles(p.ix, mt::ZX);
     d.fty = d.pair ? tiles(p.iy, 16) : tiles(p.iy, mt::ZY);
-    d.fb = d.ftx * d.fty * p.iz;
+    d.fb = d.pair ? d.ftx * d.fty * p.iz : d.tpp * p.iz;
     d.fb_pad = tiles(d.fb, 8) * 8;
     d.e = s->d_e;
     d.sstride = sstride;
@@ -966,7 +1048,7 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.nsrc_h = (int)s->src_h.size();
     for (int q = 0; q < d.nsrc_h; ++q)
         d.src_h[q] = s->src_h[q];
-    s->nblocks_op = d.nbx * d.nby * p.iz;
+    s->nblocks_op = d.op_pad;
     s->kind = sp->zchunk > 0 ? 2 : d.pair;
     if (magnetic) {
         // every 32 x 8 tile, one cell per lane (fdtd_fortran.hip)
@@ -1138,20 +1220,16 @@ static int single_op(fwi3d_shot *s, int which, int sign, int step)
         return fail(FWI3D_EINVAL, "sign must be +1 or -1");
     switch (which) {
     case 0:
-        HIP_TRY(mt::launch_efield(mt::M_UPD | mt::M_INPLACE, s->d_desc, 1, s->d_pre, s->nblocks_op, 0,
-                                  0, sign, s->st));
+        HIP_TRY(mt::launch_efield(mt::M_UPD | mt::M_INPLACE, s->d_desc, s->nblocks_op, sign, s->st));
         break;
     case 1:
-        HIP_TRY(mt::launch_efield(mt::M_PSI | mt::M_INPLACE, s->d_desc, 1, s->d_pre, s->nblocks_op, 0,
-                                  0, 1, s->st));
+        HIP_TRY(mt::launch_efield(mt::M_PSI | mt::M_INPLACE, s->d_desc, s->nblocks_op, 1, s->st));
         break;
     case 2:
-        HIP_TRY(mt::launch_hfield(mt::M_UPD | mt::M_INPLACE, s->d_desc, 1, s->d_pre, s->nblocks_op, 0,
-                                  sign, s->st));
+        HIP_TRY(mt::launch_hfield(mt::M_UPD | mt::M_INPLACE, s->d_desc, s->nblocks_op, sign, s->st));
         break;
     case 3:
-        HIP_TRY(mt::launch_hfield(mt::M_PSI | mt::M_INPLACE, s->d_desc, 1, s->d_pre, s->nblocks_op, 0,
-                                  1, s->st));
+        HIP_TRY(mt::launch_hfield(mt::M_PSI | mt::M_INPLACE, s->d_desc, s->nblocks_op, 1, s->st));
         break;
     case 4:
         if (step < 0 || step >= s->it - 1)

@@ -10,11 +10,27 @@ namespace mt {
 // Packed per-axis 1-D CPML profile rows on the device: prof[a][row * n_a + idx].
 enum { PR_ESIG = 0, PR_MSIG, PR_BE, PR_BH, PR_CE, PR_CH, PR_KED, PR_KHD, PR_N };
 
+// After the rows of an axis: its profiles again as one record of CQ_N doubles
+// per index (E then H: sigma, kappa*dl, b, c), so that a cell reads an axis'
+// four values with two 16-byte loads, then one word of range flags per index.
+enum { CQ_E = 0, CQ_H = 4, CQ_N = 8 };
+// Range flags of the update and CPML ranges.  A cell is in a range where the
+// words of its three indices all have the range's bit.
+enum {
+    FL_UEX = 1, FL_UEY = 2, FL_UEZ = 4,          // E updates
+    FL_PEX = 8, FL_PEY = 16, FL_PEZ = 32,        // CPML-E faces of the x, y, z axis
+    FL_UHX = 64, FL_UHY = 128, FL_UHZ = 256,     // H updates
+    FL_PHX = 512, FL_PHY = 1024, FL_PHZ = 2048,  // CPML-H faces
+    FL_IN = 4096                                 // outside every CPML shell
+};
+
 // psi arrays per axis: slab arrays of [0,nc) U [n-nc,n) along the axis.
 enum { PSI_EP = 0, PSI_EM, PSI_HP, PSI_HM, PSI_N };
 
-constexpr int TX = 64;   // threads along x (one wavefront row, 512 B coalesced)
-constexpr int TY = 4;    // rows per block
+constexpr int PT = 256;  // threads and most cells of a per-cell block
+// Tiles of the per-cell kernels: 6 (w + h) halo values fit one load per lane
+// (w + h <= PT_WH), and a component's tile with its halo fits PT_TILE doubles.
+constexpr int PT_WH = 42, PT_TILE = 400;
 // E ring slots: the volume DFT reads each slot once per `ring` steps, so it
 // costs 24 + 768/ring bytes per cell and step at 8 frequencies
 constexpr int RING_MAX = 256;
@@ -36,46 +52,62 @@ constexpr int LX = 64, LY = MT_LY, LKB = MT_LKB;
 
 // Everything a kernel needs about one shot.  Lives in device memory; blocks
 // find their shot through an exclusive prefix of per-shot block counts.
-struct ShotDev {
+struct alignas(64) ShotDev {
+    // the first cache lines are what a per-cell block needs first
     int ix, iy, iz, nc;
+    unsigned row, pb;         // bytes of a row and of a plane of one array
+    int tw, th;               // tiles of the per-cell kernels: tw x th <= PT cells of a plane
+    int ttx, tpp;             // tiles along x, tiles per plane
+    unsigned xmul, tmul;      // division by ttx and tpp: (q * mul) >> sh (see magic_div)
+    int xsh, tsh;
+    int fb, fb_pad;           // per-cell blocks (one tile each), padded to 8
     int n;                    // cells
-    int nbx, nby;             // xy tiles
-    int it;                   // samples; steps 0 .. it-2 exist
-    double dt, omega0, mu0, c1, c2;
-    double dl[3];
-    const double *prof[3];    // [PR_N][n_a]
-    const double *eps;        // eps' = sigma/2/omega0 per cell
-    const double *cbi;        // dt/eps' per cell (cb where the CPML sigma is zero)
-    int kb;                   // z-chunk length of the z-marching kernels
-    int ztx, zty, nkz;        // z-marching tiles along x, y and z-chunks
-    int zb, zb_pad;           // z-marching blocks, padded to a multiple of 8
-    int fb, fb_pad;           // per-cell fused blocks (one plane each), padded to 8
-    int ftx, fty;             // per-cell fused tiles along x and y
-    int pair;                 // 1: fused kernels update x-pairs of cells (even ix)
-    const int4 *shell;        // tiles of the per-cell kernels when the LDS kernels cover the
-                              // interior: {x0, y0, k, yend} (yend 0: a 32 x 8 tile; else a
-                              // 16 x 16 tile with rows below yend), fb entries then k = -1
-                              // padding; null: every 32 x 8 tile
-    int lo[3], hi[3];         // LDS-kernel region [lo, hi) per axis (inside the CPML-free interior)
-    int ltx, lty, lkz;        // LDS-kernel tiles along x, y and z-chunks
-    int lkb;                  // LDS-kernel z-chunk length (planes)
-    int lb, lb_pad;           // LDS-kernel blocks, padded to a multiple of 8
+    int ring, cur;            // ring slots; slot that holds E at chunk start
+    int hpar;                 // 1: the current H lives in h2
     double *e;                // E ring: slot q, comp d at e + q*sstride + d*n
     long long sstride;        // doubles between ring slots (3n + padding)
-    long long astride;        // complex elements between accumulator rows (n + padding)
-    int ring, cur;            // ring slots; slot that holds E at chunk start
     double *h;                // H [3][n]: updated in place, except by the fused E+H
                               // launches (see hsel)
     double *h2;               // second H buffer of shots that run the fused E+H interior
                               // kernel (null: none)
-    int hpar;                 // 1: the current H lives in h2
     long long hstride;        // nonzero: H in ring slots like E (slot q at h + q*hstride;
                               // a gradient replay's stored states), see hsel
+    const int4 *shell;        // tiles of the per-cell kernels when the LDS kernels cover the
+                              // interior: {x0, y0, k, yend} (yend 0: a 32 x 8 tile; else a
+                              // 16 x 16 tile with rows below yend), fb entries then k = -1
+                              // padding; null: every tw x th tile of every plane
+    const double *eps;        // eps' = sigma/2/omega0 per cell
+    const double *cbi;        // dt/eps' per cell (cb where the CPML sigma is zero)
     double *psi[3];           // [PSI_N][slab[a]]
     long long pstride;        // nonzero: psi in ring slots like E (slot q at psi[a] + q*pstride;
                               // a gradient replay's stored states), read and written by the
                               // per-cell code only
+    int *step;                // absolute step of local index j = 0 of the current chunk
+    int src_k;                // plane of the source cell (-1: no source) ...
+    unsigned src_o;           // ... and its byte offset there
     long long slab[3];
+    const double *prof[3];    // [PR_N][n_a]
+    const double *cq[3];      // [n_a][CQ_N]
+    const int *fl[3];         // [n_a] range flags
+    double dt, omega0, mu0, c1, c2;
+    double dtm;               // dt/mu0
+    double dl[3];
+    int lo[3], hi[3];         // LDS-kernel region [lo, hi) per axis (inside the CPML-free interior)
+    int it;                   // samples; steps 0 .. it-2 exist
+    int opp, osh;             // stand-alone operators: PT-cell runs of a plane, division by it
+    unsigned omul, imul;      // ... and by ix
+    int ish;
+    int op_pad;               // their blocks, padded to 8
+    int kb;                   // z-chunk length of the z-marching kernels
+    int ztx, zty, nkz;        // z-marching tiles along x, y and z-chunks
+    int zb, zb_pad;           // z-marching blocks, padded to a multiple of 8
+    int ftx, fty;             // 32 x 8 (pair: 32 x 16) tiles along x and y of the pair and
+                              // Fortran kernels
+    int pair;                 // 1: fused kernels update x-pairs of cells (even ix)
+    int ltx, lty, lkz;        // LDS-kernel tiles along x, y and z-chunks
+    int lkb;                  // LDS-kernel z-chunk length (planes)
+    int lb, lb_pad;           // LDS-kernel blocks, padded to a multiple of 8
+    long long astride;        // complex elements between accumulator rows (n + padding)
     int src_comp;
     int src_cell;             // -1: no source
     const double *amp;        // [it-1] source decrement per step
@@ -87,7 +119,6 @@ struct ShotDev {
     double *acc;              // complex [3][nf] rows of astride
     double *acc_h;            // H volume spectra, same layout (null: off)
     double *hring;            // with acc_h: H after each step, ring slots like e
-    int *step;                // absolute step of local index j = 0 of the current chunk
     int *flag;                // set to 1 once a gathered sample or the source cell's field
                               // turns NaN or infinite (divergence probe)
     int variant;              // 0: C v1.4 semantics; 1: Fortran ver0040 (fdtd_fortran.hip)
@@ -151,10 +182,8 @@ hipError_t launch_adjoint_step(const AdjArgs &A, const double *g, int nrec, cons
 
 // Kernel launchers (fdtd_kernels.hip).  `pre` is the exclusive prefix of
 // per-shot block counts (device), `nblocks` its total.
-hipError_t launch_efield(int mode, const ShotDev *d, int ns, const int *pre, int nblocks,
-                         int j, int nover, int sign, hipStream_t st);
-hipError_t launch_hfield(int mode, const ShotDev *d, int ns, const int *pre, int nblocks,
-                         int j, int sign, hipStream_t st);
+hipError_t launch_efield(int mode, const ShotDev *d, int nblocks, int sign, hipStream_t st);
+hipError_t launch_hfield(int mode, const ShotDev *d, int nblocks, int sign, hipStream_t st);
 hipError_t launch_source(const ShotDev *d, int n, hipStream_t st);
 hipError_t launch_efield_z(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                            int sign, hipStream_t st);
@@ -165,10 +194,9 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // hsel(S, j + 1, 1)); 0: H updated in place.  nt (also for the _l launches):
 // the once-touched field values go non-temporal (M_NT).
 hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           int sign, hipStream_t st, bool rec_prev = false, int hf = 0,
-                           bool nt = false);
+                           hipStream_t st, bool rec_prev = false, int hf = 0, bool nt = false);
 hipError_t launch_hfield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           int sign, hipStream_t st, int hf = 0, bool nt = false);
+                           hipStream_t st, int hf = 0, bool nt = false);
 hipError_t launch_efield_p(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                            int sign, hipStream_t st);
 hipError_t launch_hfield_p(const ShotDev *d, int ns, const int *pre, int nblocks, int j,

@@ -4,7 +4,7 @@
 // batches alike: every block looks its shot up in an exclusive prefix of
 // per-shot block counts, so shots of different grid sizes share one launch.
 //
-// E kernel (per cell, x fastest, 64x4 threads per block):
+// E kernel (per cell, x fastest):
 //   E-update of satan_i/fwi3d_cpu_function_v1.4.c:1184-1236, then the CPML-E
 //   corrections of satan_i/fwi3d_cpu_cpmlabc_v1.4.c:402-543 in the order
 //   x, y, z, then the source (function.c:514-529).  Coefficients
@@ -107,12 +107,89 @@ __device__ __forceinline__ double uload(const double *p)
     return *(const __attribute__((address_space(4))) double *)p;
 }
 
-// One cell of the E update + CPML-E corrections + source, general path.
-// Every load a cell needs is issued before the arithmetic that uses any of
-// them (the loads a flag does not ask for are skipped and their values left
-// zero), so a cell pays one memory round trip instead of one per branch.  The
-// arithmetic is the same expressions in the same order as one branch after the
-// other, so the result is unchanged to the bit.
+// Addresses of the per-cell kernels.  A block's cells lie in one plane, so every
+// access is a wave-uniform base (component and plane, scalar arithmetic) plus a
+// 32-bit byte offset within the plane: one scalar-base load instruction, no
+// 64-bit vector arithmetic per access.  A grid below 2^31 cells has at least 8
+// planes (two CPML shells of 2 cells and 4 more), so a plane is below 2^31
+// bytes.
+typedef const GLOBAL char *gcp;
+typedef GLOBAL char *gmp;
+__device__ __forceinline__ gcp cb(const void *p) { return (gcp)p; }
+__device__ __forceinline__ gmp mb(void *p) { return (gmp)p; }
+__device__ __forceinline__ double at(gcp b, unsigned o, int d = 0)
+{
+    return *(const GLOBAL double *)(b + o + d);
+}
+template <bool NT> __device__ __forceinline__ double at_s(gcp b, unsigned o)
+{
+    return ld_s<NT>((const GLOBAL double *)(b + o));
+}
+template <bool NT> __device__ __forceinline__ void put_s(gmp b, unsigned o, double v)
+{
+    st_s<NT>((GLOBAL double *)(b + o), v);
+}
+
+// ring slot q of a descriptor, q < 2 * ring (or any q when there is one slot)
+__device__ __forceinline__ int ring_slot(const ShotDev &S, int q)
+{
+    return S.ring == 1 ? 0 : (q >= S.ring ? q - S.ring : q);
+}
+
+// An axis' sigma, kappa*dl, b and c: of a lane's x or y index (rows, so that
+// neighbouring lanes read neighbouring words), or of one index for the whole
+// wave (a record, scalar loads)
+struct Quad {
+    double s, k, b, c;
+};
+template <bool H> __device__ __forceinline__ Quad quad(const double *prof, int n, int r)
+{
+    const gcp p = cb(prof);
+    const unsigned o = (unsigned)r * 8u, m = (unsigned)n * 8u;
+    return {at(p, o + m * (H ? PR_MSIG : PR_ESIG)), at(p, o + m * (H ? PR_KHD : PR_KED)),
+            at(p, o + m * (H ? PR_BH : PR_BE)), at(p, o + m * (H ? PR_CH : PR_CE))};
+}
+template <bool H> __device__ __forceinline__ Quad uquad(const double *cq, int r)
+{
+    const double *p = cq + (size_t)r * CQ_N + (H ? CQ_H : CQ_E);
+    return {uload(p), uload(p + 1), uload(p + 2), uload(p + 3)};
+}
+__device__ __forceinline__ int uload(const int *p)
+{
+    return *(const __attribute__((address_space(4))) int *)p;
+}
+// range flags of a cell
+__device__ __forceinline__ int flags(const ShotDev &S, int i, int jj, int k)
+{
+    const int fx = *(const GLOBAL int *)(cb(S.fl[0]) + (unsigned)(i * 4));
+    const int fy = *(const GLOBAL int *)(cb(S.fl[1]) + (unsigned)(jj * 4));
+    return fx & fy & uload(S.fl[2] + k);
+}
+
+// Byte offsets of a cell in its plane and of its x and y neighbours, clamped
+// into the plane: a clamped value reaches only results that the cell's range
+// flags discard.  x neighbours are at x + 8 d for d in [-LO, HI].
+template <int LO, int HI> struct Off {
+    unsigned o, ym1, ym2, yp1, yp2, x;
+    __device__ __forceinline__ Off(const ShotDev &S, unsigned oc)
+    {
+        const int row = (int)S.row, oi = (int)oc;
+        const unsigned last = S.pb - 8u;
+        o = oc;
+        ym1 = max(oi - row, 0);
+        ym2 = max(oi - 2 * row, 0);
+        yp1 = min(oc + S.row, last);
+        yp2 = min(oc + 2u * S.row, last);
+        x = min(max(oc, 8u * LO), last - 8u * HI);
+    }
+};
+
+// One cell of the E update + CPML-E corrections + source, general path (k is
+// the same for every lane; o: the cell's byte offset in its plane).  Every
+// load a cell needs is issued before the arithmetic that uses any of them, so
+// a cell pays one memory round trip instead of one per branch; the stencil
+// loads depend on no flag.  The arithmetic is the reference's expressions in
+// its order.
 __device__ __forceinline__ double dm(double f0, double fm1, double fp1, double fm2, double c1,
                                      double c2)
 {
@@ -121,129 +198,62 @@ __device__ __forceinline__ double dm(double f0, double fm1, double fp1, double f
 
 template <int MODE>
 __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, int i, int jj, int k,
-                                            int n, int si, int so, int sign)
+                                            unsigned oc, int fl, int n, int si, int so, int sign)
 {
-    constexpr bool NT = (MODE & M_NT) != 0;
-    const int ix = S.ix, iy = S.iy, iz = S.iz, nc = S.nc, N = S.n;
-    const int sy = ix, sz = ix * iy;
-    const int c = (k * iy + jj) * ix + i;
-
-    const GLOBAL double *__restrict__ Ein = gc(S.e + (size_t)si * S.sstride);
-    GLOBAL double *__restrict__ Eout = gm(S.e + (size_t)so * S.sstride);
-    const GLOBAL double *__restrict__ Hx = gc(H);
-    const GLOBAL double *__restrict__ Hy = gc(H + N);
-    const GLOBAL double *__restrict__ Hz = gc(H + 2 * (size_t)N);
-
-    const double c1 = S.c1, c2 = S.c2, dt = S.dt;
-    const GLOBAL double *__restrict__ px = gc(S.prof[0]);
-    const GLOBAL double *__restrict__ py = gc(S.prof[1]);
-    const GLOBAL double *__restrict__ pz = gc(S.prof[2]);
-
-    const bool rx1 = i >= 1 && i < ix - 1, rx2 = i >= 2 && i < ix - 1;
-    const bool ry1 = jj >= 1 && jj < iy - 1, ry2 = jj >= 2 && jj < iy - 1;
-    const bool rz1 = k >= 1 && k < iz - 1, rz2 = k >= 2 && k < iz - 1;
-    const bool upx = (MODE & M_UPD) && rx1 && ry2 && rz2;
-    const bool upy = (MODE & M_UPD) && rx2 && ry1 && rz2;
-    const bool upz = (MODE & M_UPD) && rx2 && ry2 && rz1;
-    // CPML-E faces: x [2,nc-1)U[ix-nc+1,ix-2); y,z [2,nc)U[n-nc+1,n-2)
-    const bool fx = (MODE & M_PSI) && ((i >= 2 && i < nc - 1) || (i >= ix - nc + 1 && i < ix - 2)) &&
-                    jj < iy - 1 && k < iz - 1;
-    const bool fy = (MODE & M_PSI) && ((jj >= 2 && jj < nc) || (jj >= iy - nc + 1 && jj < iy - 2)) &&
-                    i < ix - 1 && k < iz - 1;
-    const bool fz = (MODE & M_PSI) && ((k >= 2 && k < nc) || (k >= iz - nc + 1 && k < iz - 2)) &&
-                    i < ix - 1 && jj < iy - 1;
+    constexpr bool NT = (MODE & M_NT) != 0, UPD = (MODE & M_UPD) != 0, PSI = (MODE & M_PSI) != 0;
+    const bool upx = UPD && (fl & FL_UEX), upy = UPD && (fl & FL_UEY), upz = UPD && (fl & FL_UEZ);
+    const bool fx = PSI && (fl & FL_PEX), fy = PSI && (fl & FL_PEY), fz = PSI && (fl & FL_PEZ);
+    if (!UPD && !(fx || fy || fz))
+        return;   // the corrections alone, in place: nothing to add
+    const int nc = S.nc;
+    const size_t nb = (size_t)S.n * 8, pb = S.pb, kp = (size_t)k * pb;
 
     // ---- loads
-    double ex = ld_s<NT>(Ein + c), ey = ld_s<NT>(Ein + N + c), ez = ld_s<NT>(Ein + 2 * (size_t)N + c);
-    // every backward stencil in bounds: all six derivatives are loaded
-    const bool all = rx2 && ry2 && rz2;
-    const bool nzy = all || upx || fy, nyz = all || upx || fz, nxz = all || upy || fz;
-    const bool nzx = all || upy || fx, nyx = all || upz || fx, nxy = all || upz || fy;
-    double z0 = 0.0, zym1 = 0.0, zyp1 = 0.0, zym2 = 0.0, zxm1 = 0.0, zxp1 = 0.0, zxm2 = 0.0;
-    double y0 = 0.0, yzm1 = 0.0, yzp1 = 0.0, yzm2 = 0.0, yxm1 = 0.0, yxp1 = 0.0, yxm2 = 0.0;
-    double x0 = 0.0, xzm1 = 0.0, xzp1 = 0.0, xzm2 = 0.0, xym1 = 0.0, xyp1 = 0.0, xym2 = 0.0;
-    if (nzy || nzx)
-        z0 = Hz[c];
-    if (nzy) {
-        zym1 = Hz[c - sy];
-        zyp1 = Hz[c + sy];
-        zym2 = Hz[c - 2 * sy];
-    }
-    if (nzx) {
-        zxm1 = Hz[c - 1];
-        zxp1 = Hz[c + 1];
-        zxm2 = Hz[c - 2];
-    }
-    if (nyz || nyx)
-        y0 = Hy[c];
-    if (nyz) {
-        yzm1 = Hy[c - sz];
-        yzp1 = Hy[c + sz];
-        yzm2 = Hy[c - 2 * sz];
-    }
-    if (nyx) {
-        yxm1 = Hy[c - 1];
-        yxp1 = Hy[c + 1];
-        yxm2 = Hy[c - 2];
-    }
-    if (nxz || nxy)
-        x0 = Hx[c];
-    if (nxz) {
-        xzm1 = Hx[c - sz];
-        xzp1 = Hx[c + sz];
-        xzm2 = Hx[c - 2 * sz];
-    }
-    if (nxy) {
-        xym1 = Hx[c - sy];
-        xyp1 = Hx[c + sy];
-        xym2 = Hx[c - 2 * sy];
-    }
-    const double eps2 = gc(S.eps)[c];
-    const double sgx = px[PR_ESIG * ix + i], sgy = py[PR_ESIG * iy + jj], sgz = pz[PR_ESIG * iz + k];
-    double kx = 1.0, ky = 1.0, kz = 1.0;
-    if (MODE & M_UPD) {
-        kx = px[PR_KED * ix + i];
-        ky = py[PR_KED * iy + jj];
-        kz = pz[PR_KED * iz + k];
-    }
+    const Off<2, 1> q(S, oc);
+    const size_t zm1 = k >= 1 ? kp - pb : kp, zm2 = k >= 2 ? kp - 2 * pb : kp;
+    const size_t zp1 = k + 1 < S.iz ? kp + pb : kp;
+    const gcp Hb = cb(H), Hx = Hb + kp, Hy = Hb + nb + kp, Hz = Hb + 2 * nb + kp;
+    const gcp Ein = cb(S.e + (size_t)si * S.sstride) + kp;
+    const gmp Eout = mb(S.e + (size_t)so * S.sstride) + kp;
+    const double z0 = at(Hz, q.o), zym1 = at(Hz, q.ym1), zyp1 = at(Hz, q.yp1), zym2 = at(Hz, q.ym2);
+    const double zxm1 = at(Hz, q.x, -8), zxp1 = at(Hz, q.x, 8), zxm2 = at(Hz, q.x, -16);
+    const double y0 = at(Hy, q.o), yzm1 = at(Hb + nb + zm1, q.o), yzp1 = at(Hb + nb + zp1, q.o),
+                 yzm2 = at(Hb + nb + zm2, q.o);
+    const double yxm1 = at(Hy, q.x, -8), yxp1 = at(Hy, q.x, 8), yxm2 = at(Hy, q.x, -16);
+    const double x0 = at(Hx, q.o), xzm1 = at(Hb + zm1, q.o), xzp1 = at(Hb + zp1, q.o),
+                 xzm2 = at(Hb + zm2, q.o);
+    const double xym1 = at(Hx, q.ym1), xyp1 = at(Hx, q.yp1), xym2 = at(Hx, q.ym2);
+    double ex = at_s<NT>(Ein, q.o), ey = at_s<NT>(Ein + nb, q.o), ez = at_s<NT>(Ein + 2 * nb, q.o);
+    const double eps2 = at(cb(S.eps) + kp, q.o);
+    const Quad X = quad<false>(S.prof[0], S.ix, i), Y = quad<false>(S.prof[1], S.iy, jj);
+    const Quad Z = uquad<false>(S.cq[2], k);
     // psi in place, or (pstride set) read from ring slot si and written to
     // slot so like E
     const size_t pr = S.pstride ? (size_t)si * S.pstride : 0;
     const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
-    const GLOBAL double *Q0 = gc(S.psi[0] + pr), *Q1 = gc(S.psi[1] + pr), *Q2 = gc(S.psi[2] + pr);
-    GLOBAL double *P0 = gm(S.psi[0] + pw), *P1 = gm(S.psi[1] + pw), *P2 = gm(S.psi[2] + pw);
-    const size_t L0 = (size_t)S.slab[0], L1 = (size_t)S.slab[1], L2 = (size_t)S.slab[2];
-    size_t q0 = 0, q1 = 0, q2 = 0;
-    double bx = 0.0, cx = 0.0, ax0 = 0.0, ax1 = 0.0;
-    double by = 0.0, cy = 0.0, ay0 = 0.0, ay1 = 0.0;
-    double bz = 0.0, cz = 0.0, az0 = 0.0, az1 = 0.0;
+    const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
+    const size_t b0 = (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
+    const size_t b1 = (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
+    const size_t b2 = (size_t)(unsigned)slab_pos(k, S.iz, nc) * pb;   // k in a shell (fz) only
+    unsigned q0 = 0, q1 = 0;
+    double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, az0 = 0.0, az1 = 0.0;
     if (fx) {
-        q0 = ((size_t)k * iy + jj) * (2 * nc) + slab_pos(i, ix, nc);
-        bx = px[PR_BE * ix + i];
-        cx = px[PR_CE * ix + i];
-        ax0 = Q0[q0];
-        ax1 = Q0[L0 + q0];
+        q0 = (unsigned)(jj * (2 * nc) + slab_pos(i, S.ix, nc)) * 8u;
+        ax0 = at(cb(S.psi[0] + pr) + b0, q0);
+        ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
     }
     if (fy) {
-        q1 = ((size_t)k * (2 * nc) + slab_pos(jj, iy, nc)) * ix + i;
-        by = py[PR_BE * iy + jj];
-        cy = py[PR_CE * iy + jj];
-        ay0 = Q1[q1];
-        ay1 = Q1[L1 + q1];
+        q1 = (unsigned)(slab_pos(jj, S.iy, nc) * S.ix + i) * 8u;
+        ay0 = at(cb(S.psi[1] + pr) + b1, q1);
+        ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
     }
     if (fz) {
-        q2 = ((size_t)slab_pos(k, iz, nc) * iy + jj) * ix + i;
-        bz = pz[PR_BE * iz + k];
-        cz = pz[PR_CE * iz + k];
-        az0 = Q2[q2];
-        az1 = Q2[L2 + q2];
+        az0 = at(cb(S.psi[2] + pr) + b2, q.o);
+        az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
     }
-    const bool src = (MODE & M_SRC) && c == S.src_cell;
-    double amp = 0.0;
-    if (src)
-        amp = gc(S.amp)[n];
 
     // ---- arithmetic
+    const double c1 = S.c1, c2 = S.c2, dt = S.dt;
     const double hzy = dm(z0, zym1, zyp1, zym2, c1, c2);
     const double hyz = dm(y0, yzm1, yzp1, yzm2, c1, c2);
     const double hxz = dm(x0, xzm1, xzp1, xzm2, c1, c2);
@@ -256,33 +266,29 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
     // divisions are skipped there (most shell cells lie in one axis' CPML)
     const double dte = dt / eps2;
     double cax = 1.0, cay = 1.0, caz = 1.0, cbx = dte, cby = dte, cbz = dte;
-    if (sgx != 0.0) {
-        const double se = sgx * dt / (2.0 * eps2);
+    if (X.s != 0.0) {
+        const double se = X.s * dt / (2.0 * eps2);
         cbx = dte / (1.0 + se);
         cax = (1.0 - se) / (1.0 + se);
     }
-    if (sgy != 0.0) {
-        const double se = sgy * dt / (2.0 * eps2);
+    if (Y.s != 0.0) {
+        const double se = Y.s * dt / (2.0 * eps2);
         cby = dte / (1.0 + se);
         cay = (1.0 - se) / (1.0 + se);
     }
-    if (sgz != 0.0) {
-        const double se = sgz * dt / (2.0 * eps2);
+    if (Z.s != 0.0) {
+        const double se = Z.s * dt / (2.0 * eps2);
         cbz = dte / (1.0 + se);
         caz = (1.0 - se) / (1.0 + se);
     }
 
-    if (upx) {
-        const double cu = hzy / ky - hyz / kz;
-        ex = sign > 0 ? cax * ex + cbx * cu : cax * ex - cbx * cu;
-    }
-    if (upy) {
-        const double cu = hxz / kz - hzx / kx;
-        ey = sign > 0 ? cay * ey + cby * cu : cay * ey - cby * cu;
-    }
-    if (upz) {
-        const double cu = hyx / kx - hxy / ky;
-        ez = sign > 0 ? caz * ez + cbz * cu : caz * ez - cbz * cu;
+    if (UPD) {
+        const double cux = hzy / Y.k - hyz / Z.k;
+        const double cuy = hxz / Z.k - hzx / X.k;
+        const double cuz = hyx / X.k - hxy / Y.k;
+        ex = upx ? (sign > 0 ? cax * ex + cbx * cux : cax * ex - cbx * cux) : ex;
+        ey = upy ? (sign > 0 ? cay * ey + cby * cuy : cay * ey - cby * cuy) : ey;
+        ez = upz ? (sign > 0 ? caz * ez + cbz * cuz : caz * ez - cbz * cuz) : ez;
     }
     // The psi values are stored after all arithmetic: a store issued before a
     // later face's branch would make that branch's wait for its loads also
@@ -290,26 +296,27 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
     double px0 = 0.0, px1 = 0.0, py0 = 0.0, py1 = 0.0, pz0 = 0.0, pz1 = 0.0;
     if (fx) {
         const double h = S.dl[0];
-        px0 = bx * ax0 + cx * hyx / h;
-        px1 = bx * ax1 + cx * hzx / h;
+        px0 = X.b * ax0 + X.c * hyx / h;
+        px1 = X.b * ax1 + X.c * hzx / h;
         ez += cbz * px0;
         ey -= cby * px1;
     }
     if (fy) {
         const double h = S.dl[1];
-        py0 = by * ay0 + cy * hzy / h;
-        py1 = by * ay1 + cy * hxy / h;
+        py0 = Y.b * ay0 + Y.c * hzy / h;
+        py1 = Y.b * ay1 + Y.c * hxy / h;
         ex += cbx * py0;
         ez -= cbz * py1;
     }
     if (fz) {
         const double h = S.dl[2];
-        pz0 = bz * az0 + cz * hxz / h;
-        pz1 = bz * az1 + cz * hyz / h;
+        pz0 = Z.b * az0 + Z.c * hxz / h;
+        pz1 = Z.b * az1 + Z.c * hyz / h;
         ey += cby * pz0;
         ex -= cbx * pz1;
     }
-    if (src) {
+    if ((MODE & M_SRC) && k == S.src_k && oc == S.src_o) {
+        const double amp = gc(S.amp)[n];
         if (S.src_comp == 0)
             ex -= amp;
         else if (S.src_comp == 1)
@@ -318,55 +325,24 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
             ez -= amp;
     }
     if (fx) {
-        st_s<NT>(P0 + q0, px0);
-        st_s<NT>(P0 + L0 + q0, px1);
+        put_s<NT>(mb(S.psi[0] + pw) + b0, q0, px0);
+        put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, px1);
     }
     if (fy) {
-        st_s<NT>(P1 + q1, py0);
-        st_s<NT>(P1 + L1 + q1, py1);
+        put_s<NT>(mb(S.psi[1] + pw) + b1, q1, py0);
+        put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, py1);
     }
     if (fz) {
-        st_s<NT>(P2 + q2, pz0);
-        st_s<NT>(P2 + L2 + q2, pz1);
+        put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, pz0);
+        put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, pz1);
     }
-    st_s<NT>(Eout + c, ex);
-    st_s<NT>(Eout + N + c, ey);
-    st_s<NT>(Eout + 2 * (size_t)N + c, ez);
+    put_s<NT>(Eout, q.o, ex);
+    put_s<NT>(Eout + nb, q.o, ey);
+    put_s<NT>(Eout + 2 * nb, q.o, ez);
 }
 
-
-template <int MODE>
-__global__ __launch_bounds__(TX *TY) void k_efield(const ShotDev *__restrict__ D, int ns,
-                                                   const int *__restrict__ pre, int j, int nover,
-                                                   int sign)
-{
-    const int s = find_shot(pre, ns, blockIdx.x);
-    const ShotDev &S = D[s];
-    int n = nover;
-    if (n < 0) {
-        n = chunk_step(S) + j;
-        if (n >= S.it - 1)
-            return;  // this shot has finished its time loop
-    }
-    const int b = blockIdx.x - pre[s];
-    const int bx = b % S.nbx, t = b / S.nbx;
-    const int by = t % S.nby, k = t / S.nby;
-    const int i = bx * TX + threadIdx.x, jj = by * TY + threadIdx.y;
-    if (i >= S.ix || jj >= S.iy)
-        return;
-    int si, so;
-    if (MODE & M_INPLACE) {
-        si = so = S.cur;
-    } else {
-        si = (S.cur + j) % S.ring;
-        so = (S.cur + j + 1) % S.ring;
-    }
-    efield_cell<MODE>(S, hsel(S, 0, 0), i, jj, k, n, si, so, sign);
-}
-
-// One cell of the H update + CPML-H corrections, general path, with the loads
-// issued first as in efield_cell.  H is read from Hin and written to Hout (the
-// same buffer when updated in place).
+// One cell of the H update + CPML-H corrections, general path, as efield_cell.
+// H is read from Hin and written to Hout (the same buffer when updated in place).
 __device__ __forceinline__ double dp(double fp1, double f0, double fp2, double fm1, double c1,
                                      double c2)
 {
@@ -375,128 +351,64 @@ __device__ __forceinline__ double dp(double fp1, double f0, double fp2, double f
 
 template <int MODE>
 __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin, double *Hout, int i,
-                                            int jj, int k, int so, int sign)
+                                            int jj, int k, unsigned oc, int fl, int so, int sign)
 {
-    constexpr bool NT = (MODE & M_NT) != 0;
-    const int ix = S.ix, iy = S.iy, iz = S.iz, nc = S.nc, N = S.n;
-    const int sy = ix, sz = ix * iy;
-    const int c = (k * iy + jj) * ix + i;
-
-    const GLOBAL double *__restrict__ Ex = gc(S.e + (size_t)so * S.sstride);
-    const GLOBAL double *__restrict__ Ey = gc(Ex + N);
-    const GLOBAL double *__restrict__ Ez = gc(Ex + 2 * (size_t)N);
-
-    const double c1 = S.c1, c2 = S.c2, dt = S.dt;
-    const GLOBAL double *__restrict__ px = gc(S.prof[0]);
-    const GLOBAL double *__restrict__ py = gc(S.prof[1]);
-    const GLOBAL double *__restrict__ pz = gc(S.prof[2]);
-
-    const bool ax1 = i >= 1 && i < ix - 1, ax2 = i >= 1 && i < ix - 2;
-    const bool ay1 = jj >= 1 && jj < iy - 1, ay2 = jj >= 1 && jj < iy - 2;
-    const bool az1 = k >= 1 && k < iz - 1, az2 = k >= 1 && k < iz - 2;
-    const bool upx = (MODE & M_UPD) && ax1 && ay2 && az2;
-    const bool upy = (MODE & M_UPD) && ax2 && ay1 && az2;
-    const bool upz = (MODE & M_UPD) && ax2 && ay2 && az1;
-    // CPML-H faces: [1,nc-1)U[n-nc,n-2) on every axis
-    const bool gx = (MODE & M_PSI) && ((i >= 1 && i < nc - 1) || (i >= ix - nc && i < ix - 2)) &&
-                    jj < iy - 1 && k < iz - 1;
-    const bool gy = (MODE & M_PSI) && ((jj >= 1 && jj < nc - 1) || (jj >= iy - nc && jj < iy - 2)) &&
-                    i < ix - 1 && k < iz - 1;
-    const bool gz = (MODE & M_PSI) && ((k >= 1 && k < nc - 1) || (k >= iz - nc && k < iz - 2)) &&
-                    i < ix - 1 && jj < iy - 1;
+    constexpr bool NT = (MODE & M_NT) != 0, UPD = (MODE & M_UPD) != 0, PSI = (MODE & M_PSI) != 0;
+    const bool upx = UPD && (fl & FL_UHX), upy = UPD && (fl & FL_UHY), upz = UPD && (fl & FL_UHZ);
+    const bool gx = PSI && (fl & FL_PHX), gy = PSI && (fl & FL_PHY), gz = PSI && (fl & FL_PHZ);
     if (!(upx || upy || upz || gx || gy || gz))
         return;
+    const int nc = S.nc;
+    const size_t nb = (size_t)S.n * 8, pb = S.pb, kp = (size_t)k * pb;
 
     // ---- loads
-    // every forward stencil in bounds: all six derivatives are loaded
-    const bool all = ax2 && ay2 && az2;
-    const bool nzy = all || upx || gy, nyz = all || upx || gz, nxz = all || upy || gz;
-    const bool nzx = all || upy || gx, nyx = all || upz || gx, nxy = all || upz || gy;
-    double z0 = 0.0, zyp1 = 0.0, zyp2 = 0.0, zym1 = 0.0, zxp1 = 0.0, zxp2 = 0.0, zxm1 = 0.0;
-    double y0 = 0.0, yzp1 = 0.0, yzp2 = 0.0, yzm1 = 0.0, yxp1 = 0.0, yxp2 = 0.0, yxm1 = 0.0;
-    double x0 = 0.0, xzp1 = 0.0, xzp2 = 0.0, xzm1 = 0.0, xyp1 = 0.0, xyp2 = 0.0, xym1 = 0.0;
-    if (nzy || nzx)
-        z0 = Ez[c];
-    if (nzy) {
-        zyp1 = Ez[c + sy];
-        zyp2 = Ez[c + 2 * sy];
-        zym1 = Ez[c - sy];
-    }
-    if (nzx) {
-        zxp1 = Ez[c + 1];
-        zxp2 = Ez[c + 2];
-        zxm1 = Ez[c - 1];
-    }
-    if (nyz || nyx)
-        y0 = Ey[c];
-    if (nyz) {
-        yzp1 = Ey[c + sz];
-        yzp2 = Ey[c + 2 * sz];
-        yzm1 = Ey[c - sz];
-    }
-    if (nyx) {
-        yxp1 = Ey[c + 1];
-        yxp2 = Ey[c + 2];
-        yxm1 = Ey[c - 1];
-    }
-    if (nxz || nxy)
-        x0 = Ex[c];
-    if (nxz) {
-        xzp1 = Ex[c + sz];
-        xzp2 = Ex[c + 2 * sz];
-        xzm1 = Ex[c - sz];
-    }
-    if (nxy) {
-        xyp1 = Ex[c + sy];
-        xyp2 = Ex[c + 2 * sy];
-        xym1 = Ex[c - sy];
-    }
-    const double msx = px[PR_MSIG * ix + i], msy = py[PR_MSIG * iy + jj], msz = pz[PR_MSIG * iz + k];
+    const Off<1, 2> q(S, oc);
+    const size_t zm1 = k >= 1 ? kp - pb : kp;
+    const size_t zp1 = k + 1 < S.iz ? kp + pb : kp, zp2 = k + 2 < S.iz ? kp + 2 * pb : kp;
+    const gcp Eb = cb(S.e + (size_t)so * S.sstride), Ex = Eb + kp, Ey = Eb + nb + kp,
+              Ez = Eb + 2 * nb + kp;
+    const gcp Hi = cb(Hin) + kp;
+    const double z0 = at(Ez, q.o), zyp1 = at(Ez, q.yp1), zyp2 = at(Ez, q.yp2), zym1 = at(Ez, q.ym1);
+    const double zxp1 = at(Ez, q.x, 8), zxp2 = at(Ez, q.x, 16), zxm1 = at(Ez, q.x, -8);
+    const double y0 = at(Ey, q.o), yzp1 = at(Eb + nb + zp1, q.o), yzp2 = at(Eb + nb + zp2, q.o),
+                 yzm1 = at(Eb + nb + zm1, q.o);
+    const double yxp1 = at(Ey, q.x, 8), yxp2 = at(Ey, q.x, 16), yxm1 = at(Ey, q.x, -8);
+    const double x0 = at(Ex, q.o), xzp1 = at(Eb + zp1, q.o), xzp2 = at(Eb + zp2, q.o),
+                 xzm1 = at(Eb + zm1, q.o);
+    const double xyp1 = at(Ex, q.yp1), xyp2 = at(Ex, q.yp2), xym1 = at(Ex, q.ym1);
+    double hx = at_s<NT>(Hi, q.o), hy = at_s<NT>(Hi + nb, q.o), hz = at_s<NT>(Hi + 2 * nb, q.o);
     // eps' is only used where a magnetic CPML conductivity is nonzero; loading
     // it beside the conductivities rather than after them saves a round trip
-    const double eps2 = gc(S.eps)[c];
-    const GLOBAL double *__restrict__ Hi = gc(Hin);
-    double hx = ld_s<NT>(Hi + c), hy = ld_s<NT>(Hi + N + c), hz = ld_s<NT>(Hi + 2 * (size_t)N + c);
-    double kx = 1.0, ky = 1.0, kz = 1.0;
-    if (MODE & M_UPD) {
-        kx = px[PR_KHD * ix + i];
-        ky = py[PR_KHD * iy + jj];
-        kz = pz[PR_KHD * iz + k];
-    }
+    const double eps2 = at(cb(S.eps) + kp, q.o);
+    const Quad X = quad<true>(S.prof[0], S.ix, i), Y = quad<true>(S.prof[1], S.iy, jj);
+    const Quad Z = uquad<true>(S.cq[2], k);
     // psi in place, or (pstride set) read from the ring slot before so and
     // written to slot so like H
-    const size_t pr = S.pstride ? (size_t)((so + S.ring - 1) % S.ring) * S.pstride : 0;
+    const size_t pr = S.pstride ? (size_t)(so == 0 ? S.ring - 1 : so - 1) * S.pstride : 0;
     const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
-    const GLOBAL double *Q0 = gc(S.psi[0] + pr), *Q1 = gc(S.psi[1] + pr), *Q2 = gc(S.psi[2] + pr);
-    GLOBAL double *P0 = gm(S.psi[0] + pw), *P1 = gm(S.psi[1] + pw), *P2 = gm(S.psi[2] + pw);
-    const size_t L0 = (size_t)S.slab[0], L1 = (size_t)S.slab[1], L2 = (size_t)S.slab[2];
-    size_t q0 = 0, q1 = 0, q2 = 0;
-    double bx = 0.0, cx = 0.0, ax0 = 0.0, ax1v = 0.0;
-    double by = 0.0, cy = 0.0, ay0 = 0.0, ay1v = 0.0;
-    double bz = 0.0, cz = 0.0, az0 = 0.0, az1v = 0.0;
+    const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
+    const size_t b0 = 2 * L0 + (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
+    const size_t b1 = 2 * L1 + (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
+    const size_t b2 = 2 * L2 + (size_t)(unsigned)slab_pos(k, S.iz, nc) * pb;   // k in a shell only
+    unsigned q0 = 0, q1 = 0;
+    double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, az0 = 0.0, az1 = 0.0;
     if (gx) {
-        q0 = ((size_t)k * iy + jj) * (2 * nc) + slab_pos(i, ix, nc);
-        bx = px[PR_BH * ix + i];
-        cx = px[PR_CH * ix + i];
-        ax0 = Q0[2 * L0 + q0];
-        ax1v = Q0[3 * L0 + q0];
+        q0 = (unsigned)(jj * (2 * nc) + slab_pos(i, S.ix, nc)) * 8u;
+        ax0 = at(cb(S.psi[0] + pr) + b0, q0);
+        ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
     }
     if (gy) {
-        q1 = ((size_t)k * (2 * nc) + slab_pos(jj, iy, nc)) * ix + i;
-        by = py[PR_BH * iy + jj];
-        cy = py[PR_CH * iy + jj];
-        ay0 = Q1[2 * L1 + q1];
-        ay1v = Q1[3 * L1 + q1];
+        q1 = (unsigned)(slab_pos(jj, S.iy, nc) * S.ix + i) * 8u;
+        ay0 = at(cb(S.psi[1] + pr) + b1, q1);
+        ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
     }
     if (gz) {
-        q2 = ((size_t)slab_pos(k, iz, nc) * iy + jj) * ix + i;
-        bz = pz[PR_BH * iz + k];
-        cz = pz[PR_CH * iz + k];
-        az0 = Q2[2 * L2 + q2];
-        az1v = Q2[3 * L2 + q2];
+        az0 = at(cb(S.psi[2] + pr) + b2, q.o);
+        az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
     }
 
     // ---- arithmetic
+    const double c1 = S.c1, c2 = S.c2, dt = S.dt;
     const double ezy = dp(zyp1, z0, zyp2, zym1, c1, c2);
     const double eyz = dp(yzp1, y0, yzp2, yzm1, c1, c2);
     const double exz = dp(xzp1, x0, xzp2, xzm1, c1, c2);
@@ -506,100 +418,110 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
 
     // db = dt/mu0/(1 + s) and da = (1 - s)/(1 + s) with s = msig dt/(2 eps');
     // exactly dt/mu0 and 1 where an axis' magnetic CPML sigma is zero
-    const double dtm = dt / S.mu0;
+    const double dtm = S.dtm;
     double dax = 1.0, day = 1.0, daz = 1.0, dbx = dtm, dby = dtm, dbz = dtm;
-    if (msx != 0.0) {
-        const double sm = msx * dt / (2.0 * eps2);
+    if (X.s != 0.0) {
+        const double sm = X.s * dt / (2.0 * eps2);
         dbx = dtm / (1.0 + sm);
         dax = (1.0 - sm) / (1.0 + sm);
     }
-    if (msy != 0.0) {
-        const double sm = msy * dt / (2.0 * eps2);
+    if (Y.s != 0.0) {
+        const double sm = Y.s * dt / (2.0 * eps2);
         dby = dtm / (1.0 + sm);
         day = (1.0 - sm) / (1.0 + sm);
     }
-    if (msz != 0.0) {
-        const double sm = msz * dt / (2.0 * eps2);
+    if (Z.s != 0.0) {
+        const double sm = Z.s * dt / (2.0 * eps2);
         dbz = dtm / (1.0 + sm);
         daz = (1.0 - sm) / (1.0 + sm);
     }
 
-    if (upx) {
-        const double cu = ezy / ky - eyz / kz;
-        hx = sign > 0 ? dax * hx - dbx * cu : dax * hx + dbx * cu;
-    }
-    if (upy) {
-        const double cu = exz / kz - ezx / kx;
-        hy = sign > 0 ? day * hy - dby * cu : day * hy + dby * cu;
-    }
-    if (upz) {
-        const double cu = eyx / kx - exy / ky;
-        hz = sign > 0 ? daz * hz - dbz * cu : daz * hz + dbz * cu;
+    if (UPD) {
+        const double cux = ezy / Y.k - eyz / Z.k;
+        const double cuy = exz / Z.k - ezx / X.k;
+        const double cuz = eyx / X.k - exy / Y.k;
+        hx = upx ? (sign > 0 ? dax * hx - dbx * cux : dax * hx + dbx * cux) : hx;
+        hy = upy ? (sign > 0 ? day * hy - dby * cuy : day * hy + dby * cuy) : hy;
+        hz = upz ? (sign > 0 ? daz * hz - dbz * cuz : daz * hz + dbz * cuz) : hz;
     }
     // psi stored after all arithmetic, as in efield_cell
     double px0 = 0.0, px1 = 0.0, py0 = 0.0, py1 = 0.0, pz0 = 0.0, pz1 = 0.0;
     if (gx) {
         const double h = S.dl[0];
-        px0 = bx * ax0 + cx * ezx / h;
-        px1 = bx * ax1v + cx * eyx / h;
+        px0 = X.b * ax0 + X.c * ezx / h;
+        px1 = X.b * ax1 + X.c * eyx / h;
         hy += dby * px0;
         hz -= dbz * px1;
     }
     if (gy) {
         const double h = S.dl[1];
-        py0 = by * ay0 + cy * exy / h;
-        py1 = by * ay1v + cy * ezy / h;
+        py0 = Y.b * ay0 + Y.c * exy / h;
+        py1 = Y.b * ay1 + Y.c * ezy / h;
         hz += dbz * py0;
         hx -= dbx * py1;
     }
     if (gz) {
         const double h = S.dl[2];
-        pz0 = bz * az0 + cz * eyz / h;
-        pz1 = bz * az1v + cz * exz / h;
+        pz0 = Z.b * az0 + Z.c * eyz / h;
+        pz1 = Z.b * az1 + Z.c * exz / h;
         hx += dbx * pz0;
         hy -= dby * pz1;
     }
     if (gx) {
-        st_s<NT>(P0 + 2 * L0 + q0, px0);
-        st_s<NT>(P0 + 3 * L0 + q0, px1);
+        put_s<NT>(mb(S.psi[0] + pw) + b0, q0, px0);
+        put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, px1);
     }
     if (gy) {
-        st_s<NT>(P1 + 2 * L1 + q1, py0);
-        st_s<NT>(P1 + 3 * L1 + q1, py1);
+        put_s<NT>(mb(S.psi[1] + pw) + b1, q1, py0);
+        put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, py1);
     }
     if (gz) {
-        st_s<NT>(P2 + 2 * L2 + q2, pz0);
-        st_s<NT>(P2 + 3 * L2 + q2, pz1);
+        put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, pz0);
+        put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, pz1);
     }
-    GLOBAL double *__restrict__ Ho = gm(Hout);
-    st_s<NT>(Ho + c, hx);
-    st_s<NT>(Ho + N + c, hy);
-    st_s<NT>(Ho + 2 * (size_t)N + c, hz);
+    const gmp Ho = mb(Hout) + kp;
+    put_s<NT>(Ho, q.o, hx);
+    put_s<NT>(Ho + nb, q.o, hy);
+    put_s<NT>(Ho + 2 * nb, q.o, hz);
 }
 
+// Cell of this lane in the single operators: PT consecutive cells of a plane
+// per block, each XCD owning a contiguous run of blocks
+__device__ __forceinline__ bool plane_cell(const ShotDev &S, int b, int &i, int &jj, int &k, unsigned &o)
+{
+    const unsigned q = (b & 7) * (S.op_pad >> 3) + (b >> 3);
+    k = (int)(((unsigned long long)q * S.omul) >> S.osh);
+    const unsigned c = (q - (unsigned)k * S.opp) * PT + threadIdx.x;
+    o = c * 8u;
+    if (k >= S.iz || o >= S.pb)
+        return false;
+    jj = (int)(__umulhi(c, S.imul) >> (S.ish - 32));
+    i = (int)c - jj * S.ix;
+    return true;
+}
+
+// The single operators: one launch over every cell, E and H in place.
+template <int MODE>
+__global__ __launch_bounds__(PT) void k_efield(const ShotDev *__restrict__ D, int sign)
+{
+    const ShotDev &S = D[0];
+    int i, jj, k;
+    unsigned o;
+    if (!plane_cell(S, blockIdx.x, i, jj, k, o))
+        return;
+    efield_cell<MODE>(S, hsel(S, 0, 0), i, jj, k, o, flags(S, i, jj, k), 0, S.cur, S.cur, sign);
+}
 
 template <int MODE>
-__global__ __launch_bounds__(TX *TY) void k_hfield(const ShotDev *__restrict__ D, int ns,
-                                                   const int *__restrict__ pre, int j, int sign)
+__global__ __launch_bounds__(PT) void k_hfield(const ShotDev *__restrict__ D, int sign)
 {
-    const int s = find_shot(pre, ns, blockIdx.x);
-    const ShotDev &S = D[s];
-    int so;
-    if (MODE & M_INPLACE) {
-        so = S.cur;
-    } else {
-        if (chunk_step(S) + j >= S.it - 1)
-            return;
-        so = (S.cur + j + 1) % S.ring;
-    }
-    const int b = blockIdx.x - pre[s];
-    const int bx = b % S.nbx, t = b / S.nbx;
-    const int by = t % S.nby, k = t / S.nby;
-    const int i = bx * TX + threadIdx.x, jj = by * TY + threadIdx.y;
-    if (i >= S.ix || jj >= S.iy)
+    const ShotDev &S = D[0];
+    int i, jj, k;
+    unsigned o;
+    if (!plane_cell(S, blockIdx.x, i, jj, k, o))
         return;
     double *H = hsel(S, 0, 0);
-    hfield_cell<MODE>(S, H, H, i, jj, k, so, sign);
+    hfield_cell<MODE>(S, H, H, i, jj, k, o, flags(S, i, jj, k), S.cur, sign);
 }
 
 // read_source_3d as a stand-alone operator (in place on the current slot)
@@ -1325,27 +1247,53 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 
 
 // ------------------------------------------------------------------------
-// Per-cell kernels of the fused step (32 x 8 tiles, one plane per block,
-// blocks numbered so each XCD owns a contiguous run of tiles).  Waves whose
-// cells all lie outside every CPML shell take a branch-free path with all 25
-// loads issued up front; there the reference's coefficients reduce exactly to
-// ca = 1, cb = dt/eps' (E) and da = 1, db = dt/mu0 (H), so no division by the
-// coefficient denominators is needed and the result is bit-identical.  Any
-// other wave runs the general per-cell code.
+// Per-cell kernels of the fused step: one tile of one plane per block.  The
+// stencil's x and y neighbours come from LDS: every lane loads its own cell of
+// the three source components and one value of the tile's halo (6 (w + h) <= PT
+// values), so a cell costs 4 loads there instead of 15, and its values wait in
+// LDS instead of registers; the z neighbours, which no other lane of the block
+// needs, are loaded directly.  All loads of a block are issued before its one
+// barrier.  What bounds them: above 2.5 M cells, where they take the CPML
+// shells, and for batches beyond the Infinity Cache, memory (5 TB/s on their own
+// bytes at 288^3); on grids that fit that cache a plain copy of the same bytes
+// reaches 6.5 TB/s plus 3 us a launch, and these kernels 60-75 % of that, held
+// back by the instructions a wave issues around its one round trip.  Against
+// the same per-cell code with every stencil value loaded by its own lane
+// (116 / 112 VGPRs, 4 waves per SIMD; now 77 / 76, 6 waves), E and H half-step
+// by rocprofv3: shells of 288^3 187 + 200 -> 161 + 168 us, 131 x 97 x 75
+// 25.8 + 26.3 -> 22.0 + 21.7 us, 84^3 17.4 + 18.2 -> 16.4 + 16.3 us.  Tried on
+// the way and slower at 288^3: the same loads per lane from wave-uniform bases
+// with 32-bit offsets but without LDS (199 + 211 us).
+// A tile that no CPML shell touches reads no profile and takes the update where
+// ca = 1, cb = dt/eps' (E), da = 1, db = dt/mu0 (H) exactly; an axis whose
+// shell the tile does not touch contributes wave-uniform values.
 
-__device__ __forceinline__ bool fcell(const ShotDev &S, int b, int &i, int &jj, int &k)
+namespace {
+
+// Tile of a block, the same for its lanes: rows [y0, yend) x columns [x0, x0 + w)
+// of plane k, th = rows of lanes
+struct FTile {
+    int x0, y0, k, w, h, yend;
+    bool region;   // may hold cells of the LDS kernels' region
+};
+
+__device__ __forceinline__ bool ftile(const ShotDev &S, int b, FTile &T)
 {
     if (!S.shell) {
-        // every tile of the grid, each XCD owning a contiguous run of planes
-        const int q = (b & 7) * (S.fb_pad >> 3) + (b >> 3);
-        if (q >= S.fb)
+        // every tile of every plane, each XCD owning a contiguous run
+        const unsigned q = (b & 7) * (S.fb_pad >> 3) + (b >> 3);
+        if (q >= (unsigned)S.fb)
             return false;
-        const int tx = q % S.ftx, r = q / S.ftx;
-        const int ty = r % S.fty;
-        k = r / S.fty;
-        i = tx * ZX + (threadIdx.x & (ZX - 1));
-        jj = ty * ZY + threadIdx.x / ZX;
-        return i < S.ix && jj < S.iy;
+        T.k = (int)(((unsigned long long)q * S.tmul) >> S.tsh);
+        const unsigned r = q - (unsigned)T.k * S.tpp;
+        const unsigned ty = (unsigned)(((unsigned long long)r * S.xmul) >> S.xsh);
+        T.w = S.tw;
+        T.h = S.th;
+        T.x0 = (int)(r - ty * S.ttx) * T.w;
+        T.y0 = (int)ty * T.h;
+        T.yend = S.iy;
+        T.region = false;
+        return true;
     }
     // the shell tile list in launch order: at 288^3 (16-cell CPML) this runs
     // each half-step's shell launch 12 us faster than giving each XCD a
@@ -1353,24 +1301,81 @@ __device__ __forceinline__ bool fcell(const ShotDev &S, int b, int &i, int &jj, 
     // covers whole (84^3) the contiguous runs are 1.2x faster
     if (b >= S.fb)
         return false;
-    const GLOBAL int *t = (const GLOBAL int *)(S.shell + b);   // {x0, y0, k, yend}
-    const int x0 = t[0], y0 = t[1], yend = t[3];
-    k = t[2];
-    if (yend) {   // 16 x 16 tile of an x-edge segment, rows below yend
-        i = x0 + (threadIdx.x & 15);
-        jj = y0 + (threadIdx.x >> 4);
-        if (jj >= yend)
-            return false;
-    } else {
-        i = x0 + (threadIdx.x & (ZX - 1));
-        jj = y0 + threadIdx.x / ZX;
-    }
-    if (k < 0 || i >= S.ix || jj >= S.iy)
-        return false;
-    // cells of the LDS kernels' region are theirs
-    return !(i >= S.lo[0] && i < S.hi[0] && jj >= S.lo[1] && jj < S.hi[1] && k >= S.lo[2] &&
-             k < S.hi[2]);
+    const int *t = (const int *)(S.shell + b);   // {x0, y0, k, yend}
+    T.x0 = uload(t);
+    T.y0 = uload(t + 1);
+    T.k = uload(t + 2);
+    const int yend = uload(t + 3);
+    T.w = yend ? 16 : ZX;
+    T.h = yend ? 16 : ZY;
+    T.yend = yend ? yend : S.iy;
+    T.region = !yend && T.k >= S.lo[2] && T.k < S.hi[2];
+    return T.k >= 0;
 }
+
+// A lane's cell in its tile, its LDS position (pitch w + 3, two cells before
+// the tile for E, one for H) and its halo item.  LO cells before the tile and
+// HI after it on each axis (LO + HI = 3): first the halo rows of component 2,
+// then of component 0, then the halo columns of component 2, then of component 1.
+template <int LO> struct FLane {
+    int i, jj;
+    unsigned o;        // byte offset of the (clamped) cell in its plane
+    unsigned a, p;     // LDS byte address of the cell, pitch in bytes
+    bool own;          // the lane's cell is one of the tile's
+    bool halo;         // the lane has a halo item
+    int hc;            // its component
+    unsigned ho, ha;   // its plane offset and LDS byte address
+    __device__ __forceinline__ FLane(const ShotDev &S, const FTile &T)
+    {
+        const int t = threadIdx.x, w = T.w, h = T.h;
+        const unsigned wm = (65535u + w) / (unsigned)w;   // t / w = t wm >> 16 for t < 256, w <= PT_WH
+        const int ly = (int)((t * wm) >> 16), lx = t - ly * w;
+        p = (unsigned)(w + 3) * 8u;
+        i = T.x0 + lx;
+        jj = T.y0 + ly;
+        own = ly < h;
+        o = (unsigned)min(jj, S.iy - 1) * S.row + (unsigned)min(i, S.ix - 1) * 8u;
+        a = (unsigned)(ly + LO) * p + (unsigned)(lx + LO) * 8u;
+        int u, v;   // halo position relative to the tile
+        if (t < 6 * w) {
+            const bool second = t >= 3 * w;
+            const int m = second ? t - 3 * w : t;
+            const int r = (int)((m * wm) >> 16);
+            u = m - r * w;
+            v = r < LO ? r - LO : h + r - LO;
+            hc = second ? 0 : 2;
+        } else {
+            int m = t - 6 * w;
+            const bool second = m >= 3 * h;
+            m = second ? m - 3 * h : m;
+            v = (m * 21846) >> 16;   // m / 3
+            const int r = m - 3 * v;
+            u = r < LO ? r - LO : w + r - LO;
+            hc = second ? 1 : 2;
+        }
+        halo = t < 6 * (w + h);
+        const int gx = min(max(T.x0 + u, 0), S.ix - 1), gy = min(max(T.y0 + v, 0), S.iy - 1);
+        ho = (unsigned)gy * S.row + (unsigned)gx * 8u;
+        ha = (unsigned)(v + LO) * p + (unsigned)(u + LO) * 8u + (unsigned)hc * (PT_TILE * 8u);
+    }
+};
+
+// r in [a, b) U [c, d): an axis' CPML face (a superset of a cell's face flag, so
+// psi loads need not wait for the flag words)
+__device__ __forceinline__ bool in_face(int r, int a, int b, int c, int d)
+{
+    return (r >= a && r < b) || (r >= c && r < d);
+}
+__device__ __forceinline__ double lds_at(const double *b, unsigned o, int d = 0)
+{
+    return *(const double *)((const char *)b + o + d);
+}
+__device__ __forceinline__ void lds_put(double *b, unsigned o, double v)
+{
+    *(double *)((char *)b + o) = v;
+}
+
+}  // namespace
 
 // The first recn blocks (recn: 0, or ns rounded up to a multiple of 8 so that
 // the tile blocks keep their XCD) gather the receivers of the previous local
@@ -1380,10 +1385,10 @@ __device__ __forceinline__ bool fcell(const ShotDev &S, int b, int &i, int &jj, 
 // they overlap the tile blocks instead of trailing the launch.  hf: the step
 // is a fused E+H launch sequence (H before step j is hsel(S, j, 1)).
 template <bool NT>
-__global__ __launch_bounds__(ZX *ZY) void k_efield_f(const ShotDev *__restrict__ D, int ns,
-                                                     const int *__restrict__ pre, int j, int sign,
-                                                     int recn, int hf)
+__global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, int ns,
+                                                 const int *__restrict__ pre, int j, int recn, int hf)
 {
+    __shared__ double sh[3 * PT_TILE];
     if ((int)blockIdx.x < recn) {
         if ((int)blockIdx.x < ns) {
             const ShotDev &R = D[blockIdx.x];
@@ -1394,150 +1399,385 @@ __global__ __launch_bounds__(ZX *ZY) void k_efield_f(const ShotDev *__restrict__
         return;
     }
     const int b = blockIdx.x - recn;
-    const int s = find_shot(pre, ns, b);
+    const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
+    FTile T;
+    if (!ftile(S, ns > 1 ? b - pre[s] : b, T))
+        return;   // uniform over the block
+    const int k = T.k, nc = S.nc;
+    const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
+    const bool az = k < nc || k >= S.iz - nc;
+    const int si = ring_slot(S, S.cur + j), so = ring_slot(S, S.cur + j + 1);
+    const size_t nb = (size_t)S.n * 8, pb = S.pb, kp = (size_t)k * pb;
+    const size_t zm1 = k >= 1 ? kp - pb : kp, zm2 = k >= 2 ? kp - 2 * pb : kp;
+    const size_t zp1 = k + 1 < S.iz ? kp + pb : kp;
+    const gcp Hb = cb(hsel(S, j, hf)), Ein = cb(S.e + (size_t)si * S.sstride) + kp;
+    const FLane<2> q(S, T);
+
+    // ---- loads
+    const double z0 = at(Hb + 2 * nb + kp, q.o), y0 = at(Hb + nb + kp, q.o), x0 = at(Hb + kp, q.o);
+    double hv = 0.0;
+    if (q.halo)
+        hv = *(const GLOBAL double *)(Hb + kp + (size_t)q.hc * nb + q.ho);
+    const double yzm1 = at(Hb + nb + zm1, q.o), yzp1 = at(Hb + nb + zp1, q.o), yzm2 = at(Hb + nb + zm2, q.o);
+    const double xzm1 = at(Hb + zm1, q.o), xzp1 = at(Hb + zp1, q.o), xzm2 = at(Hb + zm2, q.o);
+    double ex = at_s<NT>(Ein, q.o), ey = at_s<NT>(Ein + nb, q.o), ez = at_s<NT>(Ein + 2 * nb, q.o);
+    const bool shell = ax || ay || az;
+    const double mat = shell ? at(cb(S.eps) + kp, q.o) : at_s<NT>(cb(S.cbi) + kp, q.o);
+    Quad X{0.0, 0.0, 0.0, 0.0}, Y = X, Z = X;
+    int fl = 0;
+    const size_t pr = S.pstride ? (size_t)si * S.pstride : 0;
+    const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
+    const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
+    const size_t b0 = (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
+    const size_t b1 = (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
+    const size_t b2 = (size_t)(unsigned)slab_pos(k, S.iz, nc) * pb;   // k in a shell only
+    unsigned q0 = 0, q1 = 0;
+    double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, az0 = 0.0, az1 = 0.0;
+    const int ci = min(q.i, S.ix - 1), cj = min(q.jj, S.iy - 1);
+    Z.k = uload(S.cq[2] + (size_t)k * CQ_N + CQ_E + 1);
+    if (shell) {
+        Z = uquad<false>(S.cq[2], k);
+        fl = uload(S.fl[2] + k);
+        if (ax) {
+            X = quad<false>(S.prof[0], S.ix, ci);
+            fl &= *(const GLOBAL int *)(cb(S.fl[0]) + (unsigned)(ci * 4));
+            if (in_face(ci, 2, nc - 1, S.ix - nc + 1, S.ix - 2)) {
+                q0 = (unsigned)(cj * (2 * nc) + slab_pos(ci, S.ix, nc)) * 8u;
+                ax0 = at(cb(S.psi[0] + pr) + b0, q0);
+                ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
+            }
+        } else {
+            X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_E + 1);
+            fl &= uload(S.fl[0] + T.x0);
+        }
+        if (ay) {
+            Y = quad<false>(S.prof[1], S.iy, cj);
+            fl &= *(const GLOBAL int *)(cb(S.fl[1]) + (unsigned)(cj * 4));
+            if (in_face(cj, 2, nc, S.iy - nc + 1, S.iy - 2)) {
+                q1 = (unsigned)(slab_pos(cj, S.iy, nc) * S.ix + ci) * 8u;
+                ay0 = at(cb(S.psi[1] + pr) + b1, q1);
+                ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
+            }
+        } else {
+            Y.k = uload(S.cq[1] + (size_t)T.y0 * CQ_N + CQ_E + 1);
+            fl &= uload(S.fl[1] + T.y0);
+        }
+        if (in_face(k, 2, nc, S.iz - nc + 1, S.iz - 2)) {
+            az0 = at(cb(S.psi[2] + pr) + b2, q.o);
+            az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
+        }
+    } else {
+        X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_E + 1);
+        Y.k = uload(S.cq[1] + (size_t)T.y0 * CQ_N + CQ_E + 1);
+    }
+    if (q.own) {
+        lds_put(sh, q.a, x0);
+        lds_put(sh + PT_TILE, q.a, y0);
+        lds_put(sh + 2 * PT_TILE, q.a, z0);
+    }
+    if (q.halo)
+        lds_put(sh, q.ha, hv);
+    __syncthreads();
+    // the step is looked up behind the loads (it costs two dependent scalar
+    // loads): a shot that has finished its time loop stores nothing
     const int n = chunk_step(S) + j;
-    if (n >= S.it - 1)
+    if (n >= S.it - 1 || !q.own || q.i >= S.ix || q.jj >= T.yend)
         return;
-    int i, jj, k;
-    if (!fcell(S, b - pre[s], i, jj, k))
-        return;
-    const int ix = S.ix, iy = S.iy, iz = S.iz, nc = S.nc;
-    const int si = (S.cur + j) % S.ring, so = (S.cur + j + 1) % S.ring;
-    const bool inner = i >= nc && i < ix - nc && jj >= nc && jj < iy - nc && k >= nc && k < iz - nc;
-    const double *Hc = hsel(S, j, hf);
-    if (!__all(inner)) {
-        efield_cell<M_UPD | M_PSI | M_SRC | (NT ? M_NT : 0)>(S, Hc, i, jj, k, n, si, so, sign);
-        return;
-    }
-    const size_t N = (size_t)S.n;
-    const int sy = ix, sz = ix * iy;
-    const int c = (k * iy + jj) * ix + i;
-    const GLOBAL double *__restrict__ Ein = gc(S.e + (size_t)si * S.sstride);
-    GLOBAL double *__restrict__ Eout = gm(S.e + (size_t)so * S.sstride);
-    const GLOBAL double *__restrict__ Hx = gc(Hc);
-    const GLOBAL double *__restrict__ Hy = gc(Hc + N);
-    const GLOBAL double *__restrict__ Hz = gc(Hc + 2 * N);
-    const double ex0 = ld_s<NT>(Ein + c), ey0 = ld_s<NT>(Ein + N + c), ez0 = ld_s<NT>(Ein + 2 * N + c);
-    const double cb = ld_s<NT>(gc(S.cbi) + c);
-    const double z0 = Hz[c], zym1 = Hz[c - sy], zyp1 = Hz[c + sy], zym2 = Hz[c - 2 * sy];
-    const double zxm1 = Hz[c - 1], zxp1 = Hz[c + 1], zxm2 = Hz[c - 2];
-    const double y0 = Hy[c], yzm1 = Hy[c - sz], yzp1 = Hy[c + sz], yzm2 = Hy[c - 2 * sz];
-    const double yxm1 = Hy[c - 1], yxp1 = Hy[c + 1], yxm2 = Hy[c - 2];
-    const double x0 = Hx[c], xzm1 = Hx[c - sz], xzp1 = Hx[c + sz], xzm2 = Hx[c - 2 * sz];
-    const double xym1 = Hx[c - sy], xyp1 = Hx[c + sy], xym2 = Hx[c - 2 * sy];
-    const double kedx = gc(S.prof[0])[PR_KED * ix + i];
-    const double kedy = gc(S.prof[1])[PR_KED * iy + jj];
-    const double kedz = gc(S.prof[2])[PR_KED * iz + k];
+    if (T.region && q.i >= S.lo[0] && q.i < S.hi[0] && q.jj >= S.lo[1] && q.jj < S.hi[1])
+        return;   // cells of the LDS kernels' region are theirs
+
+    // ---- arithmetic
     const double c1 = S.c1, c2 = S.c2;
-    const double hzy = c1 * z0 - c1 * zym1 + c2 * zyp1 - c2 * zym2;
-    const double hyz = c1 * y0 - c1 * yzm1 + c2 * yzp1 - c2 * yzm2;
-    const double hxz = c1 * x0 - c1 * xzm1 + c2 * xzp1 - c2 * xzm2;
-    const double hzx = c1 * z0 - c1 * zxm1 + c2 * zxp1 - c2 * zxm2;
-    const double hyx = c1 * y0 - c1 * yxm1 + c2 * yxp1 - c2 * yxm2;
-    const double hxy = c1 * x0 - c1 * xym1 + c2 * xyp1 - c2 * xym2;
-    const double cux = hzy / kedy - hyz / kedz;
-    const double cuy = hxz / kedz - hzx / kedx;
-    const double cuz = hyx / kedx - hxy / kedy;
-    double ex = sign > 0 ? ex0 + cb * cux : ex0 - cb * cux;
-    double ey = sign > 0 ? ey0 + cb * cuy : ey0 - cb * cuy;
-    double ez = sign > 0 ? ez0 + cb * cuz : ez0 - cb * cuz;
-    if (c == S.src_cell) {
-        const double a = gc(S.amp)[n];
-        if (S.src_comp == 0)
-            ex -= a;
-        else if (S.src_comp == 1)
-            ey -= a;
-        else
-            ez -= a;
+    const double *sx = sh, *sy = sh + PT_TILE, *sz = sh + 2 * PT_TILE;
+    const unsigned am1 = q.a - q.p, am2 = am1 - q.p, ap1 = q.a + q.p;
+    const double hzy = dm(z0, lds_at(sz, am1), lds_at(sz, ap1), lds_at(sz, am2), c1, c2);
+    const double hyz = dm(y0, yzm1, yzp1, yzm2, c1, c2);
+    const double hxz = dm(x0, xzm1, xzp1, xzm2, c1, c2);
+    const double hzx = dm(z0, lds_at(sz, q.a, -8), lds_at(sz, q.a, 8), lds_at(sz, q.a, -16), c1, c2);
+    const double hyx = dm(y0, lds_at(sy, q.a, -8), lds_at(sy, q.a, 8), lds_at(sy, q.a, -16), c1, c2);
+    const double hxy = dm(x0, lds_at(sx, am1), lds_at(sx, ap1), lds_at(sx, am2), c1, c2);
+    const double cux = hzy / Y.k - hyz / Z.k;
+    const double cuy = hxz / Z.k - hzx / X.k;
+    const double cuz = hyx / X.k - hxy / Y.k;
+    const gmp Eout = mb(S.e + (size_t)so * S.sstride) + kp;
+    if (!shell) {
+        ex = ex + mat * cux;
+        ey = ey + mat * cuy;
+        ez = ez + mat * cuz;
+    } else {
+        // cb = dt/eps'/(1 + s) and ca = (1 - s)/(1 + s) with s = sig dt/(2 eps');
+        // where an axis' CPML sigma is zero they are exactly dt/eps' and 1, so
+        // the divisions are skipped there (most shell cells lie in one axis' CPML)
+        const double dt = S.dt, dte = dt / mat;
+        double cax = 1.0, cay = 1.0, caz = 1.0, cbx = dte, cby = dte, cbz = dte;
+        if (ax && X.s != 0.0) {
+            const double se = X.s * dt / (2.0 * mat);
+            cbx = dte / (1.0 + se);
+            cax = (1.0 - se) / (1.0 + se);
+        }
+        if (ay && Y.s != 0.0) {
+            const double se = Y.s * dt / (2.0 * mat);
+            cby = dte / (1.0 + se);
+            cay = (1.0 - se) / (1.0 + se);
+        }
+        if (az && Z.s != 0.0) {
+            const double se = Z.s * dt / (2.0 * mat);
+            cbz = dte / (1.0 + se);
+            caz = (1.0 - se) / (1.0 + se);
+        }
+        ex = (fl & FL_UEX) ? cax * ex + cbx * cux : ex;
+        ey = (fl & FL_UEY) ? cay * ey + cby * cuy : ey;
+        ez = (fl & FL_UEZ) ? caz * ez + cbz * cuz : ez;
+        if (ax && (fl & FL_PEX)) {
+            const double h = S.dl[0];
+            ax0 = X.b * ax0 + X.c * hyx / h;
+            ax1 = X.b * ax1 + X.c * hzx / h;
+            ez += cbz * ax0;
+            ey -= cby * ax1;
+        }
+        if (ay && (fl & FL_PEY)) {
+            const double h = S.dl[1];
+            ay0 = Y.b * ay0 + Y.c * hzy / h;
+            ay1 = Y.b * ay1 + Y.c * hxy / h;
+            ex += cbx * ay0;
+            ez -= cbz * ay1;
+        }
+        if (az && (fl & FL_PEZ)) {
+            const double h = S.dl[2];
+            az0 = Z.b * az0 + Z.c * hxz / h;
+            az1 = Z.b * az1 + Z.c * hyz / h;
+            ey += cby * az0;
+            ex -= cbx * az1;
+        }
     }
-    st_s<NT>(Eout + c, ex);
-    st_s<NT>(Eout + N + c, ey);
-    st_s<NT>(Eout + 2 * N + c, ez);
+    if (k == S.src_k && q.o == S.src_o) {
+        const double amp = gc(S.amp)[n];
+        if (S.src_comp == 0)
+            ex -= amp;
+        else if (S.src_comp == 1)
+            ey -= amp;
+        else
+            ez -= amp;
+    }
+    if (ax && (fl & FL_PEX)) {
+        put_s<NT>(mb(S.psi[0] + pw) + b0, q0, ax0);
+        put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, ax1);
+    }
+    if (ay && (fl & FL_PEY)) {
+        put_s<NT>(mb(S.psi[1] + pw) + b1, q1, ay0);
+        put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, ay1);
+    }
+    if (az && (fl & FL_PEZ)) {
+        put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, az0);
+        put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, az1);
+    }
+    put_s<NT>(Eout, q.o, ex);
+    put_s<NT>(Eout + nb, q.o, ey);
+    put_s<NT>(Eout + 2 * nb, q.o, ez);
 }
 
 template <bool NT>
-__global__ __launch_bounds__(ZX *ZY) void k_hfield_f(const ShotDev *__restrict__ D, int ns,
-                                                     const int *__restrict__ pre, int j, int sign,
-                                                     int hf)
+__global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, int ns,
+                                                 const int *__restrict__ pre, int j, int hf)
 {
-    const int s = find_shot(pre, ns, blockIdx.x);
+    __shared__ double sh[3 * PT_TILE];
+    const int b = blockIdx.x;
+    const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
-    if (chunk_step(S) + j >= S.it - 1)
-        return;
-    int i, jj, k;
-    if (!fcell(S, blockIdx.x - pre[s], i, jj, k))
-        return;
-    const int ix = S.ix, iy = S.iy, iz = S.iz, nc = S.nc;
-    const int so = (S.cur + j + 1) % S.ring;
-    const bool inner = i >= nc && i < ix - nc && jj >= nc && jj < iy - nc && k >= nc && k < iz - nc;
-    double *Hi = hsel(S, j, hf), *Ho = hsel(S, j + 1, hf);
-    if (!__all(inner)) {
-        hfield_cell<M_UPD | M_PSI | (NT ? M_NT : 0)>(S, Hi, Ho, i, jj, k, so, sign);
-        return;
+    FTile T;
+    if (!ftile(S, ns > 1 ? b - pre[s] : b, T))
+        return;   // uniform over the block
+    const int k = T.k, nc = S.nc;
+    const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
+    const bool az = k < nc || k >= S.iz - nc;
+    const int so = ring_slot(S, S.cur + j + 1);
+    const size_t nb = (size_t)S.n * 8, pb = S.pb, kp = (size_t)k * pb;
+    const size_t zm1 = k >= 1 ? kp - pb : kp;
+    const size_t zp1 = k + 1 < S.iz ? kp + pb : kp, zp2 = k + 2 < S.iz ? kp + 2 * pb : kp;
+    const gcp Eb = cb(S.e + (size_t)so * S.sstride), Hin = cb(hsel(S, j, hf)) + kp;
+    const FLane<1> q(S, T);
+
+    // ---- loads
+    const double z0 = at(Eb + 2 * nb + kp, q.o), y0 = at(Eb + nb + kp, q.o), x0 = at(Eb + kp, q.o);
+    double hv = 0.0;
+    if (q.halo)
+        hv = *(const GLOBAL double *)(Eb + kp + (size_t)q.hc * nb + q.ho);
+    const double yzp1 = at(Eb + nb + zp1, q.o), yzp2 = at(Eb + nb + zp2, q.o), yzm1 = at(Eb + nb + zm1, q.o);
+    const double xzp1 = at(Eb + zp1, q.o), xzp2 = at(Eb + zp2, q.o), xzm1 = at(Eb + zm1, q.o);
+    double hx = at_s<NT>(Hin, q.o), hy = at_s<NT>(Hin + nb, q.o), hz = at_s<NT>(Hin + 2 * nb, q.o);
+    const bool shell = ax || ay || az;
+    Quad X{0.0, 0.0, 0.0, 0.0}, Y = X, Z = X;
+    double mat = 1.0;
+    int fl = 0;
+    const size_t pr = S.pstride ? (size_t)(so == 0 ? S.ring - 1 : so - 1) * S.pstride : 0;
+    const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
+    const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
+    const size_t b0 = 2 * L0 + (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
+    const size_t b1 = 2 * L1 + (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
+    const size_t b2 = 2 * L2 + (size_t)(unsigned)slab_pos(k, S.iz, nc) * pb;   // k in a shell only
+    unsigned q0 = 0, q1 = 0;
+    double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, az0 = 0.0, az1 = 0.0;
+    const int ci = min(q.i, S.ix - 1), cj = min(q.jj, S.iy - 1);
+    Z.k = uload(S.cq[2] + (size_t)k * CQ_N + CQ_H + 1);
+    if (shell) {
+        mat = at(cb(S.eps) + kp, q.o);
+        Z = uquad<true>(S.cq[2], k);
+        fl = uload(S.fl[2] + k);
+        if (ax) {
+            X = quad<true>(S.prof[0], S.ix, ci);
+            fl &= *(const GLOBAL int *)(cb(S.fl[0]) + (unsigned)(ci * 4));
+            if (in_face(ci, 1, nc - 1, S.ix - nc, S.ix - 2)) {
+                q0 = (unsigned)(cj * (2 * nc) + slab_pos(ci, S.ix, nc)) * 8u;
+                ax0 = at(cb(S.psi[0] + pr) + b0, q0);
+                ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
+            }
+        } else {
+            X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_H + 1);
+            fl &= uload(S.fl[0] + T.x0);
+        }
+        if (ay) {
+            Y = quad<true>(S.prof[1], S.iy, cj);
+            fl &= *(const GLOBAL int *)(cb(S.fl[1]) + (unsigned)(cj * 4));
+            if (in_face(cj, 1, nc - 1, S.iy - nc, S.iy - 2)) {
+                q1 = (unsigned)(slab_pos(cj, S.iy, nc) * S.ix + ci) * 8u;
+                ay0 = at(cb(S.psi[1] + pr) + b1, q1);
+                ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
+            }
+        } else {
+            Y.k = uload(S.cq[1] + (size_t)T.y0 * CQ_N + CQ_H + 1);
+            fl &= uload(S.fl[1] + T.y0);
+        }
+        if (in_face(k, 1, nc - 1, S.iz - nc, S.iz - 2)) {
+            az0 = at(cb(S.psi[2] + pr) + b2, q.o);
+            az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
+        }
+    } else {
+        X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_H + 1);
+        Y.k = uload(S.cq[1] + (size_t)T.y0 * CQ_N + CQ_H + 1);
     }
-    const size_t N = (size_t)S.n;
-    const int sy = ix, sz = ix * iy;
-    const int c = (k * iy + jj) * ix + i;
-    const GLOBAL double *__restrict__ Ex = gc(S.e + (size_t)so * S.sstride);
-    const GLOBAL double *__restrict__ Ey = gc(Ex + N);
-    const GLOBAL double *__restrict__ Ez = gc(Ex + 2 * N);
-    const GLOBAL double *__restrict__ Hxi = gc(Hi);
-    const GLOBAL double *__restrict__ Hyi = gc(Hi + N);
-    const GLOBAL double *__restrict__ Hzi = gc(Hi + 2 * N);
-    GLOBAL double *__restrict__ Hx = gm(Ho);
-    GLOBAL double *__restrict__ Hy = gm(Ho + N);
-    GLOBAL double *__restrict__ Hz = gm(Ho + 2 * N);
-    const double hx0 = ld_s<NT>(Hxi + c), hy0 = ld_s<NT>(Hyi + c), hz0 = ld_s<NT>(Hzi + c);
-    const double z0 = Ez[c], zyp1 = Ez[c + sy], zyp2 = Ez[c + 2 * sy], zym1 = Ez[c - sy];
-    const double zxp1 = Ez[c + 1], zxp2 = Ez[c + 2], zxm1 = Ez[c - 1];
-    const double y0 = Ey[c], yzp1 = Ey[c + sz], yzp2 = Ey[c + 2 * sz], yzm1 = Ey[c - sz];
-    const double yxp1 = Ey[c + 1], yxp2 = Ey[c + 2], yxm1 = Ey[c - 1];
-    const double x0 = Ex[c], xzp1 = Ex[c + sz], xzp2 = Ex[c + 2 * sz], xzm1 = Ex[c - sz];
-    const double xyp1 = Ex[c + sy], xyp2 = Ex[c + 2 * sy], xym1 = Ex[c - sy];
-    const double khdx = gc(S.prof[0])[PR_KHD * ix + i];
-    const double khdy = gc(S.prof[1])[PR_KHD * iy + jj];
-    const double khdz = gc(S.prof[2])[PR_KHD * iz + k];
-    const double c1 = S.c1, c2 = S.c2;
-    const double db = S.dt / S.mu0 / 1.0;
-    const double ezy = c1 * zyp1 - c1 * z0 + c2 * zyp2 - c2 * zym1;
-    const double eyz = c1 * yzp1 - c1 * y0 + c2 * yzp2 - c2 * yzm1;
-    const double exz = c1 * xzp1 - c1 * x0 + c2 * xzp2 - c2 * xzm1;
-    const double ezx = c1 * zxp1 - c1 * z0 + c2 * zxp2 - c2 * zxm1;
-    const double eyx = c1 * yxp1 - c1 * y0 + c2 * yxp2 - c2 * yxm1;
-    const double exy = c1 * xyp1 - c1 * x0 + c2 * xyp2 - c2 * xym1;
-    const double cux = ezy / khdy - eyz / khdz;
-    const double cuy = exz / khdz - ezx / khdx;
-    const double cuz = eyx / khdx - exy / khdy;
-    st_s<NT>(Hx + c, sign > 0 ? hx0 - db * cux : hx0 + db * cux);
-    st_s<NT>(Hy + c, sign > 0 ? hy0 - db * cuy : hy0 + db * cuy);
-    st_s<NT>(Hz + c, sign > 0 ? hz0 - db * cuz : hz0 + db * cuz);
+    if (q.own) {
+        lds_put(sh, q.a, x0);
+        lds_put(sh + PT_TILE, q.a, y0);
+        lds_put(sh + 2 * PT_TILE, q.a, z0);
+    }
+    if (q.halo)
+        lds_put(sh, q.ha, hv);
+    __syncthreads();
+    // the step is looked up behind the loads (it costs two dependent scalar
+    // loads): a shot that has finished its time loop stores nothing
+    const int n = chunk_step(S) + j;
+    if (n >= S.it - 1 || !q.own || q.i >= S.ix || q.jj >= T.yend)
+        return;
+    if (T.region && q.i >= S.lo[0] && q.i < S.hi[0] && q.jj >= S.lo[1] && q.jj < S.hi[1])
+        return;   // cells of the LDS kernels' region are theirs
+    // cells no range holds stay as they are; written to another buffer they are
+    // copied, so that a replay's stored states are complete
+    if (!S.hstride && shell && !(fl & (FL_UHX | FL_UHY | FL_UHZ | FL_PHX | FL_PHY | FL_PHZ)))
+        return;
+
+    // ---- arithmetic
+    const double c1 = S.c1, c2 = S.c2, dtm = S.dtm;
+    const double *sx = sh, *sy = sh + PT_TILE, *sz = sh + 2 * PT_TILE;
+    const unsigned am1 = q.a - q.p, ap1 = q.a + q.p, ap2 = ap1 + q.p;
+    const double ezy = dp(lds_at(sz, ap1), z0, lds_at(sz, ap2), lds_at(sz, am1), c1, c2);
+    const double eyz = dp(yzp1, y0, yzp2, yzm1, c1, c2);
+    const double exz = dp(xzp1, x0, xzp2, xzm1, c1, c2);
+    const double ezx = dp(lds_at(sz, q.a, 8), z0, lds_at(sz, q.a, 16), lds_at(sz, q.a, -8), c1, c2);
+    const double eyx = dp(lds_at(sy, q.a, 8), y0, lds_at(sy, q.a, 16), lds_at(sy, q.a, -8), c1, c2);
+    const double exy = dp(lds_at(sx, ap1), x0, lds_at(sx, ap2), lds_at(sx, am1), c1, c2);
+    const double cux = ezy / Y.k - eyz / Z.k;
+    const double cuy = exz / Z.k - ezx / X.k;
+    const double cuz = eyx / X.k - exy / Y.k;
+    if (!shell) {
+        hx = hx - dtm * cux;
+        hy = hy - dtm * cuy;
+        hz = hz - dtm * cuz;
+    } else {
+        // db = dt/mu0/(1 + s) and da = (1 - s)/(1 + s) with s = msig dt/(2 eps');
+        // exactly dt/mu0 and 1 where an axis' magnetic CPML sigma is zero
+        const double dt = S.dt;
+        double dax = 1.0, day = 1.0, daz = 1.0, dbx = dtm, dby = dtm, dbz = dtm;
+        if (ax && X.s != 0.0) {
+            const double sm = X.s * dt / (2.0 * mat);
+            dbx = dtm / (1.0 + sm);
+            dax = (1.0 - sm) / (1.0 + sm);
+        }
+        if (ay && Y.s != 0.0) {
+            const double sm = Y.s * dt / (2.0 * mat);
+            dby = dtm / (1.0 + sm);
+            day = (1.0 - sm) / (1.0 + sm);
+        }
+        if (az && Z.s != 0.0) {
+            const double sm = Z.s * dt / (2.0 * mat);
+            dbz = dtm / (1.0 + sm);
+            daz = (1.0 - sm) / (1.0 + sm);
+        }
+        hx = (fl & FL_UHX) ? dax * hx - dbx * cux : hx;
+        hy = (fl & FL_UHY) ? day * hy - dby * cuy : hy;
+        hz = (fl & FL_UHZ) ? daz * hz - dbz * cuz : hz;
+        if (ax && (fl & FL_PHX)) {
+            const double h = S.dl[0];
+            ax0 = X.b * ax0 + X.c * ezx / h;
+            ax1 = X.b * ax1 + X.c * eyx / h;
+            hy += dby * ax0;
+            hz -= dbz * ax1;
+        }
+        if (ay && (fl & FL_PHY)) {
+            const double h = S.dl[1];
+            ay0 = Y.b * ay0 + Y.c * exy / h;
+            ay1 = Y.b * ay1 + Y.c * ezy / h;
+            hz += dbz * ay0;
+            hx -= dbx * ay1;
+        }
+        if (az && (fl & FL_PHZ)) {
+            const double h = S.dl[2];
+            az0 = Z.b * az0 + Z.c * eyz / h;
+            az1 = Z.b * az1 + Z.c * exz / h;
+            hx += dbx * az0;
+            hy -= dby * az1;
+        }
+        if (ax && (fl & FL_PHX)) {
+            put_s<NT>(mb(S.psi[0] + pw) + b0, q0, ax0);
+            put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, ax1);
+        }
+        if (ay && (fl & FL_PHY)) {
+            put_s<NT>(mb(S.psi[1] + pw) + b1, q1, ay0);
+            put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, ay1);
+        }
+        if (az && (fl & FL_PHZ)) {
+            put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, az0);
+            put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, az1);
+        }
+    }
+    const gmp Hout = mb(hsel(S, j + 1, hf)) + kp;
+    put_s<NT>(Hout, q.o, hx);
+    put_s<NT>(Hout + nb, q.o, hy);
+    put_s<NT>(Hout + 2 * nb, q.o, hz);
 }
 
-hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j, int sign,
-                           hipStream_t st, bool rec_prev, int hf, bool nt)
+hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j, hipStream_t st,
+                           bool rec_prev, int hf, bool nt)
 {
     if (nblocks <= 0)
         return rec_prev ? hipErrorInvalidValue : hipSuccess;
     const int recn = rec_prev && j > 0 ? (ns + 7) & ~7 : 0;
     if (nt)
-        hipLaunchKernelGGL(k_efield_f<true>, dim3(recn + nblocks), dim3(ZX * ZY), 0, st, d, ns, pre, j,
-                           sign, recn, hf);
+        hipLaunchKernelGGL(k_efield_f<true>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
     else
-        hipLaunchKernelGGL(k_efield_f<false>, dim3(recn + nblocks), dim3(ZX * ZY), 0, st, d, ns, pre, j,
-                           sign, recn, hf);
+        hipLaunchKernelGGL(k_efield_f<false>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
     return hipGetLastError();
 }
 
-hipError_t launch_hfield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j, int sign,
-                           hipStream_t st, int hf, bool nt)
+hipError_t launch_hfield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j, hipStream_t st,
+                           int hf, bool nt)
 {
     if (nblocks <= 0)
         return hipSuccess;
     if (nt)
-        hipLaunchKernelGGL(k_hfield_f<true>, dim3(nblocks), dim3(ZX * ZY), 0, st, d, ns, pre, j, sign, hf);
+        hipLaunchKernelGGL(k_hfield_f<true>, dim3(nblocks), dim3(PT), 0, st, d, ns, pre, j, hf);
     else
-        hipLaunchKernelGGL(k_hfield_f<false>, dim3(nblocks), dim3(ZX * ZY), 0, st, d, ns, pre, j, sign, hf);
+        hipLaunchKernelGGL(k_hfield_f<false>, dim3(nblocks), dim3(PT), 0, st, d, ns, pre, j, hf);
     return hipGetLastError();
 }
 
@@ -2243,8 +2483,10 @@ __global__ __launch_bounds__(256) void k_efield_p(const ShotDev *__restrict__ D,
     const bool inner =
         i >= nc && i + 1 < ix - nc && jj >= nc && jj < iy - nc && k >= nc && k < iz - nc;
     if (!__all(inner)) {
-        efield_cell<M_UPD | M_PSI | M_SRC>(S, hsel(S, 0, 0), i, jj, k, n, si, so, sign);
-        efield_cell<M_UPD | M_PSI | M_SRC>(S, hsel(S, 0, 0), i + 1, jj, k, n, si, so, sign);
+        for (int d = 0; d < 2; ++d)
+            efield_cell<M_UPD | M_PSI | M_SRC>(S, hsel(S, 0, 0), i + d, jj, k,
+                                               (unsigned)(jj * ix + i + d) * 8u,
+                                               flags(S, i + d, jj, k), n, si, so, sign);
         return;
     }
     const size_t N = (size_t)S.n;
@@ -2328,8 +2570,9 @@ __global__ __launch_bounds__(256) void k_hfield_p(const ShotDev *__restrict__ D,
         i >= nc && i + 1 < ix - nc && jj >= nc && jj < iy - nc && k >= nc && k < iz - nc;
     if (!__all(inner)) {
         double *H = hsel(S, 0, 0);
-        hfield_cell<M_UPD | M_PSI>(S, H, H, i, jj, k, so, sign);
-        hfield_cell<M_UPD | M_PSI>(S, H, H, i + 1, jj, k, so, sign);
+        for (int d = 0; d < 2; ++d)
+            hfield_cell<M_UPD | M_PSI>(S, H, H, i + d, jj, k, (unsigned)(jj * ix + i + d) * 8u,
+                                       flags(S, i + d, jj, k), so, sign);
         return;
     }
     const size_t N = (size_t)S.n;
@@ -2401,39 +2644,29 @@ hipError_t launch_hfield_p(const ShotDev *d, int ns, const int *pre, int nblocks
     return hipGetLastError();
 }
 
-#define LAUNCH_E(M)                                                                          \
-    hipLaunchKernelGGL(k_efield<M>, dim3(nblocks), dim3(TX, TY), 0, st, d, ns, pre, j, nover, \
-                       sign)
-hipError_t launch_efield(int mode, const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                         int nover, int sign, hipStream_t st)
+hipError_t launch_efield(int mode, const ShotDev *d, int nblocks, int sign, hipStream_t st)
 {
     if (nblocks <= 0)
         return hipSuccess;
-    switch (mode) {
-    case M_UPD | M_PSI | M_SRC: LAUNCH_E(M_UPD | M_PSI | M_SRC); break;
-    case M_UPD | M_PSI: LAUNCH_E(M_UPD | M_PSI); break;
-    case M_UPD | M_INPLACE: LAUNCH_E(M_UPD | M_INPLACE); break;
-    case M_PSI | M_INPLACE: LAUNCH_E(M_PSI | M_INPLACE); break;
-    case M_UPD | M_PSI | M_INPLACE: LAUNCH_E(M_UPD | M_PSI | M_INPLACE); break;
-    default: return hipErrorInvalidValue;
-    }
+    if (mode == (M_UPD | M_INPLACE))
+        hipLaunchKernelGGL((k_efield<M_UPD | M_INPLACE>), dim3(nblocks), dim3(PT), 0, st, d, sign);
+    else if (mode == (M_PSI | M_INPLACE))
+        hipLaunchKernelGGL((k_efield<M_PSI | M_INPLACE>), dim3(nblocks), dim3(PT), 0, st, d, sign);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
-#define LAUNCH_H(M) \
-    hipLaunchKernelGGL(k_hfield<M>, dim3(nblocks), dim3(TX, TY), 0, st, d, ns, pre, j, sign)
-hipError_t launch_hfield(int mode, const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                         int sign, hipStream_t st)
+hipError_t launch_hfield(int mode, const ShotDev *d, int nblocks, int sign, hipStream_t st)
 {
     if (nblocks <= 0)
         return hipSuccess;
-    switch (mode) {
-    case M_UPD | M_PSI: LAUNCH_H(M_UPD | M_PSI); break;
-    case M_UPD | M_INPLACE: LAUNCH_H(M_UPD | M_INPLACE); break;
-    case M_PSI | M_INPLACE: LAUNCH_H(M_PSI | M_INPLACE); break;
-    case M_UPD | M_PSI | M_INPLACE: LAUNCH_H(M_UPD | M_PSI | M_INPLACE); break;
-    default: return hipErrorInvalidValue;
-    }
+    if (mode == (M_UPD | M_INPLACE))
+        hipLaunchKernelGGL((k_hfield<M_UPD | M_INPLACE>), dim3(nblocks), dim3(PT), 0, st, d, sign);
+    else if (mode == (M_PSI | M_INPLACE))
+        hipLaunchKernelGGL((k_hfield<M_PSI | M_INPLACE>), dim3(nblocks), dim3(PT), 0, st, d, sign);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -1,0 +1,95 @@
+"""Tiles of the per-cell forward kernels: every tile shape the host picks (16
+to 38 columns), rows and columns cut by the grid's edges, planes of less than
+one tile, and the thinnest CPML, against the oracle bit for bit: all six fields
+and the traces, in place and with E in ring slots, per operator and fused."""
+import numpy as np
+import pytest
+
+import oracle
+from mittet_main_amd import Grid, Model, firstderiv_gauss
+from mittet_main_amd.adjoint import GradientProblem, ShotSpec
+from mittet_main_amd.configs import dt_for
+
+pytestmark = pytest.mark.gpu
+
+OM0 = 2 * np.pi
+# ix, iy, iz, ncpml: a plane below one tile; one cell more or less than a
+# tile's columns or rows; sizes with tiles of 16, 21, 28, 32, 36 columns
+GRIDS = [(8, 8, 8, 2), (9, 31, 8, 2), (17, 13, 9, 2), (21, 12, 11, 3), (22, 37, 13, 3),
+         (33, 24, 14, 5), (43, 25, 12, 4), (71, 20, 15, 5), (96, 19, 12, 4), (131, 11, 12, 3)]
+
+
+@pytest.mark.parametrize("ring", [0, 5])
+@pytest.mark.parametrize("dims", GRIDS)
+def test_tiles_bitwise(dims, ring):
+    ix, iy, iz, nc = dims
+    print(f"tiles {dims} ring {ring}", flush=True)
+    rng = np.random.default_rng(ix + iy)
+    sig = np.exp(rng.uniform(np.log(0.05), np.log(3.0), (iz, iy, ix)))
+    dl = (50.0, 45.0, 40.0)
+    dt, cmax = dt_for(*dl, sig_min=0.05)
+    it = 17
+    signal = firstderiv_gauss(it, dt, 0.5 / dt / it)
+    src = (ix // 2, iy // 2, iz // 2)
+    rec = np.array([[1, 1, 1], [ix - 2, iy - 2, iz - 2], [ix // 2, iy - 3, iz // 2]], np.int32)
+    m = Model(Grid(ix, iy, iz, nc, *dl, dt, OM0, cmax))
+    m.media_coeff_3d(sig)
+    S = oracle.OracleSim(ix, iy, iz, nc, *dl, dt, OM0, cmax)
+    S.set_sigma(sig)
+    S.init_cpml()
+    S.media_coeff_3d()
+    # fields of every magnitude at the edges too: random, the same on both sides
+    shot = m.shot(it, signal, src, 1, rec, [3.0] if ring else None, ring)
+    for q, nm in enumerate(oracle.FIELD_NAMES):
+        v = rng.standard_normal((iz, iy, ix))
+        shot.set_field(q, v)
+        S.arr(nm)[...] = v
+    src1 = tuple(c + 1 for c in src)
+    if ring:
+        shot.step_n(7)
+    else:   # three steps by the single operators, which advance no step counter
+        for n in range(3):
+            shot.e_field_cpml42()
+            shot.epml_abcs4()
+            shot.read_source_3d(n)
+            shot.h_field_cpml42()
+            shot.hpml_abcs4()
+        S.forward(1, signal, src1, 3)
+    shot.run()
+    tr, _ = S.forward(1, signal, src1, it - 1, rec1=rec + 1, it=it)
+    np.testing.assert_array_equal(shot.traces()[:3, :, : it - 1], tr[:, :, : it - 1])
+    for q, nm in enumerate(oracle.FIELD_NAMES):
+        np.testing.assert_array_equal(shot.field(q), S.arr(nm), err_msg=nm)
+    m.close()
+
+
+def test_replayed_states_are_complete():
+    """A replay writes each state to memory no step has written before; H cells
+    outside every update range are part of it.  The gradient is the same
+    whatever the memory held: before and after NaN fields lived there."""
+    ix, iy, iz, nc, it = 30, 27, 25, 5, 40
+    dt, cmax = dt_for(50.0, 45.0, 40.0, sig_min=0.1)
+    g = Grid(ix, iy, iz, nc, 50.0, 45.0, 40.0, dt, OM0, cmax)
+    sig = np.exp(np.random.default_rng(5).uniform(np.log(0.1), np.log(2.0), g.shape))
+
+    def gradient():
+        P = GradientProblem(g, [ShotSpec((15, 13, 12), firstderiv_gauss(it, dt, 0.2 / dt))],
+                            [[9, 9, 9], [20, 12, 14]], it, [6.0])
+        P.d_obs = [np.zeros((3, 2, 1))]
+        out = P.value_and_grad(np.log(sig))
+        P.close()
+        return out
+
+    J0, g0 = gradient()
+    m = Model(g)
+    m.media_coeff_3d(sig)
+    poison = [m.shot(it, None, ring=r, omega_vol=[1.0] if r else None) for r in (0, 8, 16)]
+    for s in poison:
+        for q in range(6):
+            s.set_field(q, np.full(g.shape, np.nan))
+        s.run()
+        s.sync()
+    m.close()
+    J1, g1 = gradient()
+    assert J0 == J1 and np.all(np.isfinite(g1))
+    np.testing.assert_array_equal(g0, g1)
