@@ -538,29 +538,28 @@ struct Fam {
     bool nt;      // E/H launches with non-temporal once-touched values (stream_nt)
 };
 
-// Families whose E half-step has a per-cell launch that can carry the
-// receiver gather of the previous step.  Only where every shot has a ring of
-// more than one slot: step j reads slot (cur + j) % ring and writes the next
-// one, so the gather of step j - 1 (slot (cur + j) % ring) is not written by
-// that launch.  With one slot E is updated in place, and the leading gather
-// blocks would race the tile blocks that overwrite it.
+// Families whose per-cell launches can carry the receiver gathers of a chunk's
+// steps but its last (see k_efield_f): E and H of step j - 1 with the E launch of
+// step j where every shot keeps E in a ring of more than one slot; with one slot
+// E of step j goes with its H launch and H with the next E launch.
 bool rec_folds(const Fam &f)
 {
-    return (f.kind == 0 || f.kind == 3) && f.nblocks > 0 && f.rings;
+    return (f.kind == 0 || f.kind == 3 || f.kind == 4) && f.nblocks > 0;
 }
 
-// rec_prev: the E launch of step j also gathers step j - 1's receivers
-// (rec_folds(f) must hold).  Fused family 3: the E half-step is the shell E
-// launch plus the fused E+H interior launch, the H half-step the shell H
-// launch alone.
+// rec_prev, rec_here (rec_folds(f) must hold): the gathers of step j - 1 go with
+// the E launch, and the E gather of step j with the H launch of shots without
+// rings.  Fused family 3: the E half-step is the shell E launch plus the fused
+// E+H interior launch, the H half-step the shell H launch alone.
 int launch_eh(const Fam &f, const ShotDev *d, int ns, int j, bool h, hipStream_t st,
-              bool rec_prev = false)
+              bool rec_prev = false, bool rec_here = false)
 {
     hipError_t e;
+    const bool e_here = rec_here && (!f.rings || f.kind == 4);
     if (f.kind == 4) {
         if (!h)
-            HIP_TRY(mt::launch_source_hz(d, ns, j, st));
-        e = h ? mt::launch_hfield_v(d, ns, f.pre, f.nblocks, j, st)
+            HIP_TRY(mt::launch_source_hz(d, ns, j, st, rec_prev));
+        e = h ? mt::launch_hfield_v(d, ns, f.pre, f.nblocks, j, st, e_here)
               : mt::launch_efield_v(d, ns, f.pre, f.nblocks, j, st);
         HIP_TRY(e);
         return FWI3D_OK;
@@ -572,8 +571,8 @@ int launch_eh(const Fam &f, const ShotDev *d, int ns, int j, bool h, hipStream_t
         e = h ? mt::launch_hfield_p(d, ns, f.pre, f.nblocks, j, 1, st)
               : mt::launch_efield_p(d, ns, f.pre, f.nblocks, j, 1, st);
     else
-        e = h ? mt::launch_hfield_f(d, ns, f.pre, f.nblocks, j, st, f.fused, f.nt)
-              : mt::launch_efield_f(d, ns, f.pre, f.nblocks, j, st, rec_prev, f.fused, f.nt);
+        e = h ? mt::launch_hfield_f(d, ns, f.pre, f.nblocks, j, st, e_here, f.fused, f.nt)
+              : mt::launch_efield_f(d, ns, f.pre, f.nblocks, j, st, rec_prev, f.rings, f.fused, f.nt);
     HIP_TRY(e);
     if (f.kind == 3 && f.fused) {
         if (!h)
@@ -590,11 +589,11 @@ int launch_chunk(const ShotDev *d, int ns, const Fam &f, const int *pre_cells, i
                  int L, bool any_dft, bool any_rec, hipStream_t st, bool any_hdft = false)
 {
     int rc;
-    const bool fold = any_rec && rec_folds(f);   // step j's gather rides on step j + 1's E launch
+    const bool fold = any_rec && rec_folds(f);   // gathers ride on the steps' launches
     const int hf = f.fused ? 1 : 0;
     for (int j = 0; j < L; ++j) {
         if ((rc = launch_eh(f, d, ns, j, false, st, fold && j > 0)) ||
-            (rc = launch_eh(f, d, ns, j, true, st)))
+            (rc = launch_eh(f, d, ns, j, true, st, false, fold && j + 1 < L)))
             return rc;
         if (any_rec && !(fold && j + 1 < L))
             HIP_TRY(mt::launch_receivers(d, ns, j, -1, 0, st, hf));
@@ -2128,7 +2127,7 @@ static int replay_segment(fwi3d_grad *g, int L)
         int rc = FWI3D_OK;
         for (int j = 0; j < L && !rc; ++j) {
             if ((rc = launch_eh(f, g->d_rdesc, 1, j, false, s->st, fold && j > 0)) ||
-                (rc = launch_eh(f, g->d_rdesc, 1, j, true, s->st)))
+                (rc = launch_eh(f, g->d_rdesc, 1, j, true, s->st, false, fold && j + 1 < L)))
                 break;
             if (s->nrec && !(fold && j + 1 < L) &&
                 mt::launch_receivers(g->d_rdesc, 1, j, -1, 0, s->st) != hipSuccess)

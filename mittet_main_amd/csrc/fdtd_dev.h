@@ -189,14 +189,17 @@ hipError_t launch_efield_z(const ShotDev *d, int ns, const int *pre, int nblocks
                            int sign, hipStream_t st);
 hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                            int sign, hipStream_t st);
-// rec_prev (j > 0): ns more blocks gather the receivers of local step j - 1.
+// rec_prev (j > 0): ns more blocks gather the receivers of local step j - 1: H,
+// and E too if rec_e (every shot with E in ring slots).  The H launch's rec_e:
+// they gather E of step j itself (shots that update E in place).
 // hf: part of a fused E+H step (H read from hsel(S, j, 1), written to
 // hsel(S, j + 1, 1)); 0: H updated in place.  nt (also for the _l launches):
 // the once-touched field values go non-temporal (M_NT).
 hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           hipStream_t st, bool rec_prev = false, int hf = 0, bool nt = false);
+                           hipStream_t st, bool rec_prev = false, bool rec_e = true, int hf = 0,
+                           bool nt = false);
 hipError_t launch_hfield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           hipStream_t st, int hf = 0, bool nt = false);
+                           hipStream_t st, bool rec_e = false, int hf = 0, bool nt = false);
 hipError_t launch_efield_p(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                            int sign, hipStream_t st);
 hipError_t launch_hfield_p(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
@@ -211,12 +214,14 @@ hipError_t launch_hfield_l(const ShotDev *d, int ns, const int *pre, int nblocks
 hipError_t launch_ehfield_l(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                             hipStream_t st);
 // Fortran-variant step (fdtd_fortran.hip): Hz source points before the E
-// update, then per-cell E + CPML-E and H + CPML-H over 32 x 8 tiles
-hipError_t launch_source_hz(const ShotDev *d, int ns, int j, hipStream_t st);
+// update (rec_prev, j > 0: after the H receivers of local step j - 1), then
+// per-cell E + CPML-E and H + CPML-H over 32 x 8 tiles (rec_e: the H launch also
+// gathers the E receivers of step j)
+hipError_t launch_source_hz(const ShotDev *d, int ns, int j, hipStream_t st, bool rec_prev = false);
 hipError_t launch_efield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                            hipStream_t st);
 hipError_t launch_hfield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           hipStream_t st);
+                           hipStream_t st, bool rec_e = false);
 hipError_t launch_receivers(const ShotDev *d, int ns, int j, int nover, int inplace,
                             hipStream_t st, int hf = 0);
 // h: the H ring into acc_h (shots with H sums) instead of the E ring into acc

@@ -82,15 +82,29 @@ __device__ __forceinline__ bool h_shell(int r, int n, int nc)
 
 }  // namespace
 
-// Hz(src) -= s[n] dt / mu(src) / dx / dy / dz for each point, in order
-__global__ void k_source_hz(const ShotDev *__restrict__ D, int ns, int j)
+// Trace samples of step n, components [c0, c0 + 3) of Ex .. Hz, from F [3][n]
+__device__ __forceinline__ void rec_v(const ShotDev &S, int n, const double *F, int c0)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= ns)
-        return;
-    const ShotDev &S = D[s];
+    for (int q = threadIdx.x; q < 3 * S.nrec; q += blockDim.x) {
+        const int comp = q / S.nrec, r = q - comp * S.nrec;
+        const double v = cg(F)[(size_t)comp * S.n + S.rec_cell[r]];
+        mg(S.traces)[((size_t)(c0 + comp) * S.nrec + r) * S.it + n] = v;
+        if (!__builtin_isfinite(v))
+            *S.flag = 1;
+    }
+}
+
+// One block per shot: with rec, H at the receivers after local step j - 1 (no
+// launch has written H since); then Hz(src) -= s[n] dt / mu(src) / dx / dy / dz
+// for each point, in order
+__global__ __launch_bounds__(256) void k_source_hz(const ShotDev *__restrict__ D, int j, int rec)
+{
+    const ShotDev &S = D[blockIdx.x];
     const int n = *S.step + j;
-    if (n >= S.it - 1 || S.nsrc_h <= 0)
+    if (rec && n - 1 < S.it - 1)
+        rec_v(S, n - 1, S.h, 3);
+    __syncthreads();
+    if (threadIdx.x || n >= S.it - 1)
         return;
     GLOBAL double *Hz = mg(S.h + 2 * (size_t)S.n);
     for (int q = 0; q < S.nsrc_h && q < 4; ++q)
@@ -182,15 +196,27 @@ __global__ __launch_bounds__(ZX *ZY) void k_efield_v(const ShotDev *__restrict__
     Eout[2 * N + c] = ez;
 }
 
+// The first recn blocks gather E of step j at the receivers, block s for shot s
+// (E is not written by this launch).
 __global__ __launch_bounds__(ZX *ZY) void k_hfield_v(const ShotDev *__restrict__ D, int ns,
-                                                     const int *__restrict__ pre, int j)
+                                                     const int *__restrict__ pre, int j, int recn)
 {
-    const int s = shot_of(pre, ns, blockIdx.x);
+    if ((int)blockIdx.x < recn) {
+        if ((int)blockIdx.x < ns) {
+            const ShotDev &R = D[blockIdx.x];
+            const int n = *R.step + j;
+            if (n < R.it - 1)
+                rec_v(R, n, R.e + (size_t)((R.cur + j + 1) % R.ring) * R.sstride, 0);
+        }
+        return;
+    }
+    const int b = blockIdx.x - recn;
+    const int s = shot_of(pre, ns, b);
     const ShotDev &S = D[s];
     if (*S.step + j >= S.it - 1)
         return;
     int i, jj, k;
-    if (!vcell(S, blockIdx.x - pre[s], i, jj, k))
+    if (!vcell(S, b - pre[s], i, jj, k))
         return;
     const int ix = S.ix, iy = S.iy, iz = S.iz, nc = S.nc;
     const size_t N = (size_t)S.n, sy = ix, sz = (size_t)ix * iy;
@@ -267,9 +293,9 @@ __global__ __launch_bounds__(ZX *ZY) void k_hfield_v(const ShotDev *__restrict__
     Hz[c] = hz;
 }
 
-hipError_t launch_source_hz(const ShotDev *d, int ns, int j, hipStream_t st)
+hipError_t launch_source_hz(const ShotDev *d, int ns, int j, hipStream_t st, bool rec_prev)
 {
-    hipLaunchKernelGGL(k_source_hz, dim3((ns + 63) / 64), dim3(64), 0, st, d, ns, j);
+    hipLaunchKernelGGL(k_source_hz, dim3(ns), dim3(256), 0, st, d, j, rec_prev && j > 0 ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -283,11 +309,12 @@ hipError_t launch_efield_v(const ShotDev *d, int ns, const int *pre, int nblocks
 }
 
 hipError_t launch_hfield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           hipStream_t st)
+                           hipStream_t st, bool rec_e)
 {
     if (nblocks <= 0)
-        return hipSuccess;
-    hipLaunchKernelGGL(k_hfield_v, dim3(nblocks), dim3(ZX * ZY), 0, st, d, ns, pre, j);
+        return rec_e ? hipErrorInvalidValue : hipSuccess;
+    const int recn = rec_e ? (ns + 7) & ~7 : 0;
+    hipLaunchKernelGGL(k_hfield_v, dim3(recn + nblocks), dim3(ZX * ZY), 0, st, d, ns, pre, j, recn);
     return hipGetLastError();
 }
 

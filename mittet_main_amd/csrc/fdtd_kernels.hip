@@ -535,11 +535,12 @@ __global__ void k_source(const ShotDev *__restrict__ D, int n)
 }
 
 // Trace samples of step n: E from ring slot so and H from buffer H, one block
-// per shot.
-__device__ __forceinline__ void rec_store(const ShotDev &S, int n, int so, const double *H)
+// per shot; the components [c0, c1) of Ex .. Hz.
+__device__ __forceinline__ void rec_store(const ShotDev &S, int n, int so, const double *H, int c0 = 0,
+                                          int c1 = 6)
 {
-    const int tot = 6 * S.nrec;
-    for (int q = threadIdx.x; q < tot; q += blockDim.x) {
+    const int tot = c1 * S.nrec;
+    for (int q = c0 * S.nrec + threadIdx.x; q < tot; q += blockDim.x) {
         const int comp = q / S.nrec, r = q - comp * S.nrec;
         const int cell = S.rec_cell[r];
         const double v = comp < 3 ? S.e[(size_t)so * S.sstride + (size_t)comp * S.n + cell]
@@ -1378,15 +1379,20 @@ __device__ __forceinline__ void lds_put(double *b, unsigned o, double v)
 }  // namespace
 
 // The first recn blocks (recn: 0, or ns rounded up to a multiple of 8 so that
-// the tile blocks keep their XCD) gather the receivers of the previous local
-// step j - 1, block s for shot s: its E slot is the one this step reads and H
-// is not written until the H half-step, so the samples are the ones a receiver
-// launch after step j - 1 takes, with one graph node less per step.  Leading,
-// they overlap the tile blocks instead of trailing the launch.  hf: the step
-// is a fused E+H launch sequence (H before step j is hsel(S, j, 1)).
+// the tile blocks keep their XCD) gather receivers, block s for shot s, with one
+// graph node less per step than a launch of their own (4.6 us at 131 x 97 x 75
+// with 25 receivers, 9.4 us at 288^3 with 256).  Leading, they overlap the tile
+// blocks instead of trailing the launch.  An E launch gathers what the launch
+// does not write: H of the previous local step j - 1 (H is not written until the
+// H half-step), and with E in ring slots (rec_e) also E of that step, which is
+// the slot this step reads.  With one slot, E is overwritten by that launch, so
+// the H launch of the step itself gathers E.  The samples are the ones a
+// receiver launch after the step takes.  hf: the step is a fused E+H launch
+// sequence (H before step j is hsel(S, j, 1)).
 template <bool NT>
 __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, int ns,
-                                                 const int *__restrict__ pre, int j, int recn, int hf)
+                                                 const int *__restrict__ pre, int j, int recn, int rec_e,
+                                                 int hf)
 {
     __shared__ double sh[3 * PT_TILE];
     if ((int)blockIdx.x < recn) {
@@ -1394,7 +1400,7 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
             const ShotDev &R = D[blockIdx.x];
             const int n = chunk_step(R) + j - 1;
             if (n < R.it - 1)
-                rec_store(R, n, (R.cur + j) % R.ring, hsel(R, j, hf));
+                rec_store(R, n, (R.cur + j) % R.ring, hsel(R, j, hf), rec_e ? 0 : 3);
         }
         return;
     }
@@ -1579,10 +1585,19 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
 
 template <bool NT>
 __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, int ns,
-                                                 const int *__restrict__ pre, int j, int hf)
+                                                 const int *__restrict__ pre, int j, int recn, int hf)
 {
     __shared__ double sh[3 * PT_TILE];
-    const int b = blockIdx.x;
+    if ((int)blockIdx.x < recn) {
+        if ((int)blockIdx.x < ns) {
+            const ShotDev &R = D[blockIdx.x];
+            const int n = chunk_step(R) + j;
+            if (n < R.it - 1)
+                rec_store(R, n, (R.cur + j + 1) % R.ring, nullptr, 0, 3);
+        }
+        return;
+    }
+    const int b = blockIdx.x - recn;
     const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
     FTile T;
@@ -1756,28 +1771,33 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     put_s<NT>(Hout + 2 * nb, q.o, hz);
 }
 
+static int rec_blocks(bool rec, int ns) { return rec ? (ns + 7) & ~7 : 0; }
+
 hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j, hipStream_t st,
-                           bool rec_prev, int hf, bool nt)
+                           bool rec_prev, bool rec_e, int hf, bool nt)
 {
     if (nblocks <= 0)
         return rec_prev ? hipErrorInvalidValue : hipSuccess;
-    const int recn = rec_prev && j > 0 ? (ns + 7) & ~7 : 0;
+    const int recn = rec_blocks(rec_prev && j > 0, ns);
     if (nt)
-        hipLaunchKernelGGL(k_efield_f<true>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
+        hipLaunchKernelGGL(k_efield_f<true>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn,
+                           rec_e ? 1 : 0, hf);
     else
-        hipLaunchKernelGGL(k_efield_f<false>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
+        hipLaunchKernelGGL(k_efield_f<false>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn,
+                           rec_e ? 1 : 0, hf);
     return hipGetLastError();
 }
 
 hipError_t launch_hfield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j, hipStream_t st,
-                           int hf, bool nt)
+                           bool rec_e, int hf, bool nt)
 {
     if (nblocks <= 0)
-        return hipSuccess;
+        return rec_e ? hipErrorInvalidValue : hipSuccess;
+    const int recn = rec_blocks(rec_e, ns);
     if (nt)
-        hipLaunchKernelGGL(k_hfield_f<true>, dim3(nblocks), dim3(PT), 0, st, d, ns, pre, j, hf);
+        hipLaunchKernelGGL(k_hfield_f<true>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
     else
-        hipLaunchKernelGGL(k_hfield_f<false>, dim3(nblocks), dim3(PT), 0, st, d, ns, pre, j, hf);
+        hipLaunchKernelGGL(k_hfield_f<false>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
     return hipGetLastError();
 }
 

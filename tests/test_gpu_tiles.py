@@ -93,3 +93,33 @@ def test_replayed_states_are_complete():
     J1, g1 = gradient()
     assert J0 == J1 and np.all(np.isfinite(g1))
     np.testing.assert_array_equal(g0, g1)
+
+
+@pytest.mark.parametrize("members", [1, 3])
+def test_fortran_receivers_on_the_source_cells(members):
+    """H of a step is sampled before the next step's source changes it, alone
+    and in a batch, over chunk borders (32 steps)."""
+    from mittet_main_amd import Batch
+    from tests.test_gpu_fortran import gpu_shot, oracle_run, setup
+
+    nt = 37
+    g, sig, mu, sigw, src, rec, *_ = setup(27, 23, 21, nt=nt)
+    rec = np.concatenate([rec, np.array(src)])
+    _, tr_o = oracle_run(g, sig, mu, sigw, src, rec, nt)
+    m = Model(g, variant=1)
+    m.set_mu(mu)
+    m.media_coeff_3d(sig)
+    shots = [gpu_shot(m, g, sigw, src, rec, nt) for _ in range(members)]
+    if members > 1:
+        b = Batch(members)
+        for s in shots:
+            b.add(s)
+        b.step(nt)
+        b.sync()
+        for s in shots:
+            b.remove(s)
+    else:
+        shots[0].run()
+    for s in shots:
+        np.testing.assert_array_equal(s.traces()[:, :, :nt], tr_o[:, :, :nt])
+    m.close()
