@@ -1992,12 +1992,12 @@ struct fwi3d_grad {
     std::vector<double *> inner;      // depth l >= 1: slots for the starts of a segment's pieces
     double *buf = nullptr;            // leaf + 1 states
     double *adj = nullptr;            // adjoint state (one state)
-    double *tmp = nullptr;            // 3N + psi slabs
+    double *tmp = nullptr;            // region state as weights (2 x 3N), weights of the per-cell
+                                      // passes (2 x 6N)
     double *grad = nullptr;           // N
     double *grad_src = nullptr;       // 1
     double *g = nullptr;              // [it][3][nrec] trace sensitivities
     double *rp = nullptr;             // per axis: 1/ked, 1/khd
-    int kappa_one = 0;                // ked = khd = dl on every axis
     int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};   // LDS region of the adjoint (empty: lo = hi)
     int4 *tiles = nullptr;            // per-cell tiles outside it (ntiles, multiple of 8)
     int ntiles = 0;
@@ -2217,7 +2217,7 @@ static std::vector<int4> adj_tiles(const fwi3d_shot *s)
 static long long grad_plan_bytes(const fwi3d_shot *s, const GradPlan &P)
 {
     const size_t N = (size_t)s->desc.n, st = state_doubles(s);
-    const size_t tmp = st - 3 * N;
+    const size_t tmp = 12 * N;
     const size_t other = tmp + N + 1 + std::max<size_t>(1, 3 * (size_t)s->nrec * s->it) +
                          2 * ((size_t)s->desc.ix + s->desc.iy + s->desc.iz) +
                          2 * adj_tiles(s).size();
@@ -2247,9 +2247,7 @@ static int grad_new(fwi3d_shot *s, int levels, int segment, fwi3d_grad **out)
     g->leaf = g->plan.seglen[levels - 1];
     state_layout(g);
     const size_t N = (size_t)s->desc.n;
-    size_t tmp = 3 * N;
-    for (int a = 0; a < 3; ++a)
-        tmp += mt::PSI_N * (size_t)s->desc.slab[a];
+    const size_t tmp = 12 * N;
     bool ok = dalloc(&g->ckpt, g->state * g->nseg) == hipSuccess;
     for (int l = 1; l < levels && ok; ++l) {
         const size_t pieces =
@@ -2277,7 +2275,6 @@ static int grad_new(fwi3d_shot *s, int levels, int segment, fwi3d_grad **out)
             for (int q = 0; q < n; ++q)
                 rp.push_back(1.0 / s->m->prof[a][(size_t)row * n + q]);
     }
-    g->kappa_one = kappa_is_one(s);
     adj_region(s, g->lo, g->hi);
     const std::vector<int4> tl = adj_tiles(s);
     g->ntiles = (int)tl.size();
@@ -2385,16 +2382,20 @@ static int adj_range(fwi3d_grad *g, int depth, int n0, int L, double *start, mt:
         // replay the segment keeping every state, then step the adjoint back
         if ((rc = state_copy(g, g->buf, true)) || (rc = replay_segment(g, L)))
             return rc;
+        // the H local part of step t runs with step t + 1 (both states at hand),
+        // that of the segment's last step on its own
+        auto state = [&](int t) { return g->buf + g->state * t; };
+        A.H0 = state(L - 1) + g->off_h;
+        A.H1 = state(L) + g->off_h;
+        HIP_TRY(mt::launch_adjoint_local(A, s->st));
         for (int t = L - 1; t >= 0; --t) {
             const int n = n0 + t;
-            const double *u0 = g->buf + g->state * t, *u1 = g->buf + g->state * (t + 1);
-            A.uE0 = u0;
-            A.uH0 = u0 + g->off_h;
-            A.uE1 = u1;
-            for (int a = 0; a < 3; ++a)
-                A.upsi1[a] = u1 + g->off_psi[a];
+            A.E0 = state(t);
+            A.E1 = state(t + 1);
+            A.H0 = state(std::max(t - 1, 0)) + g->off_h;
+            A.H1 = state(t) + g->off_h;
             A.amp_n = amp[n];
-            HIP_TRY(mt::launch_adjoint_step(A, g->g + (size_t)n * 3 * nrec, nrec, s->d_rec, s->st));
+            HIP_TRY(mt::launch_adjoint_step(A, g->g + (size_t)n * 3 * nrec, nrec, s->d_rec, t > 0, s->st));
         }
         return FWI3D_OK;
     }
@@ -2434,6 +2435,7 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
                 gt[((size_t)n * 3 + c) * nrec + r] = djdt[((size_t)c * nrec + r) * it + n];
     HIP_TRY(hipMemcpyAsync(g->g, gt.data(), sizeof(double) * gt.size(), hipMemcpyHostToDevice, s->st));
     HIP_TRY(mt::launch_fill(g->adj, g->state, 0.0, s->st));
+    HIP_TRY(mt::launch_fill(g->tmp, 6 * N, 0.0, s->st));   // uh
     HIP_TRY(mt::launch_fill(g->grad, N, 0.0, s->st));
     HIP_TRY(mt::launch_fill(g->grad_src, 1, 0.0, s->st));
     std::vector<double> amp(it, 0.0);
@@ -2452,12 +2454,21 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
     A.nc = d.nc;
     A.n = d.n;
     A.dt = d.dt;
-    A.mu0 = d.mu0;
+    A.rdt = 1.0 / d.dt;
+    A.dbi = d.dtm;
     A.c1 = d.c1;
     A.c2 = d.c2;
-    A.ftx = tiles(d.ix, mt::ZX);
-    A.fty = tiles(d.iy, mt::ZY);
-    A.fb = A.ftx * A.fty * d.iz;
+    A.row = d.row;
+    A.pb = d.pb;
+    A.tw = d.tw;
+    A.th = d.th;
+    A.ttx = d.ttx;
+    A.tpp = d.tpp;
+    A.xmul = d.xmul;
+    A.tmul = d.tmul;
+    A.xsh = d.xsh;
+    A.tsh = d.tsh;
+    A.fb = d.tpp * d.iz;
     A.fb_pad = tiles(A.fb, 8) * 8;
     A.shell = nullptr;
     for (int a = 0; a < 3; ++a) {
@@ -2475,13 +2486,6 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
         A.lb = A.ltx * A.lty * A.lkz;
         A.lb_pad = tiles(A.lb, 8) * 8;
     }
-    // [nc, n - nc) is free of CPML terms when nc >= 2 (the update ranges start
-    // at index 1 or 2); with a thinner CPML no cell takes the fast paths
-    for (int a = 0; a < 3; ++a) {
-        const int n = a == 0 ? d.ix : (a == 1 ? d.iy : d.iz);
-        A.inner_hi[a] = d.nc >= 2 ? n - d.nc : 0;
-    }
-    A.kappa_one = g->kappa_one;
     const double *rp = g->rp;
     for (int a = 0; a < 3; ++a) {
         const int n = a == 0 ? d.ix : (a == 1 ? d.iy : d.iz);
@@ -2490,6 +2494,7 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
         A.rp[a] = rp;
         rp += 2 * n;
         A.prof[a] = d.prof[a];
+        A.fl[a] = d.fl[a];
         A.slab[a] = d.slab[a];
         A.lpsi[a] = g->adj + g->off_psi[a];
     }
@@ -2497,12 +2502,8 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
     A.cbi = d.cbi;
     A.lE = g->adj;
     A.lH = g->adj + g->off_h;
-    A.t3 = g->tmp;
-    size_t o = 3 * N;
-    for (int a = 0; a < 3; ++a) {
-        A.tpsi[a] = g->tmp + o;
-        o += mt::PSI_N * (size_t)d.slab[a];
-    }
+    A.uh = g->tmp;
+    A.ue = g->tmp + 6 * N;
     A.grad = g->grad;
     A.grad_src = g->grad_src;
     A.src_cell = s->src_cell;

@@ -149,7 +149,11 @@ __host__ __device__ inline double *hsel(const ShotDev &S, int j, int hf)
 // Arguments of one adjoint step (fdtd_adjoint.hip), passed by value.
 struct AdjArgs {
     int ix, iy, iz, nc, n;
-    int ftx, fty, fb, fb_pad;        // 32 x 8 tiles per plane, as the fused forward kernels
+    unsigned row, pb;                // as in ShotDev, with the per-cell tiles
+    int tw, th, ttx, tpp;
+    unsigned xmul, tmul;
+    int xsh, tsh;
+    int fb, fb_pad;
     const int4 *shell;               // non-null: fb tiles {x0, y0, k, yend} of the cells
                                      // outside the LDS region (ShotDev::shell's format)
     // LDS region of the adjoint, [lo, hi) on each axis (empty: lo = hi = 0):
@@ -158,27 +162,32 @@ struct AdjArgs {
     int lo[3], hi[3];
     int ltx, lty, lkz, lb, lb_pad;   // 64 x LY tiles, z-chunks of lkb planes
     int lkb;
-    int inner_hi[3];                 // cells in [nc, inner_hi[a]) on every axis see no CPML term
-    int kappa_one;                   // ked = khd = dl everywhere
-    double dt, mu0, c1, c2;
+    double dt, rdt, dbi, c1, c2;     // rdt = 1/dt, dbi = dt/mu0
     double dl[3], rdl[3];
     const double *prof[3];
+    const int *fl[3];                // range flags (FL_*)
     const double *rp[3];             // per axis: 1/ked (row 0) and 1/khd (row 1)
     const double *eps;
     const double *cbi;               // dt/eps' per cell
     long long slab[3];
-    double *lE, *lH, *lpsi[3];       // adjoint state (forward layout)
-    double *t3, *tpsi[3];            // per-step weights for the transposed stencils
-    const double *uE0, *uH0;         // forward state before the step
-    const double *uE1, *upsi1[3];    // forward state after the step
+    double *lE, *lH, *lpsi[3];       // adjoint state (forward layout); in the region lE and lH
+                                     // hold the weights cb lE and db lH
+    double *uh, *ue;                 // [6][n] weights of the transposed H- and E-phase stencils
+                                     // of the per-cell passes
+    const double *E0, *E1;           // forward E before and after the step
+    const double *H0, *H1;           // forward H before and after the step whose H part is local
     double *grad;                    // dJ/d eps' per cell (accumulated)
     double *grad_src;                // dJ/d sigma[src] from the source scaling
     int src_cell, src_comp;
     double amp_n, sig_src;
 };
 
+// One adjoint step but for the cell-local H part of its own step, which
+// launch_adjoint_local has done (first step of a replayed segment) or the step
+// before (next_local: this one does that of the next, with H0 and H1 its H).
+hipError_t launch_adjoint_local(const AdjArgs &A, hipStream_t st);
 hipError_t launch_adjoint_step(const AdjArgs &A, const double *g, int nrec, const int *rec,
-                               hipStream_t st);
+                               bool next_local, hipStream_t st);
 
 // Kernel launchers (fdtd_kernels.hip).  `pre` is the exclusive prefix of
 // per-shot block counts (device), `nblocks` its total.

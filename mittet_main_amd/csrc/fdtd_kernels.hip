@@ -15,7 +15,7 @@
 //
 // All arithmetic keeps the reference's evaluation order; the library is built
 // with -ffp-contract=off so results equal the reference's bit for bit.
-#include "fdtd_dev.h"
+#include "fdtd_tile.h"
 
 // Minimum resident waves per SIMD requested for the streaming kernels; it caps
 // their VGPR budget (512 / waves) so enough waves are in flight to cover HBM
@@ -31,38 +31,7 @@
 #endif
 
 
-// Pointers read out of the shot descriptor are generic; casting them to the
-// global address space lets the compiler emit global_load/store instead of
-// flat accesses (which also count against the LDS wait counter).
-#define GLOBAL __attribute__((address_space(1)))
-
 namespace mt {
-
-__device__ __forceinline__ const GLOBAL double *gc(const double *p) { return (const GLOBAL double *)p; }
-__device__ __forceinline__ GLOBAL double *gm(double *p) { return (GLOBAL double *)p; }
-__device__ __forceinline__ const GLOBAL int *gc(const int *p) { return (const GLOBAL int *)p; }
-__device__ __forceinline__ const GLOBAL double *gc(const GLOBAL double *p) { return p; }
-__device__ __forceinline__ GLOBAL double *gm(GLOBAL double *p) { return p; }
-
-// Field values each half-step reads or writes once (own E or H, coefficient,
-// the updated field, psi).  With NT they are non-temporal, so they do not
-// evict the stencil neighbours that other tiles still read from L2 and the
-// Infinity Cache; the host sets NT only for launches whose fields do not fit
-// that cache anyway.
-template <bool NT> __device__ __forceinline__ double ld_s(const GLOBAL double *p)
-{
-    if constexpr (NT)
-        return __builtin_nontemporal_load(p);
-    else
-        return *p;
-}
-template <bool NT> __device__ __forceinline__ void st_s(GLOBAL double *p, double v)
-{
-    if constexpr (NT)
-        __builtin_nontemporal_store(v, p);
-    else
-        *p = v;
-}
 
 __device__ __forceinline__ double dminus(const GLOBAL double *__restrict__ F, int c, int s,
                                          double c1, double c2)
@@ -99,37 +68,6 @@ __device__ __forceinline__ int chunk_step(const ShotDev &S)
     return *(const __attribute__((address_space(4))) int *)S.step;
 }
 
-// A wave-uniform double (a z-profile value of the current plane) through the
-// scalar cache.  A vector load issued after a plane's prefetch would make the
-// wait for it also wait for every prefetch load issued before it.
-__device__ __forceinline__ double uload(const double *p)
-{
-    return *(const __attribute__((address_space(4))) double *)p;
-}
-
-// Addresses of the per-cell kernels.  A block's cells lie in one plane, so every
-// access is a wave-uniform base (component and plane, scalar arithmetic) plus a
-// 32-bit byte offset within the plane: one scalar-base load instruction, no
-// 64-bit vector arithmetic per access.  A grid below 2^31 cells has at least 8
-// planes (two CPML shells of 2 cells and 4 more), so a plane is below 2^31
-// bytes.
-typedef const GLOBAL char *gcp;
-typedef GLOBAL char *gmp;
-__device__ __forceinline__ gcp cb(const void *p) { return (gcp)p; }
-__device__ __forceinline__ gmp mb(void *p) { return (gmp)p; }
-__device__ __forceinline__ double at(gcp b, unsigned o, int d = 0)
-{
-    return *(const GLOBAL double *)(b + o + d);
-}
-template <bool NT> __device__ __forceinline__ double at_s(gcp b, unsigned o)
-{
-    return ld_s<NT>((const GLOBAL double *)(b + o));
-}
-template <bool NT> __device__ __forceinline__ void put_s(gmp b, unsigned o, double v)
-{
-    st_s<NT>((GLOBAL double *)(b + o), v);
-}
-
 // ring slot q of a descriptor, q < 2 * ring (or any q when there is one slot)
 __device__ __forceinline__ int ring_slot(const ShotDev &S, int q)
 {
@@ -153,10 +91,6 @@ template <bool H> __device__ __forceinline__ Quad uquad(const double *cq, int r)
 {
     const double *p = cq + (size_t)r * CQ_N + (H ? CQ_H : CQ_E);
     return {uload(p), uload(p + 1), uload(p + 2), uload(p + 3)};
-}
-__device__ __forceinline__ int uload(const int *p)
-{
-    return *(const __attribute__((address_space(4))) int *)p;
 }
 // range flags of a cell
 __device__ __forceinline__ int flags(const ShotDev &S, int i, int jj, int k)
@@ -1269,114 +1203,8 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // ca = 1, cb = dt/eps' (E), da = 1, db = dt/mu0 (H) exactly; an axis whose
 // shell the tile does not touch contributes wave-uniform values.
 
-namespace {
-
-// Tile of a block, the same for its lanes: rows [y0, yend) x columns [x0, x0 + w)
-// of plane k, th = rows of lanes
-struct FTile {
-    int x0, y0, k, w, h, yend;
-    bool region;   // may hold cells of the LDS kernels' region
-};
-
-__device__ __forceinline__ bool ftile(const ShotDev &S, int b, FTile &T)
-{
-    if (!S.shell) {
-        // every tile of every plane, each XCD owning a contiguous run
-        const unsigned q = (b & 7) * (S.fb_pad >> 3) + (b >> 3);
-        if (q >= (unsigned)S.fb)
-            return false;
-        T.k = (int)(((unsigned long long)q * S.tmul) >> S.tsh);
-        const unsigned r = q - (unsigned)T.k * S.tpp;
-        const unsigned ty = (unsigned)(((unsigned long long)r * S.xmul) >> S.xsh);
-        T.w = S.tw;
-        T.h = S.th;
-        T.x0 = (int)(r - ty * S.ttx) * T.w;
-        T.y0 = (int)ty * T.h;
-        T.yend = S.iy;
-        T.region = false;
-        return true;
-    }
-    // the shell tile list in launch order: at 288^3 (16-cell CPML) this runs
-    // each half-step's shell launch 12 us faster than giving each XCD a
-    // contiguous run of the list, while on grids that the per-cell family
-    // covers whole (84^3) the contiguous runs are 1.2x faster
-    if (b >= S.fb)
-        return false;
-    const int *t = (const int *)(S.shell + b);   // {x0, y0, k, yend}
-    T.x0 = uload(t);
-    T.y0 = uload(t + 1);
-    T.k = uload(t + 2);
-    const int yend = uload(t + 3);
-    T.w = yend ? 16 : ZX;
-    T.h = yend ? 16 : ZY;
-    T.yend = yend ? yend : S.iy;
-    T.region = !yend && T.k >= S.lo[2] && T.k < S.hi[2];
-    return T.k >= 0;
-}
-
-// A lane's cell in its tile, its LDS position (pitch w + 3, two cells before
-// the tile for E, one for H) and its halo item.  LO cells before the tile and
-// HI after it on each axis (LO + HI = 3): first the halo rows of component 2,
-// then of component 0, then the halo columns of component 2, then of component 1.
-template <int LO> struct FLane {
-    int i, jj;
-    unsigned o;        // byte offset of the (clamped) cell in its plane
-    unsigned a, p;     // LDS byte address of the cell, pitch in bytes
-    bool own;          // the lane's cell is one of the tile's
-    bool halo;         // the lane has a halo item
-    int hc;            // its component
-    unsigned ho, ha;   // its plane offset and LDS byte address
-    __device__ __forceinline__ FLane(const ShotDev &S, const FTile &T)
-    {
-        const int t = threadIdx.x, w = T.w, h = T.h;
-        const unsigned wm = (65535u + w) / (unsigned)w;   // t / w = t wm >> 16 for t < 256, w <= PT_WH
-        const int ly = (int)((t * wm) >> 16), lx = t - ly * w;
-        p = (unsigned)(w + 3) * 8u;
-        i = T.x0 + lx;
-        jj = T.y0 + ly;
-        own = ly < h;
-        o = (unsigned)min(jj, S.iy - 1) * S.row + (unsigned)min(i, S.ix - 1) * 8u;
-        a = (unsigned)(ly + LO) * p + (unsigned)(lx + LO) * 8u;
-        int u, v;   // halo position relative to the tile
-        if (t < 6 * w) {
-            const bool second = t >= 3 * w;
-            const int m = second ? t - 3 * w : t;
-            const int r = (int)((m * wm) >> 16);
-            u = m - r * w;
-            v = r < LO ? r - LO : h + r - LO;
-            hc = second ? 0 : 2;
-        } else {
-            int m = t - 6 * w;
-            const bool second = m >= 3 * h;
-            m = second ? m - 3 * h : m;
-            v = (m * 21846) >> 16;   // m / 3
-            const int r = m - 3 * v;
-            u = r < LO ? r - LO : w + r - LO;
-            hc = second ? 1 : 2;
-        }
-        halo = t < 6 * (w + h);
-        const int gx = min(max(T.x0 + u, 0), S.ix - 1), gy = min(max(T.y0 + v, 0), S.iy - 1);
-        ho = (unsigned)gy * S.row + (unsigned)gx * 8u;
-        ha = (unsigned)(v + LO) * p + (unsigned)(u + LO) * 8u + (unsigned)hc * (PT_TILE * 8u);
-    }
-};
-
-// r in [a, b) U [c, d): an axis' CPML face (a superset of a cell's face flag, so
-// psi loads need not wait for the flag words)
-__device__ __forceinline__ bool in_face(int r, int a, int b, int c, int d)
-{
-    return (r >= a && r < b) || (r >= c && r < d);
-}
-__device__ __forceinline__ double lds_at(const double *b, unsigned o, int d = 0)
-{
-    return *(const double *)((const char *)b + o + d);
-}
-__device__ __forceinline__ void lds_put(double *b, unsigned o, double v)
-{
-    *(double *)((char *)b + o) = v;
-}
-
-}  // namespace
+// Component of a halo item: components 2 and 0 have halo rows, 2 and 1 columns
+__device__ __forceinline__ int halo_comp(int hk) { return hk == 1 ? 0 : (hk == 3 ? 1 : 2); }
 
 // The first recn blocks (recn: 0, or ns rounded up to a multiple of 8 so that
 // the tile blocks keep their XCD) gather receivers, block s for shot s, with one
@@ -1419,12 +1247,13 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     const size_t zp1 = k + 1 < S.iz ? kp + pb : kp;
     const gcp Hb = cb(hsel(S, j, hf)), Ein = cb(S.e + (size_t)si * S.sstride) + kp;
     const FLane<2> q(S, T);
+    const int hc = halo_comp(q.hk);
 
     // ---- loads
     const double z0 = at(Hb + 2 * nb + kp, q.o), y0 = at(Hb + nb + kp, q.o), x0 = at(Hb + kp, q.o);
     double hv = 0.0;
     if (q.halo)
-        hv = *(const GLOBAL double *)(Hb + kp + (size_t)q.hc * nb + q.ho);
+        hv = *(const GLOBAL double *)(Hb + kp + (size_t)hc * nb + q.ho);
     const double yzm1 = at(Hb + nb + zm1, q.o), yzp1 = at(Hb + nb + zp1, q.o), yzm2 = at(Hb + nb + zm2, q.o);
     const double xzm1 = at(Hb + zm1, q.o), xzp1 = at(Hb + zp1, q.o), xzm2 = at(Hb + zm2, q.o);
     double ex = at_s<NT>(Ein, q.o), ey = at_s<NT>(Ein + nb, q.o), ez = at_s<NT>(Ein + 2 * nb, q.o);
@@ -1483,7 +1312,7 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
         lds_put(sh + 2 * PT_TILE, q.a, z0);
     }
     if (q.halo)
-        lds_put(sh, q.ha, hv);
+        lds_put(sh, q.ha + (unsigned)hc * (PT_TILE * 8u), hv);
     __syncthreads();
     // the step is looked up behind the loads (it costs two dependent scalar
     // loads): a shot that has finished its time loop stores nothing
@@ -1612,12 +1441,13 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     const size_t zp1 = k + 1 < S.iz ? kp + pb : kp, zp2 = k + 2 < S.iz ? kp + 2 * pb : kp;
     const gcp Eb = cb(S.e + (size_t)so * S.sstride), Hin = cb(hsel(S, j, hf)) + kp;
     const FLane<1> q(S, T);
+    const int hc = halo_comp(q.hk);
 
     // ---- loads
     const double z0 = at(Eb + 2 * nb + kp, q.o), y0 = at(Eb + nb + kp, q.o), x0 = at(Eb + kp, q.o);
     double hv = 0.0;
     if (q.halo)
-        hv = *(const GLOBAL double *)(Eb + kp + (size_t)q.hc * nb + q.ho);
+        hv = *(const GLOBAL double *)(Eb + kp + (size_t)hc * nb + q.ho);
     const double yzp1 = at(Eb + nb + zp1, q.o), yzp2 = at(Eb + nb + zp2, q.o), yzm1 = at(Eb + nb + zm1, q.o);
     const double xzp1 = at(Eb + zp1, q.o), xzp2 = at(Eb + zp2, q.o), xzm1 = at(Eb + zm1, q.o);
     double hx = at_s<NT>(Hin, q.o), hy = at_s<NT>(Hin + nb, q.o), hz = at_s<NT>(Hin + 2 * nb, q.o);
@@ -1677,7 +1507,7 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
         lds_put(sh + 2 * PT_TILE, q.a, z0);
     }
     if (q.halo)
-        lds_put(sh, q.ha, hv);
+        lds_put(sh, q.ha + (unsigned)hc * (PT_TILE * 8u), hv);
     __syncthreads();
     // the step is looked up behind the loads (it costs two dependent scalar
     // loads): a shot that has finished its time loop stores nothing

@@ -84,6 +84,31 @@ def test_lds_adjoint_matches_the_per_cell_adjoint(monkeypatch):
     assert np.abs(g1 - g0).max() <= 1e-12 * np.abs(g0).max()
 
 
+@pytest.mark.parametrize("ix, iy, iz, nc", [
+    (81, 31, 33, 7),   # region from ncpml + 1 on x: the passes' P_x of the last CPML cells are in reach
+    (33, 27, 19, 2),   # thin CPML, region tiles partial on both axes, short last z-chunk
+    (18, 18, 18, 7),   # region of 2 x 2 cells by 2 planes: every cell is a rim cell on all faces
+    (26, 47, 21, 6),   # 12 region columns, 33 rows
+])
+def test_lds_adjoint_at_region_edges(ix, iy, iz, nc, monkeypatch):
+    """Weights handed over between the region's kernels and the per-cell passes
+    at ragged region sizes: the gradient is that of the per-cell passes alone up
+    to rounding (1e-12 of the largest component: 80 steps of some 50 operations
+    at 1.1e-16 each)."""
+    def run():
+        P, sig0, _ = problem(seed=5, ix=ix, iy=iy, iz=iz, nc=nc, it=80)
+        _, g = P.value_and_grad(np.log(sig0))
+        P.close()
+        return g
+
+    print(f"LDS adjoint at region edges: {ix} x {iy} x {iz}, ncpml {nc}", flush=True)
+    g1 = run()
+    monkeypatch.setenv("MITTET_FDTD_NOLDS", "1")
+    g0 = run()
+    assert np.all(np.isfinite(g1)) and np.abs(g0).max() > 0
+    assert np.abs(g1 - g0).max() <= 1e-12 * np.abs(g0).max()
+
+
 def test_segment_length_does_not_change_gradient():
     P1, sig0, _ = problem(seed=3, segment=7)
     P2, _, _ = problem(seed=3, segment=64)
