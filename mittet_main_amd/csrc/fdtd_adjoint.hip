@@ -96,7 +96,7 @@ __global__ __launch_bounds__(PT) void k_adj_cell(AdjArgs A, int gather, int loca
 {
     __shared__ double sh[4 * PT_TILE];   // P_x, Q_x (x stencils), P_y, Q_y (y stencils)
     FTile T;
-    if (!ftile(A, blockIdx.x, T))
+    if (!ftile<false>(A, blockIdx.x, T))
         return;   // uniform over the block
     const int k = T.k, nc = A.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > A.ix - nc, ay = T.y0 < nc || T.y0 + T.h > A.iy - nc;

@@ -300,32 +300,48 @@ void cell_tile(int ix, int iy, int &w, int &h)
 // planes outside the region and rows of 32 x 8 tiles not inside it in y get
 // every tile; rows inside it in y get 16 x 16 tiles over the two x-edge
 // segments [0, lo_x) and [hi_x, ix) only.  Cells of the region that a tile
-// still holds are skipped by the kernels.  Padded to a multiple of 8 entries
-// with k = -1.
+// still holds are skipped by the kernels.
+//
+// Order: a plane's tiles fill a multiple of 8 entries (k = -1 beyond them), entry e
+// of these being tile (e mod 8) P / 8 + e / 8 of the P there: blocks go to the XCDs
+// in turn, so each XCD gets consecutive tiles of a plane, and of the next planes
+// the tiles above them, whose stencils share values in its L2.  Each 8 planes the
+// parts move on by one XCD (see ftile).  Shell launches (E + H) with the tiles of a
+// plane dealt to the XCDs one by one, and so: 152^3 46.1 + 47.9 -> 38.2 + 38.6 us,
+// 216^3 95.9 + 96.9 -> 90.0 + 91.2, 288^3 161 + 168 -> 158 + 164; without the
+// change of XCD 39.8 + 40.4, 98.6 + 99.8, 163 + 171; changing every 2, 4, 16 planes
+// 40.2 + 42.5, 38.1 + 38.8, 38.2 + 38.5 at 152^3.
 std::vector<int4> complement_tiles(int ix, int iy, int iz, const int lo[3], const int hi[3])
 {
     std::vector<int4> shell;
     const int ftx = tiles(ix, mt::ZX), fty = tiles(iy, mt::ZY);
     const int ya = tiles(lo[1], mt::ZY), yb = hi[1] / mt::ZY;   // tile rows inside [lo_y, hi_y)
+    std::vector<int4> plane;
+    auto deal = [&](int k) {
+        const int P = (int)plane.size(), e = tiles(P, 8);
+        for (int b = 0; b < 8 * e; ++b) {
+            const int t = ((b + k / 8) & 7) * e + b / 8;
+            shell.push_back(t < P ? plane[t] : int4{0, 0, -1, 0});
+        }
+        plane.clear();
+    };
     for (int k = 0; k < iz; ++k) {
         const bool inz = k >= lo[2] && k < hi[2];
         for (int ty = 0; ty < fty; ++ty) {
             if (inz && ty >= ya && ty < yb)
                 continue;
             for (int tx = 0; tx < ftx; ++tx)
-                shell.push_back(int4{tx * mt::ZX, ty * mt::ZY, k, 0});
+                plane.push_back(int4{tx * mt::ZX, ty * mt::ZY, k, 0});
         }
-        if (!inz || ya >= yb)
-            continue;
         const int yend = yb * mt::ZY;
-        for (int y0 = ya * mt::ZY; y0 < yend; y0 += 16) {
+        for (int y0 = ya * mt::ZY; inz && y0 < yend; y0 += 16) {
             for (int x0 = 0; x0 < lo[0]; x0 += 16)
-                shell.push_back(int4{x0, y0, k, yend});
+                plane.push_back(int4{x0, y0, k, yend});
             for (int x0 = hi[0]; x0 < ix; x0 += 16)
-                shell.push_back(int4{x0, y0, k, yend});
+                plane.push_back(int4{x0, y0, k, yend});
         }
+        deal(k);
     }
-    shell.resize((size_t)tiles((int)shell.size(), 8) * 8, int4{0, 0, -1, 0});
     return shell;
 }
 
@@ -439,6 +455,7 @@ struct fwi3d_shot {
     int kind = 0;          // fused kernel family (see launch_eh)
     int nblocks = 0;       // fused blocks (padded to a multiple of 8)
     int nblocks_l = 0;     // LDS-kernel blocks of family 3 (padded to a multiple of 8)
+    int nlayer = 0, nlayer_l = 0;   // ... and in layers (non-temporal launches, see ftile)
     int4 *d_shell = nullptr;  // family 3: tiles of the per-cell kernels
     int nblocks_op = 0;    // per-cell blocks of the stand-alone operators
     int ncellblocks = 0;
@@ -456,6 +473,7 @@ struct fwi3d_batch {
     ShotDev *d_desc = nullptr;
     int *d_pre = nullptr, *d_pre_l = nullptr, *d_pre_cells = nullptr;
     int nblocks = 0, nblocks_l = 0, ncellblocks = 0;
+    bool rings = false, fused = false, nt = false;   // the members' Fam
     int kind = 0;         // fused kernel family of the members (all equal)
     bool dirty = true;
     hipGraphExec_t graph = nullptr;
@@ -978,6 +996,7 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.tpp = d.ttx * tiles(p.iy, d.th);
     magic_div((unsigned)d.ttx, d.xmul, d.xsh);
     magic_div((unsigned)d.tpp, d.tmul, d.tsh);
+    magic_div((unsigned)tiles(d.tpp, 8), d.emul, d.esh);
     d.opp = tiles(p.ix * p.iy, mt::PT);
     magic_div((unsigned)d.opp, d.omul, d.osh);
     magic_div((unsigned)p.ix, d.imul, d.ish);
@@ -1109,6 +1128,8 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
         }
     }
     s->nblocks = s->kind == 2 ? d.zb_pad : d.fb_pad;
+    s->nlayer = s->kind == 0 ? tiles(d.tpp, 8) * 8 * p.iz : s->nblocks;
+    s->nlayer_l = tiles(d.ltx * d.lty, 8) * 8 * d.lkz;
     s->ncellblocks = tiles((int)N, mt::FLUSH_CELLS);
     if ((rc = upload_desc(s)) || (rc = fwi3d_set_zero_eh(s))) {
         fwi3d_shot_destroy(s);
@@ -1276,10 +1297,19 @@ bool stream_nt(long long touch_bytes)
     return touch_bytes > kNtMinBytes;
 }
 
+// Blocks of the per-cell and the LDS kernels' launches: non-temporal launches take
+// their tiles in layers (ftile), the fused E+H launch does not.
+static int cell_blocks(const fwi3d_shot *s, bool nt) { return nt ? s->nlayer : s->nblocks; }
+static int lds_blocks(const fwi3d_shot *s, bool nt, bool fused)
+{
+    return nt && !fused ? s->nlayer_l : s->nblocks_l;
+}
+
 static Fam shot_fam(const fwi3d_shot *s)
 {
-    return {s->kind, s->d_pre, s->nblocks, s->d_pre, s->nblocks_l, s->ring > 1,
-            s->kind == 3 && s->fused, stream_nt(step_touch_bytes(s))};
+    const bool nt = stream_nt(step_touch_bytes(s)), fused = s->kind == 3 && s->fused;
+    return {s->kind, s->d_pre, cell_blocks(s, nt), s->d_pre, lds_blocks(s, nt, fused), s->ring > 1,
+            fused, nt};
 }
 
 // After `steps` steps of a fused schedule the current H is in the other buffer
@@ -2119,6 +2149,8 @@ static int replay_segment(fwi3d_grad *g, int L)
         // (and psi) both ways plus the coefficients, 112 B per cell (88 where H
         // is updated in place and copied)
         f.nt = stream_nt((long long)s->desc.n * (hring ? 112 : 88));
+        f.nblocks = cell_blocks(s, f.nt);
+        f.nblocks_l = lds_blocks(s, f.nt, f.fused);
         const bool fold = s->nrec && rec_folds(f);
         const mt::StateSegs segs = state_segs_from(g, 1);   // H and psi, without the rings
         hipGraph_t graph = nullptr;
@@ -2966,10 +2998,20 @@ static int batch_upload(fwi3d_batch *b)
     const int ns = (int)b->shots.size();
     std::vector<ShotDev> descs(ns);
     std::vector<int> pre(ns + 1, 0), prel(ns + 1, 0), prec(ns + 1, 0);
+    b->rings = true;
+    b->fused = b->kind == 3;
+    long long touch = 0;
+    for (const auto *s : b->shots) {
+        b->rings = b->rings && s->ring > 1;
+        b->fused = b->fused && s->kind == 3 && s->fused;
+        touch += step_touch_bytes(s);
+    }
+    b->nt = stream_nt(touch);
     for (int q = 0; q < ns; ++q) {
-        descs[q] = b->shots[q]->desc;
-        pre[q + 1] = pre[q] + b->shots[q]->nblocks;
-        prel[q + 1] = prel[q] + b->shots[q]->nblocks_l;
+        const fwi3d_shot *s = b->shots[q];
+        descs[q] = s->desc;
+        pre[q + 1] = pre[q] + cell_blocks(s, b->nt);
+        prel[q + 1] = prel[q] + lds_blocks(s, b->nt, b->fused);
         prec[q + 1] = prec[q] + b->shots[q]->ncellblocks;
     }
     b->nblocks = pre[ns];
@@ -2996,14 +3038,7 @@ static int batch_upload(fwi3d_batch *b)
 
 static Fam batch_fam(const fwi3d_batch *b)
 {
-    bool rings = true, fused = b->kind == 3;
-    long long touch = 0;
-    for (const auto *s : b->shots) {
-        rings = rings && s->ring > 1;
-        fused = fused && s->kind == 3 && s->fused;
-        touch += step_touch_bytes(s);
-    }
-    return {b->kind, b->d_pre, b->nblocks, b->d_pre_l, b->nblocks_l, rings, fused, stream_nt(touch)};
+    return {b->kind, b->d_pre, b->nblocks, b->d_pre_l, b->nblocks_l, b->rings, b->fused, b->nt};
 }
 
 int fwi3d_batch_step(fwi3d_batch *b, int nsteps)

@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
     FTile T;
-    if (!ftile(S, ns > 1 ? b - pre[s] : b, T))
+    if (!ftile<NT>(S, ns > 1 ? b - pre[s] : b, T))
         return;   // uniform over the block
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
@@ -1430,7 +1430,7 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
     FTile T;
-    if (!ftile(S, ns > 1 ? b - pre[s] : b, T))
+    if (!ftile<NT>(S, ns > 1 ? b - pre[s] : b, T))
         return;   // uniform over the block
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
@@ -1683,13 +1683,28 @@ __device__ __forceinline__ void tile_store(double *lds, const double (&r)[T::R])
 }
 
 // block -> (shot region tile, z-chunk); false for padding blocks
+// (LAYERS as in ftile: an XCD's eighth of one z-chunk's tiles after another, else a
+// contiguous run of blocks.  E and H launch at 288^3: 256 + 240 us in layers, 268 +
+// 247 with runs; 216^3 112 + 106 and 114 + 108; 152^3, whose fields stay in the
+// Infinity Cache, 34.2 + 30.4 and 33.6 + 29.0)
+template <bool LAYERS>
 __device__ __forceinline__ bool lcol(const ShotDev &S, int b, int &x0, int &y0, int &k0, int &k1)
 {
-    const int L = (b & 7) * (S.lb_pad >> 3) + (b >> 3);
-    if (L >= S.lb)
-        return false;
-    const int tx = L % S.ltx, r = L / S.ltx;
-    const int ty = r % S.lty, kz = r / S.lty;
+    int kz, r;
+    if constexpr (LAYERS) {
+        const int lt = S.ltx * S.lty, e = (lt + 7) >> 3, m = b >> 3;
+        kz = m / e;
+        r = (b & 7) * e + (m - kz * e);
+        if (kz >= S.lkz || r >= lt)
+            return false;
+    } else {
+        const int L = (b & 7) * (S.lb_pad >> 3) + (b >> 3);
+        if (L >= S.lb)
+            return false;
+        kz = L / (S.ltx * S.lty);
+        r = L - kz * (S.ltx * S.lty);
+    }
+    const int ty = r / S.ltx, tx = r - ty * S.ltx;
     x0 = S.lo[0] + tx * LX;
     y0 = S.lo[1] + ty * LY;
     k0 = S.lo[2] + kz * S.lkb;
@@ -1714,7 +1729,7 @@ __global__ __launch_bounds__(LNT) void k_efield_l(const ShotDev *__restrict__ D,
     if (n >= S.it - 1)
         return;
     int x0, y0, k0, k1;
-    if (!lcol(S, blockIdx.x - pre[s], x0, y0, k0, k1))
+    if (!lcol<NT>(S, blockIdx.x - pre[s], x0, y0, k0, k1))
         return;
     const int lx = threadIdx.x % LX, ly = threadIdx.x / LX;
     const int i = x0 + lx, jj = y0 + ly;
@@ -1834,7 +1849,7 @@ __global__ __launch_bounds__(LNT) void k_hfield_l(const ShotDev *__restrict__ D,
     if (chunk_step(S) + j >= S.it - 1)
         return;
     int x0, y0, k0, k1;
-    if (!lcol(S, blockIdx.x - pre[s], x0, y0, k0, k1))
+    if (!lcol<NT>(S, blockIdx.x - pre[s], x0, y0, k0, k1))
         return;
     const int lx = threadIdx.x % LX, ly = threadIdx.x / LX;
     const int i = x0 + lx, jj = y0 + ly;
@@ -2013,7 +2028,7 @@ __global__ __launch_bounds__(LNT, 4) void k_ehfield_l(const ShotDev *__restrict_
     if (n >= S.it - 1)
         return;
     int x0, y0, k0, k1;
-    if (!lcol(S, blockIdx.x - pre[s], x0, y0, k0, k1))
+    if (!lcol<false>(S, blockIdx.x - pre[s], x0, y0, k0, k1))
         return;
     const int ix = S.ix, iy = S.iy, iz = S.iz;
     const size_t N = (size_t)S.n, pl = (size_t)ix * iy;

@@ -83,15 +83,34 @@ struct FTile {
     bool region;   // may hold cells of the LDS kernels' region
 };
 
-template <class G> __device__ __forceinline__ bool ftile(const G &S, int b, FTile &T)
+// Order of the tiles.  Blocks go to the XCDs in turn (block b to XCD b mod 8).
+// Without a list, each XCD owns a contiguous run of planes: what a launch wrote is
+// then in the L2 that the next one reads it from (84^3: 16.7 us a launch, in layers
+// 17.4).  LAYERS (the launches with non-temporal fields, which pass through the
+// caches anyway): all XCDs work on the same planes, each on its eighth of the
+// plane's tiles, so that what their stencils share is read about when it is in the
+// Infinity Cache, and each XCD gets the same part of the costly CPML planes (four
+// shots of 84^3 to 120^3: 127 us a launch with runs, 117 in layers).  Eighths of a
+// plane move on by one XCD every 8 planes: an XCD that kept the y faces' tiles
+// through all planes would finish last (132 us).  The shell list has this order too
+// (complement_tiles).
+template <bool LAYERS, class G> __device__ __forceinline__ bool ftile(const G &S, int b, FTile &T)
 {
     if (!S.shell) {
-        // every tile of every plane, each XCD owning a contiguous run
-        const unsigned q = (b & 7) * (S.fb_pad >> 3) + (b >> 3);
-        if (q >= (unsigned)S.fb)
-            return false;
-        T.k = (int)(((unsigned long long)q * S.tmul) >> S.tsh);
-        const unsigned r = q - (unsigned)T.k * S.tpp;
+        unsigned r;
+        if constexpr (LAYERS) {
+            const unsigned m = (unsigned)b >> 3, e = ((unsigned)S.tpp + 7u) >> 3;
+            T.k = (int)(((unsigned long long)m * S.emul) >> S.esh);   // m / e
+            r = ((b + (T.k >> 3)) & 7) * e + (m - (unsigned)T.k * e);
+            if (T.k >= S.iz || r >= (unsigned)S.tpp)
+                return false;
+        } else {
+            const unsigned q = (b & 7) * (S.fb_pad >> 3) + (b >> 3);
+            if (q >= (unsigned)S.fb)
+                return false;
+            T.k = (int)(((unsigned long long)q * S.tmul) >> S.tsh);
+            r = q - (unsigned)T.k * S.tpp;
+        }
         const unsigned ty = (unsigned)(((unsigned long long)r * S.xmul) >> S.xsh);
         T.w = S.tw;
         T.h = S.th;
@@ -101,10 +120,6 @@ template <class G> __device__ __forceinline__ bool ftile(const G &S, int b, FTil
         T.region = false;
         return true;
     }
-    // the shell tile list in launch order: at 288^3 (16-cell CPML) this runs
-    // each half-step's shell launch 12 us faster than giving each XCD a
-    // contiguous run of the list, while on grids that the per-cell family
-    // covers whole (84^3) the contiguous runs are 1.2x faster
     if (b >= S.fb)
         return false;
     const int *t = (const int *)(S.shell + b);   // {x0, y0, k, yend}

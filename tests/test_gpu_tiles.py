@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from mittet_main_amd import Grid, Model, firstderiv_gauss
+from mittet_main_amd import Batch, Grid, Model, firstderiv_gauss
 from mittet_main_amd.adjoint import GradientProblem, ShotSpec
 from mittet_main_amd.configs import dt_for
 
@@ -61,6 +61,56 @@ def test_tiles_bitwise(dims, ring):
     for q, nm in enumerate(oracle.FIELD_NAMES):
         np.testing.assert_array_equal(shot.field(q), S.arr(nm), err_msg=nm)
     m.close()
+
+
+@pytest.mark.parametrize("family", ["cells", "lds", "batch"])
+@pytest.mark.parametrize("dims", [(8, 8, 8, 2), (17, 13, 9, 2), (43, 25, 19, 4), (131, 11, 17, 3),
+                                  (70, 37, 22, 3)])
+def test_tiles_in_layers_bitwise(dims, family, monkeypatch):
+    """Launches that take their tiles in layers of a plane or a z-chunk (those
+    with non-temporal fields; MITTET_FDTD_NT=1): planes of fewer tiles than
+    XCDs and of a number that 8 does not divide, more and fewer than 8 planes
+    per turn, a shell list, and two shots in one launch, against the oracle
+    bit for bit."""
+    ix, iy, iz, nc = dims
+    monkeypatch.setenv("MITTET_FDTD_NT", "1")
+    monkeypatch.setenv("MITTET_FDTD_LDS" if family == "lds" else "MITTET_FDTD_NOLDS", "1")
+    print(f"layers {dims} {family}", flush=True)
+    rng = np.random.default_rng(ix)
+    dl = (50.0, 45.0, 40.0)
+    dt, cmax = dt_for(*dl, sig_min=0.05)
+    it = 12
+    signal = firstderiv_gauss(it, dt, 0.5 / dt / it)
+    src = (ix // 2, iy // 2, iz // 2)
+    rec = np.array([[1, 1, 1], [ix - 2, iy - 2, iz - 2]], np.int32)
+    runs = []
+    for _ in range(2 if family == "batch" else 1):
+        sig = np.exp(rng.uniform(np.log(0.05), np.log(3.0), (iz, iy, ix)))
+        m = Model(Grid(ix, iy, iz, nc, *dl, dt, OM0, cmax))
+        m.media_coeff_3d(sig)
+        S = oracle.OracleSim(ix, iy, iz, nc, *dl, dt, OM0, cmax)
+        S.set_sigma(sig)
+        S.init_cpml()
+        S.media_coeff_3d()
+        runs.append((m, m.shot(it, signal, src, 2, rec), S))
+    if family == "batch":
+        b = Batch(2)
+        for _, shot, _ in runs:
+            b.add(shot)
+        b.step(it - 1)
+        b.sync()
+        for _, shot, _ in runs:
+            b.remove(shot)
+        b.close()
+    else:
+        runs[0][1].run()
+    for m, shot, S in runs:
+        tr, _ = S.forward(2, signal, tuple(c + 1 for c in src), it - 1, rec1=rec + 1, it=it)
+        np.testing.assert_array_equal(shot.traces()[:3], tr)
+        for q, nm in enumerate(oracle.FIELD_NAMES):
+            np.testing.assert_array_equal(shot.field(q), S.arr(nm), err_msg=nm)
+        shot.close()
+        m.close()
 
 
 def test_replayed_states_are_complete():
