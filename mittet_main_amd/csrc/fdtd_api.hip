@@ -565,6 +565,9 @@ struct fwi3d_shot {
     double *d_h2 = nullptr;   // second H buffer of the fused E+H step (null: not fused)
     bool fused = false;       // steps run the fused E+H interior kernel
     double *d_amp = nullptr, *d_traces = nullptr, *d_w = nullptr, *d_acc = nullptr;
+    double *d_spec = nullptr;    // kept memory of spectrum requests (SpecMem) ...
+    size_t spec_size = 0;        // ... its doubles, and the request that has it
+    std::mutex spec_mu;
     double *d_acc_h = nullptr;   // H volume spectra (fwi3d_enable_volume_dft_h)
     double *d_hring = nullptr;   // H after each step of a chunk, for the H sums
     int *d_rec = nullptr, *d_step = nullptr, *d_pre = nullptr, *d_flag = nullptr;
@@ -1306,6 +1309,7 @@ int fwi3d_shot_destroy(fwi3d_shot *s)
     dfree(s->d_flag);
     dfree(s->d_pre);
     dfree(s->d_shell);
+    dfree(s->d_spec);
     dfree(s->d_desc);
     if (s->m)
         s->m->nshots--;
@@ -1754,25 +1758,55 @@ static int noalloc_scratch(double **out)
     return FWI3D_OK;
 }
 
-static int device_rows_dft(hipStream_t st, const double *d_rows, int nrows, int it, double dt,
-                           double omega0, int nfreq, const double *omegas, double *out_host)
-{
-    double *d_om = nullptr, *d_out = nullptr;
-    if (dalloc(&d_om, (size_t)nfreq) != hipSuccess ||
-        dalloc(&d_out, 2 * (size_t)nrows * nfreq) != hipSuccess) {
-        dfree(d_om);
-        return fail(FWI3D_ENOMEM, "spectrum buffers");
+// Device memory of one spectrum request: the shot's kept buffer where it is large
+// enough to hold the request or may grow to (kSpecKeep), and no other request has
+// it; else memory of its own.
+constexpr size_t kSpecKeep = 1u << 19;   // doubles (4 MiB)
+
+struct SpecMem {
+    std::unique_lock<std::mutex> own;
+    double *p = nullptr;
+    bool kept = false;
+    SpecMem(fwi3d_shot *s, size_t n)
+    {
+        if (s && n <= kSpecKeep) {
+            own = std::unique_lock<std::mutex>(s->spec_mu, std::try_to_lock);
+            if (own.owns_lock()) {
+                if (n > s->spec_size) {
+                    dfree(s->d_spec);
+                    s->spec_size = dalloc(&s->d_spec, n) == hipSuccess ? n : 0;
+                }
+                p = s->d_spec;
+                kept = true;
+                return;
+            }
+        }
+        if (dalloc(&p, n) != hipSuccess)
+            p = nullptr;
     }
-    hipError_t e = hipMemcpyAsync(d_om, omegas, sizeof(double) * nfreq, hipMemcpyHostToDevice, st);
+    ~SpecMem()
+    {
+        if (!kept)
+            dfree(p);
+    }
+};
+
+static int device_rows_dft(hipStream_t st, fwi3d_shot *s, const double *d_rows, int nrows, int it,
+                           double dt, double omega0, int nfreq, const double *omegas, double *out_host)
+{
+    const size_t off = ((size_t)nfreq + 31) / 32 * 32;
+    SpecMem d(s, off + 2 * (size_t)nrows * nfreq);
+    if (!d.p)
+        return fail(FWI3D_ENOMEM, "spectrum buffers");
+    hipError_t e = hipMemcpyAsync(d.p, omegas, sizeof(double) * nfreq, hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
-        e = mt::launch_receiver_dft(d_rows, nrows, it, dt, omega0, nfreq, d_om, d_out, st);
+        e = mt::launch_receiver_dft(d_rows, nrows, it, dt, omega0, nfreq, d.p, d.p + off, st);
     if (e == hipSuccess)
-        e = hipMemcpyAsync(out_host, d_out, sizeof(double) * 2 * nrows * nfreq,
+        e = hipMemcpyAsync(out_host, d.p + off, sizeof(double) * 2 * nrows * nfreq,
                            hipMemcpyDeviceToHost, st);
+    const hipError_t es = hipStreamSynchronize(st);   // no work on the memory beyond this call
     if (e == hipSuccess)
-        e = hipStreamSynchronize(st);
-    dfree(d_om);
-    dfree(d_out);
+        e = es;
     if (e != hipSuccess)
         return fail(FWI3D_EDEVICE, "receiver DFT: %s", hipGetErrorString(e));
     return FWI3D_OK;
@@ -1786,6 +1820,17 @@ static std::complex<double> h_factor(double omega0, double om)
     if (om == 0.0)
         return {std::nan(""), std::nan("")};
     return std::sqrt(std::complex<double>(-2.0 * omega0, 0.0) / std::complex<double>(0.0, 1.0) / om);
+}
+
+// the transform of a source waveform to its spectrum (host)
+static void source_factor(double omega0, int nfreq, const double *omegas, double *out)
+{
+    for (int f = 0; f < nfreq; ++f) {
+        std::complex<double> v(out[2 * f], out[2 * f + 1]);
+        v = omegas[f] == 0.0 ? std::complex<double>(2.0 * omega0, 0.0) : v * h_factor(omega0, omegas[f]);
+        out[2 * f] = v.real();
+        out[2 * f + 1] = v.imag();
+    }
 }
 
 // the f_to_d_h factor on the magnetic rows of receiver spectra (host)
@@ -1809,7 +1854,7 @@ int fwi3d_receiver_dft(fwi3d_shot *s, int nfreq, const double *omegas, int hfac,
         return fail(FWI3D_EINVAL, "bad receiver DFT request");
     if (s->nrec == 0)
         return FWI3D_OK;
-    int rc = device_rows_dft(s->st, s->d_traces, 6 * s->nrec, s->it, s->m->p.dt, s->m->p.omega0,
+    int rc = device_rows_dft(s->st, s, s->d_traces, 6 * s->nrec, s->it, s->m->p.dt, s->m->p.omega0,
                              nfreq, omegas, out);
     if (rc || !hfac)
         return rc;
@@ -1878,17 +1923,12 @@ int fwi3d_source_spectrum(double dt, double omega0, int it, const double *signal
     else if (hcopy(d_sig, signal, sizeof(double) * it) != hipSuccess)
         rc = fail(FWI3D_EDEVICE, "signal upload");
     if (!rc)
-        rc = device_rows_dft(st, d_sig, 1, it, dt, omega0, nfreq, omegas, out);
+        rc = device_rows_dft(st, nullptr, d_sig, 1, it, dt, omega0, nfreq, omegas, out);
     dfree(d_sig);
     del_stream(st);
     if (rc)
         return rc;
-    for (int f = 0; f < nfreq; ++f) {
-        std::complex<double> v(out[2 * f], out[2 * f + 1]);
-        v = omegas[f] == 0.0 ? std::complex<double>(2.0 * omega0, 0.0) : v * h_factor(omega0, omegas[f]);
-        out[2 * f] = v.real();
-        out[2 * f + 1] = v.imag();
-    }
+    source_factor(omega0, nfreq, omegas, out);
     return FWI3D_OK;
 }
 
@@ -1996,7 +2036,7 @@ int fwi3d_laplace_fft(fwi3d_shot *s, double *e_t, double *j_t, double *g_t)
     // spectra at every bin: rows of E, then G = E/J, then J
     std::vector<double> spec(2 * (size_t)(2 * rows + 1) * it);
     double *ew = spec.data(), *gw = ew + 2 * (size_t)rows * it, *jw = gw + 2 * (size_t)rows * it;
-    int rc = device_rows_dft(s->st, s->d_traces, rows, it, dt, omega0, it, omg.data(), ew);
+    int rc = device_rows_dft(s->st, s, s->d_traces, rows, it, dt, omega0, it, omg.data(), ew);
     if (!rc)
         rc = fwi3d_source_spectrum(dt, omega0, it, s->signal.data(), it, omg.data(), jw);
     if (rc)
@@ -2051,18 +2091,44 @@ int fwi3d_laplace_to_freq(fwi3d_shot *s, int nbins, const double *strue, double 
     const int it = s->it;
     const double dt = s->m->p.dt, omega0 = s->m->p.omega0;
     const double om = 2.0 * M_PI / it / dt;
-    std::vector<double> omg(nbins);
+    // one upload (bins, the shot's waveform, the true one) and one download (spectra of
+    // both waveforms and of the traces)
+    std::vector<double> up((size_t)nbins + 2 * (size_t)it);
     for (int n = 0; n < nbins; ++n)
-        omg[n] = om * n;
-    int rc = FWI3D_OK;
-    if (s->nrec)
-        rc = device_rows_dft(s->st, s->d_traces, 3 * s->nrec, it, dt, omega0, nbins, omg.data(), e_w);
-    if (!rc)
-        rc = fwi3d_source_spectrum(dt, omega0, it, s->signal.data(), nbins, omg.data(), j_w);
-    if (rc)
-        return rc;
-    const std::vector<std::complex<double>> tru = true_spectrum(strue, it, 0, nbins);
-    for (int row = 0; row < 3 * s->nrec; ++row)
+        up[n] = om * n;
+    std::memcpy(&up[nbins], s->signal.data(), sizeof(double) * it);
+    std::memcpy(&up[nbins + (size_t)it], strue, sizeof(double) * it);
+    const int rows = 3 * s->nrec;
+    const size_t nb2 = 2 * (size_t)nbins, off = (up.size() + 31) / 32 * 32;
+    std::vector<double> down((2 + (size_t)rows) * nb2);
+    {
+        SpecMem d(s, off + down.size());
+        if (!d.p)
+            return fail(FWI3D_ENOMEM, "spectrum buffers");
+        hipError_t e = hipMemcpyAsync(d.p, up.data(), sizeof(double) * up.size(), hipMemcpyHostToDevice, s->st);
+        if (e == hipSuccess)
+            e = mt::launch_receiver_dft(d.p + nbins, 1, it, dt, omega0, nbins, d.p, d.p + off, s->st);
+        if (e == hipSuccess)
+            e = mt::launch_bin_dft(d.p + nbins + it, it, 0, nbins, d.p + off + nb2, s->st);
+        if (e == hipSuccess)
+            e = mt::launch_receiver_dft(s->d_traces, rows, it, dt, omega0, nbins, d.p, d.p + off + 2 * nb2,
+                                        s->st);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(down.data(), d.p + off, sizeof(double) * down.size(), hipMemcpyDeviceToHost,
+                               s->st);
+        const hipError_t es = hipStreamSynchronize(s->st);   // also where a launch failed
+        if (e == hipSuccess)
+            e = es;
+        if (e != hipSuccess)
+            return fail(FWI3D_EDEVICE, "laplace_to_freq: %s", hipGetErrorString(e));
+    }
+    std::memcpy(j_w, down.data(), sizeof(double) * nb2);
+    source_factor(omega0, nbins, up.data(), j_w);
+    std::memcpy(e_w, down.data() + 2 * nb2, sizeof(double) * rows * nb2);
+    std::vector<std::complex<double>> tru(nbins);
+    for (int n = 0; n < nbins; ++n)
+        tru[n] = {down[nb2 + 2 * n], down[nb2 + 2 * n + 1]};
+    for (int row = 0; row < rows; ++row)
         for (int n = 0; n < nbins; ++n) {
             const size_t q = (size_t)row * nbins + n;
             const std::complex<double> e(e_w[2 * q], e_w[2 * q + 1]), jv(j_w[2 * n], j_w[2 * n + 1]);
@@ -2135,8 +2201,7 @@ struct fwi3d_grad {
     std::vector<double *> inner;      // depth l >= 1: slots for the starts of a segment's pieces
     double *buf = nullptr;            // leaf + 1 states
     double *adj = nullptr;            // adjoint state (one state)
-    double *tmp = nullptr;            // region state as weights (2 x 3N), weights of the per-cell
-                                      // passes (2 x 6N)
+    double *tmp = nullptr;            // weights of the per-cell passes (2 x 6N)
     double *grad = nullptr;           // N
     double *grad_src = nullptr;       // 1
     double *g = nullptr;              // [it][3][nrec] trace sensitivities

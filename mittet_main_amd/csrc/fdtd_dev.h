@@ -245,6 +245,8 @@ hipError_t launch_hstore(const ShotDev *d, int ns, const int *pre_cells, int nbl
 hipError_t launch_receiver_dft(const double *traces, int ncomp_rows, int it, double dt,
                                double omega0, int nfreq, const double *omegas,
                                double *out, hipStream_t st);
+// bins k0 .. k0 + nbins - 1 of sum_n x[n] exp(2 pi i n k / it), complex
+hipError_t launch_bin_dft(const double *x, int it, int k0, int nbins, double *out, hipStream_t st);
 hipError_t launch_bin_dft(const double *traces, int nrows, int it, double dt, double omega0,
                           int nbins, double *out, hipStream_t st);
 hipError_t launch_fill(double *p, size_t count, double v, hipStream_t st);
