@@ -697,10 +697,8 @@ int launch_eh(const Fam &f, const ShotDev *d, int ns, int j, bool h, hipStream_t
     hipError_t e;
     const bool e_here = rec_here && (!f.rings || f.kind == 4);
     if (f.kind == 4) {
-        if (!h)
-            HIP_TRY(mt::launch_source_hz(d, ns, j, st, rec_prev));
         e = h ? mt::launch_hfield_v(d, ns, f.pre, f.nblocks, j, st, e_here)
-              : mt::launch_efield_v(d, ns, f.pre, f.nblocks, j, st);
+              : mt::launch_efield_v(d, ns, f.pre, f.nblocks, j, st, rec_prev);
         HIP_TRY(e);
         return FWI3D_OK;
     }
@@ -1191,11 +1189,9 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     s->nblocks_op = d.op_pad;
     s->kind = sp->zchunk > 0 ? 2 : d.pair;
     if (magnetic) {
-        // every 32 x 8 tile, one cell per lane (fdtd_fortran.hip)
+        // the per-cell tiles (fdtd_fortran.hip)
         d.pair = 0;
-        d.ftx = tiles(p.ix, mt::ZX);
-        d.fty = tiles(p.iy, mt::ZY);
-        d.fb = d.ftx * d.fty * p.iz;
+        d.fb = d.tpp * p.iz;
         d.fb_pad = tiles(d.fb, 8) * 8;
         s->kind = 4;
     }

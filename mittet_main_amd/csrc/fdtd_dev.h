@@ -103,8 +103,7 @@ struct alignas(64) ShotDev {
     int kb;                   // z-chunk length of the z-marching kernels
     int ztx, zty, nkz;        // z-marching tiles along x, y and z-chunks
     int zb, zb_pad;           // z-marching blocks, padded to a multiple of 8
-    int ftx, fty;             // 32 x 8 (pair: 32 x 16) tiles along x and y of the pair and
-                              // Fortran kernels
+    int ftx, fty;             // 32 x 8 (pair: 32 x 16) tiles along x and y of the pair kernels
     int pair;                 // 1: fused kernels update x-pairs of cells (even ix)
     int ltx, lty, lkz;        // LDS-kernel tiles along x, y and z-chunks
     int lkb;                  // LDS-kernel z-chunk length (planes)
@@ -224,15 +223,14 @@ hipError_t launch_hfield_l(const ShotDev *d, int ns, const int *pre, int nblocks
 // ring of more than one slot
 hipError_t launch_ehfield_l(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                             hipStream_t st);
-// Fortran-variant step (fdtd_fortran.hip): Hz source points before the E
-// update (rec_prev, j > 0: after the H receivers of local step j - 1), then
-// per-cell E + CPML-E and H + CPML-H over 32 x 8 tiles (rec_e: the H launch also
-// gathers the E receivers of step j)
-hipError_t launch_source_hz(const ShotDev *d, int ns, int j, hipStream_t st, bool rec_prev = false);
-hipError_t launch_efield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           hipStream_t st);
-hipError_t launch_hfield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
-                           hipStream_t st, bool rec_e = false);
+// Fortran-variant step (fdtd_fortran.hip): per-cell E + CPML-E and H + CPML-H, both with
+// the step's Hz source points.  rec_prev (j > 0): the E launch also gathers the H
+// receivers of local step j - 1; rec_e: the H launch also gathers the E receivers of
+// step j.
+hipError_t launch_efield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j, hipStream_t st,
+                           bool rec_prev);
+hipError_t launch_hfield_v(const ShotDev *d, int ns, const int *pre, int nblocks, int j, hipStream_t st,
+                           bool rec_e);
 hipError_t launch_receivers(const ShotDev *d, int ns, int j, int nover, int inplace,
                             hipStream_t st, int hf = 0);
 // h: the H ring into acc_h (shots with H sums) instead of the E ring into acc

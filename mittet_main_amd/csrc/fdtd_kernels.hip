@@ -45,53 +45,6 @@ __device__ __forceinline__ double dplus(const GLOBAL double *__restrict__ F, int
     return c1 * F[c + s] - c1 * F[c] + c2 * F[c + 2 * s] - c2 * F[c - s];
 }
 
-__device__ __forceinline__ int find_shot(const int *__restrict__ pre, int ns, int b)
-{
-    int s = 0;
-    while (s + 1 < ns && b >= pre[s + 1])
-        ++s;
-    return s;
-}
-
-// slab position of index r on an axis of length n with nc-cell shells
-__device__ __forceinline__ int slab_pos(int r, int n, int nc)
-{
-    return r < nc ? r : r - (n - 2 * nc);
-}
-
-// Absolute step of local index 0 of the current chunk.  Every lane of a launch
-// reads the same word, which the previous chunk's k_advance wrote: a scalar
-// load through the constant address space serves it from the scalar cache
-// instead of a vector round trip to L2 per wave.
-__device__ __forceinline__ int chunk_step(const ShotDev &S)
-{
-    return *(const __attribute__((address_space(4))) int *)S.step;
-}
-
-// ring slot q of a descriptor, q < 2 * ring (or any q when there is one slot)
-__device__ __forceinline__ int ring_slot(const ShotDev &S, int q)
-{
-    return S.ring == 1 ? 0 : (q >= S.ring ? q - S.ring : q);
-}
-
-// An axis' sigma, kappa*dl, b and c: of a lane's x or y index (rows, so that
-// neighbouring lanes read neighbouring words), or of one index for the whole
-// wave (a record, scalar loads)
-struct Quad {
-    double s, k, b, c;
-};
-template <bool H> __device__ __forceinline__ Quad quad(const double *prof, int n, int r)
-{
-    const gcp p = cb(prof);
-    const unsigned o = (unsigned)r * 8u, m = (unsigned)n * 8u;
-    return {at(p, o + m * (H ? PR_MSIG : PR_ESIG)), at(p, o + m * (H ? PR_KHD : PR_KED)),
-            at(p, o + m * (H ? PR_BH : PR_BE)), at(p, o + m * (H ? PR_CH : PR_CE))};
-}
-template <bool H> __device__ __forceinline__ Quad uquad(const double *cq, int r)
-{
-    const double *p = cq + (size_t)r * CQ_N + (H ? CQ_H : CQ_E);
-    return {uload(p), uload(p + 1), uload(p + 2), uload(p + 3)};
-}
 // range flags of a cell
 __device__ __forceinline__ int flags(const ShotDev &S, int i, int jj, int k)
 {
@@ -124,12 +77,6 @@ template <int LO, int HI> struct Off {
 // a cell pays one memory round trip instead of one per branch; the stencil
 // loads depend on no flag.  The arithmetic is the reference's expressions in
 // its order.
-__device__ __forceinline__ double dm(double f0, double fm1, double fp1, double fm2, double c1,
-                                     double c2)
-{
-    return c1 * f0 - c1 * fm1 + c2 * fp1 - c2 * fm2;
-}
-
 template <int MODE>
 __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, int i, int jj, int k,
                                             unsigned oc, int fl, int n, int si, int so, int sign)
@@ -277,12 +224,6 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
 
 // One cell of the H update + CPML-H corrections, general path, as efield_cell.
 // H is read from Hin and written to Hout (the same buffer when updated in place).
-__device__ __forceinline__ double dp(double fp1, double f0, double fp2, double fm1, double c1,
-                                     double c2)
-{
-    return c1 * fp1 - c1 * f0 + c2 * fp2 - c2 * fm1;
-}
-
 template <int MODE>
 __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin, double *Hout, int i,
                                             int jj, int k, unsigned oc, int fl, int so, int sign)
@@ -1263,9 +1204,6 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // A tile that no CPML shell touches reads no profile and takes the update where
 // ca = 1, cb = dt/eps' (E), da = 1, db = dt/mu0 (H) exactly; an axis whose
 // shell the tile does not touch contributes wave-uniform values.
-
-// Component of a halo item: components 2 and 0 have halo rows, 2 and 1 columns
-__device__ __forceinline__ int halo_comp(int hk) { return hk == 1 ? 0 : (hk == 3 ? 1 : 2); }
 
 // The first recn blocks (recn: 0, or ns rounded up to a multiple of 8 so that
 // the tile blocks keep their XCD) gather receivers, block s for shot s, with one

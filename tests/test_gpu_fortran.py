@@ -80,6 +80,33 @@ def test_fortran_step_bitwise(dims):
     m.close()
 
 
+@pytest.mark.parametrize("dims, nc", [((8, 8, 8), 2), ((17, 13, 9), 2), ((43, 25, 19), 4), ((70, 37, 12), 3),
+                                      ((131, 11, 12), 3)])
+def test_fortran_tiles_bitwise(dims, nc):
+    """Tile edges of the variant's kernels: planes below one tile, columns and rows
+    cut by the grid, and source points that both launches take off the values they
+    load: two on one cell, one in a CPML corner, one next to a tile's edge."""
+    nt = 20
+    g, sig, mu, sigw, _, rec, *_ = setup(*dims, nc=nc, nt=nt)
+    ix, iy, iz = dims
+    src = [(ix // 2, iy // 2, iz // 2), (ix // 2, iy // 2, iz // 2), (2, 2, 2),
+           (min(32, ix - 3), min(8, iy - 3), iz // 2)]
+    rec = np.array([list(c) for c in src] + [[0, 0, 0], [ix - 1, iy - 1, iz - 1]])
+    print(f"fortran tiles: {dims}, ncpml {nc}", flush=True)
+    S, tr_o = oracle_run(g, sig, mu, sigw, src, rec, nt)
+    m = Model(g, variant=1)
+    m.set_mu(mu)
+    m.media_coeff_3d(sig)
+    sh = gpu_shot(m, g, sigw, src, rec, nt)
+    sh.step_n(7)
+    sh.run()
+    np.testing.assert_array_equal(sh.traces()[:, :, :nt], tr_o[:, :, :nt])
+    for q, nm in enumerate(oracle.FIELD_NAMES):
+        np.testing.assert_array_equal(sh.field(q), S.arr(nm), err_msg=nm)
+    sh.close()
+    m.close()
+
+
 def test_fortran_shots_in_a_batch_equal_alone():
     nt = 30
     g, sig, mu, sigw, src, rec, *_ = setup(28, 24, 22, nt=nt, seed=3)
