@@ -26,9 +26,6 @@
 #ifndef MT_FLUSH_WAVES
 #define MT_FLUSH_WAVES 4
 #endif
-#ifndef MT_FLUSH_G
-#define MT_FLUSH_G 8
-#endif
 
 
 namespace mt {
@@ -443,150 +440,141 @@ __global__ void k_receivers(const ShotDev *__restrict__ D, int j, int nover, int
 }
 
 // Volume running DFT over the last L ring slots: acc += E[n] * w[n] in step
-// order.  All NF accumulators of a component stay in registers while the slots
+// order.  All NF accumulators of a cell's component stay in registers while the slots
 // stream past, so every frequency is an independent dependency chain; each
 // accumulator still receives its terms in ascending step order (bit-identical
 // to the per-step running sum).
-// The chunk's weights (<= RING_MAX steps x FLUSH_NF_MAX frequencies) are staged
-// in LDS once per block and read back as wave-uniform LDS broadcasts.  A block
-// covers FLUSH_CELLS cells: two adjacent cells per lane with 16-byte loads
-// where the strides are even (one weight read serves both; at 288^3 with 8
-// frequencies the flush takes 17.4-18.1 ms per 128 steps against 19.0-19.6 ms
-// for one cell per lane), else two lane-contiguous halves one cell at a time.
-constexpr int FLUSH_NF_MAX = 8;
+// Bound by memory (24 B per cell and slot, 96 B per cell and frequency and flush).  A
+// lane has the next FLUSH_G samples of a component (one for each of two cells) in flight
+// while it sums those before; the weights are the same for every lane and come through the scalar cache.
+// A block covers FLUSH_CELLS cells of one component: two adjacent cells per lane with
+// 16-byte loads where the strides are even, else two lane-contiguous halves one cell
+// at a time.  4 frequencies: 84^3 x 64 slots 190 us (6.0 TB/s), 216^3 x 32 slots 2.08 to
+// 2.11 ms (5.5), 245 us and 2.34 ms with the components one after the other in a block, four
+// samples loaded and then summed, and weights in LDS (32 KB a block).  Two, four or
+// eight samples ahead: 186, 189, 193 us and 2.23, 2.33, 2.40 ms; with plain loads and
+// stores 221 us; two or three blocks a CU instead of four 272 or 217 us.
+constexpr int FLUSH_NF_MAX = 8, FLUSH_G = 2;
 
-template <int NF>
-__device__ __forceinline__ void flush_cell(const ShotDev &S, const double *src, double *acc, int c,
-                                           int Lv, const double2 *__restrict__ wsh)
+template <int V> struct Cells;
+template <> struct Cells<1> {
+    double v[1];
+    __device__ __forceinline__ void load(gcp p, unsigned o)
+    {
+        v[0] = __builtin_nontemporal_load((const GLOBAL double *)(p + o));
+    }
+};
+template <> struct Cells<2> {
+    double v[2];
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    __device__ __forceinline__ void load(gcp p, unsigned o)
+    {
+        const d2 t = __builtin_nontemporal_load((const GLOBAL d2 *)(p + o));
+        v[0] = t.x;
+        v[1] = t.y;
+    }
+};
+
+// cells base + o/8 ... of component d; W the chunk's weights [Lv][NF] complex
+template <int NF, int V>
+__device__ __forceinline__ void flush_cells(const ShotDev &S, const double *src, double *acc, size_t base,
+                                            unsigned o, int d, int Lv, const double *__restrict__ W)
 {
-    constexpr int G = MT_FLUSH_G;  // samples loaded together: G loads in flight per lane
-    const int N = S.n, ring = S.ring, cur = S.cur;
-    GLOBAL double *__restrict__ A = gm(acc);
-    for (int d = 0; d < 3; ++d) {
-        double2 a[NF];
+    constexpr int G = V == 2 ? FLUSH_G / 2 : FLUSH_G;
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const int ring = S.ring;
+    const size_t step = (size_t)S.sstride * 8;
+    const gcp E = cb(src) + ((size_t)d * S.n + base) * 8;
+    int slot = S.cur;
+    auto next = [&]() {   // slot of the next sample, the same for every lane
+        slot = slot + 1 == ring ? 0 : slot + 1;
+        return E + (size_t)slot * step;
+    };
+    Cells<V> e[G], p[G];
+    const int full = Lv / G * G;
+    if (full)
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            a[f].x = A[2 * (((size_t)d * NF + f) * S.astride + c)];
-            a[f].y = A[2 * (((size_t)d * NF + f) * S.astride + c) + 1];
-        }
-        for (int t0 = 0; t0 < Lv; t0 += G) {
-            double e[G];
+        for (int g = 0; g < G; ++g)
+            e[g].load(next(), o);
+    d2 a[NF][V];
+    const gmp A = mb(acc) + ((size_t)d * NF * S.astride + base) * 16;
+    const size_t row = (size_t)S.astride * 16;
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const int slot = (cur + 1 + t0 + g) % ring;
-                e[g] = t0 + g < Lv ? gc(src)[(size_t)slot * S.sstride + (size_t)d * N + c] : 0.0;
-            }
+    for (int f = 0; f < NF; ++f)
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (t0 + g < Lv) {
+        for (int v = 0; v < V; ++v)
+            a[f][v] = __builtin_nontemporal_load((const GLOBAL d2 *)(A + (size_t)f * row + 2 * o + 16 * v));
+    for (int t = 0; t < full; t += G) {
+        if (t + G < full)
 #pragma unroll
-                    for (int f = 0; f < NF; ++f) {
-                        const double2 w = wsh[(t0 + g) * NF + f];
-                        a[f].x += e[g] * w.x;
-                        a[f].y += e[g] * w.y;
-                    }
+            for (int g = 0; g < G; ++g)
+                p[g].load(next(), o);
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                const double wx = uload(W + 2 * ((size_t)(t + g) * NF + f)),
+                             wy = uload(W + 2 * ((size_t)(t + g) * NF + f) + 1);
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    a[f][v].x += e[g].v[v] * wx;
+                    a[f][v].y += e[g].v[v] * wy;
                 }
             }
-        }
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            e[g] = p[g];
+    }
+    for (int t = full; t < Lv; ++t) {
+        Cells<V> x;
+        x.load(next(), o);
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
-            A[2 * (((size_t)d * NF + f) * S.astride + c)] = a[f].x;
-            A[2 * (((size_t)d * NF + f) * S.astride + c) + 1] = a[f].y;
+            const double wx = uload(W + 2 * ((size_t)t * NF + f)), wy = uload(W + 2 * ((size_t)t * NF + f) + 1);
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                a[f][v].x += x.v[v] * wx;
+                a[f][v].y += x.v[v] * wy;
+            }
         }
     }
-}
-
-// Two adjacent cells per lane (c even; n, slot and accumulator strides even,
-// so every access is a 16-byte one): the same sums as flush_cell for each
-// cell, with one weight read from LDS per sample for both.
-template <int NF>
-__device__ __forceinline__ void flush_pair(const ShotDev &S, const double *src, double *acc, int c,
-                                           int Lv, const double2 *__restrict__ wsh)
-{
-    constexpr int G = MT_FLUSH_G / 2;
-    const int N = S.n, ring = S.ring, cur = S.cur;
-    GLOBAL double *__restrict__ A = gm(acc);
-    for (int d = 0; d < 3; ++d) {
-        double2 a[NF], b[NF];
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            const GLOBAL double2 *p =
-                (const GLOBAL double2 *)(A + 2 * (((size_t)d * NF + f) * S.astride + c));
-            a[f].x = p[0].x;
-            a[f].y = p[0].y;
-            b[f].x = p[1].x;
-            b[f].y = p[1].y;
-        }
-        for (int t0 = 0; t0 < Lv; t0 += G) {
-            double2 e[G];
+    for (int f = 0; f < NF; ++f)
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const int slot = (cur + 1 + t0 + g) % ring;
-                double2 v{0.0, 0.0};
-                if (t0 + g < Lv) {
-                    const GLOBAL double2 *p = (const GLOBAL double2 *)(gc(src) + (size_t)slot * S.sstride +
-                                                                       (size_t)d * N + c);
-                    v.x = (*p).x;
-                    v.y = (*p).y;
-                }
-                e[g] = v;
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (t0 + g < Lv) {
-#pragma unroll
-                    for (int f = 0; f < NF; ++f) {
-                        const double2 w = wsh[(t0 + g) * NF + f];
-                        a[f].x += e[g].x * w.x;
-                        a[f].y += e[g].x * w.y;
-                        b[f].x += e[g].y * w.x;
-                        b[f].y += e[g].y * w.y;
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            GLOBAL double *p = A + 2 * (((size_t)d * NF + f) * S.astride + c);
-            p[0] = a[f].x;
-            p[1] = a[f].y;
-            p[2] = b[f].x;
-            p[3] = b[f].y;
-        }
-    }
+        for (int v = 0; v < V; ++v)
+            __builtin_nontemporal_store(a[f][v], (GLOBAL d2 *)(A + (size_t)f * row + 2 * o + 16 * v));
 }
 
 // any frequency count: groups of 4 accumulators, weights from global memory
 __device__ __forceinline__ void flush_cell_any(const ShotDev &S, const double *src, double *acc,
-                                               int c, int n0, int Lv)
+                                               int c, int d, int n0, int Lv)
 {
     const int N = S.n, ring = S.ring, cur = S.cur, nf = S.nf;
     const GLOBAL double *__restrict__ W = gc(S.w) + 2 * (size_t)n0 * nf;
     GLOBAL double *__restrict__ A = gm(acc);
-    for (int d = 0; d < 3; ++d)
-        for (int f0 = 0; f0 < nf; f0 += 4) {
-            const int nq = nf - f0 < 4 ? nf - f0 : 4;
-            double2 a[4];
+    for (int f0 = 0; f0 < nf; f0 += 4) {
+        const int nq = nf - f0 < 4 ? nf - f0 : 4;
+        double2 a[4];
+        for (int q = 0; q < nq; ++q) {
+            a[q].x = A[2 * (((size_t)d * nf + f0 + q) * S.astride + c)];
+            a[q].y = A[2 * (((size_t)d * nf + f0 + q) * S.astride + c) + 1];
+        }
+        int slot = cur;
+        for (int t = 0; t < Lv; ++t) {
+            slot = slot + 1 == ring ? 0 : slot + 1;
+            const double e = gc(src)[(size_t)slot * S.sstride + (size_t)d * N + c];
             for (int q = 0; q < nq; ++q) {
-                a[q].x = A[2 * (((size_t)d * nf + f0 + q) * S.astride + c)];
-                a[q].y = A[2 * (((size_t)d * nf + f0 + q) * S.astride + c) + 1];
-            }
-            int slot = cur;
-            for (int t = 0; t < Lv; ++t) {
-                slot = slot + 1 == ring ? 0 : slot + 1;
-                const double e = gc(src)[(size_t)slot * S.sstride + (size_t)d * N + c];
-                for (int q = 0; q < nq; ++q) {
-                    const double wx = W[2 * ((size_t)t * nf + f0 + q)];
-                    const double wy = W[2 * ((size_t)t * nf + f0 + q) + 1];
-                    a[q].x += e * wx;
-                    a[q].y += e * wy;
-                }
-            }
-            for (int q = 0; q < nq; ++q) {
-                A[2 * (((size_t)d * nf + f0 + q) * S.astride + c)] = a[q].x;
-                A[2 * (((size_t)d * nf + f0 + q) * S.astride + c) + 1] = a[q].y;
+                const double wx = W[2 * ((size_t)t * nf + f0 + q)];
+                const double wy = W[2 * ((size_t)t * nf + f0 + q) + 1];
+                a[q].x += e * wx;
+                a[q].y += e * wy;
             }
         }
+        for (int q = 0; q < nq; ++q) {
+            A[2 * (((size_t)d * nf + f0 + q) * S.astride + c)] = a[q].x;
+            A[2 * (((size_t)d * nf + f0 + q) * S.astride + c) + 1] = a[q].y;
+        }
+    }
 }
 
 // HS = 0: the E ring into the E accumulators; HS = 1: the H ring into the H
@@ -596,8 +584,8 @@ template <int HS>
 __global__ __launch_bounds__(256, MT_FLUSH_WAVES) void k_flush(const ShotDev *__restrict__ D, int ns,
                                                                const int *__restrict__ pre, int L)
 {
-    __shared__ double2 wsh[RING_MAX * FLUSH_NF_MAX];
-    const int s = find_shot(pre, ns, blockIdx.x);
+    const int b = blockIdx.x, d = blockIdx.y;
+    const int s = find_shot(pre, ns, b);
     const ShotDev &S = D[s];
     const int nf = S.nf;
     const int n0 = chunk_step(S);
@@ -609,43 +597,33 @@ __global__ __launch_bounds__(256, MT_FLUSH_WAVES) void k_flush(const ShotDev *__
     if (nf == 0 || Lv <= 0 || !src || !acc)
         return;  // uniform over the block
     // a block covers FLUSH_CELLS = 2 * blockDim.x cells
-    const int base = (blockIdx.x - pre[s]) * FLUSH_CELLS;
-    const int ca = base + threadIdx.x, cb = ca + blockDim.x;   // lane-contiguous halves
+    const int base = (b - pre[s]) * FLUSH_CELLS;
     if (nf > FLUSH_NF_MAX || (nf != 1 && nf != 2 && nf != 3 && nf != 4 && nf != 8)) {
-        if (ca < S.n)
-            flush_cell_any(S, src, acc, ca, n0, Lv);
-        if (cb < S.n)
-            flush_cell_any(S, src, acc, cb, n0, Lv);
+        for (int c = base + threadIdx.x; c < base + FLUSH_CELLS && c < S.n; c += blockDim.x)
+            flush_cell_any(S, src, acc, c, d, n0, Lv);
         return;
     }
-    const GLOBAL double *__restrict__ W = gc(S.w) + 2 * (size_t)n0 * nf;
-    for (int q = threadIdx.x; q < Lv * nf; q += blockDim.x) {
-        wsh[q].x = W[2 * q];
-        wsh[q].y = W[2 * q + 1];
-    }
-    __syncthreads();
+    const double *W = S.w + 2 * (size_t)n0 * nf;
     if ((S.n & 1) == 0 && (S.sstride & 1) == 0 && (S.astride & 1) == 0) {
-        const int c = base + 2 * threadIdx.x;
-        if (c >= S.n)
+        if (base + 2 * (int)threadIdx.x >= S.n)
             return;
+        const unsigned o = threadIdx.x * 16u;
         switch (nf) {
-        case 1: flush_pair<1>(S, src, acc, c, Lv, wsh); break;
-        case 2: flush_pair<2>(S, src, acc, c, Lv, wsh); break;
-        case 3: flush_pair<3>(S, src, acc, c, Lv, wsh); break;
-        case 4: flush_pair<4>(S, src, acc, c, Lv, wsh); break;
-        default: flush_pair<8>(S, src, acc, c, Lv, wsh); break;
+        case 1: flush_cells<1, 2>(S, src, acc, base, o, d, Lv, W); break;
+        case 2: flush_cells<2, 2>(S, src, acc, base, o, d, Lv, W); break;
+        case 3: flush_cells<3, 2>(S, src, acc, base, o, d, Lv, W); break;
+        case 4: flush_cells<4, 2>(S, src, acc, base, o, d, Lv, W); break;
+        default: flush_cells<8, 2>(S, src, acc, base, o, d, Lv, W); break;
         }
         return;
     }
-    for (int c = ca; c <= cb; c += blockDim.x) {
-        if (c >= S.n)
-            return;
+    for (unsigned o = threadIdx.x * 8u; o < FLUSH_CELLS * 8u && base + (int)(o / 8u) < S.n; o += blockDim.x * 8u) {
         switch (nf) {
-        case 1: flush_cell<1>(S, src, acc, c, Lv, wsh); break;
-        case 2: flush_cell<2>(S, src, acc, c, Lv, wsh); break;
-        case 3: flush_cell<3>(S, src, acc, c, Lv, wsh); break;
-        case 4: flush_cell<4>(S, src, acc, c, Lv, wsh); break;
-        default: flush_cell<8>(S, src, acc, c, Lv, wsh); break;
+        case 1: flush_cells<1, 1>(S, src, acc, base, o, d, Lv, W); break;
+        case 2: flush_cells<2, 1>(S, src, acc, base, o, d, Lv, W); break;
+        case 3: flush_cells<3, 1>(S, src, acc, base, o, d, Lv, W); break;
+        case 4: flush_cells<4, 1>(S, src, acc, base, o, d, Lv, W); break;
+        default: flush_cells<8, 1>(S, src, acc, base, o, d, Lv, W); break;
         }
     }
 }
@@ -2557,9 +2535,9 @@ hipError_t launch_flush(const ShotDev *d, int ns, const int *pre_cells, int nblo
     if (L > RING_MAX)
         return hipErrorInvalidValue;
     if (h)
-        hipLaunchKernelGGL(k_flush<1>, dim3(nblocks), dim3(256), 0, st, d, ns, pre_cells, L);
+        hipLaunchKernelGGL(k_flush<1>, dim3(nblocks, 3), dim3(256), 0, st, d, ns, pre_cells, L);
     else
-        hipLaunchKernelGGL(k_flush<0>, dim3(nblocks), dim3(256), 0, st, d, ns, pre_cells, L);
+        hipLaunchKernelGGL(k_flush<0>, dim3(nblocks, 3), dim3(256), 0, st, d, ns, pre_cells, L);
     return hipGetLastError();
 }
 

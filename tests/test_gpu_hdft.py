@@ -55,6 +55,31 @@ def test_h_volume_dft_matches_oracle_steps(family, monkeypatch):
     np.testing.assert_array_equal(shot.volume_dft_h().reshape(3, len(om), -1), got)
 
 
+@pytest.mark.parametrize("nf", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("dims", [(27, 25, 23), (30, 26, 22)])
+def test_volume_dft_of_every_frequency_count(dims, nf):
+    """The flush's instances (1, 2, 3, 4, 8 frequencies, any other count), cell
+    pairs and, on an odd cell count, single cells, the last block partly filled;
+    chunks of a full ring, of one step and of the rest: E and H sums bit for bit."""
+    ix, iy, iz = dims
+    it = 26
+    om = tuple(0.5 + 0.7 * f for f in range(nf))
+    print(f"volume DFT: {dims}, nf {nf}", flush=True)
+    m, shot, S, sig, signal, src, rec, om, dt = setup_pair(ix=ix, iy=iy, iz=iz, seed=35, it=it, ring=7, omegas=om)
+    shot.enable_volume_dft_h()
+    for steps in (7, 1, 10, 100):
+        shot.step_n(steps)
+    w = oracle.dft_weights(it, dt, OM0, om)
+    re, im = oracle_h_sums(S, signal, src, it, w)
+    got = shot.volume_dft_h().reshape(3, nf, -1)
+    np.testing.assert_array_equal(got.real, re)
+    np.testing.assert_array_equal(got.imag, im)
+    _, _, S2, *_ = setup_pair(ix=ix, iy=iy, iz=iz, seed=35, it=it, ring=7, omegas=om)
+    _, acc = S2.forward(0, signal, tuple(c + 1 for c in src), it - 1, rec1=rec + 1, it=it, weights=w)
+    np.testing.assert_array_equal(shot.volume_dft().reshape(3, nf, -1), acc)
+    assert np.abs(got).max() > 0
+
+
 def test_h_volume_dft_in_a_batch_equals_alone():
     specs = [dict(ix=30, iy=26, iz=22, seed=32, it=50), dict(ix=26, iy=24, iz=20, seed=33, it=40)]
     alone = []
