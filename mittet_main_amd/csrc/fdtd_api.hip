@@ -395,9 +395,14 @@ void magic_div(unsigned d, unsigned &mul, int &sh)
 
 int tiles(int n, int t) { return (n + t - 1) / t; }
 
-// Tile w x h of the per-cell kernels on planes of ix x iy cells: the shape with
-// the fewest idle lanes and halo loads (6 (w + h) values per tile), rows of at
-// least 16 cells (128 B).
+// Tile w x h of the per-cell kernels' contiguous runs on planes of ix x iy cells: the
+// shape with the fewest idle lanes and halo loads (6 (w + h) values per tile), rows of
+// at least 16 cells (128 B).  Tiles in layers are 32 x 8: their rows are whole cache lines
+// where the grid's are (16 x 16 / 20 x 12 / 24 x 10 / 28 x 9 / 32 x 8 at 288^3 157 / 230 / 195 /
+// 216 / 155 ms per pass, 216^3 with a volume DFT 241 / 262 / 231 / 256 / 219), and so they are
+// in runs of launches that all but fill the Infinity Cache (kWideMinBytes: 152^3 25.4 /
+// 27.2 / 26.5 / 25.7 / 24.1); below, lanes count more (120^3 13.6 / 13.2 / 13.1 / 14.5 / 13.6,
+// 131 x 97 x 75 11.8 / 11.6 / 11.5 / 11.1 / 12.2).
 void cell_tile(int ix, int iy, int &w, int &h)
 {
     double best = 0.0;
@@ -494,15 +499,27 @@ int lds_chunk(int ltx, int lty, int nz)
     return 4;
 }
 
-// Grids from this many cells up take the LDS family.  Graph-captured steps
-// with a 4-frequency volume DFT, 16 receivers, Gcell-updates/s of the LDS /
-// per-cell family: 84^3 9.8 / 12.7, 120^3 14.3 / 16.1, 152^3 16.9 / 15.7,
-// 216^3 18.1 / 16.5.  MITTET_FDTD_LDS=1 takes it on any grid.
-constexpr long long kLdsMinCells = 2500000;
+// Shots that take the LDS family (two interior and two shell launches a step instead of
+// two over whole planes).  Since the per-cell launches take their tiles in layers
+// (ftile) they are the faster ones, ms per pass LDS / per-cell: 136^3 23.4 / 18.1, 160^3
+// 36.1 / 29.1, 176^3 48.2 / 38.5, 240^3 32.6 / 29.6, 288^3 157.2 / 156.3, 400^3 128 / 125,
+// 216^3 with a volume DFT 222 / 220, 600x500x60 42.0 / 41.7, 60x500x600 65 / 51.  Left
+// are large grids with an odd row, whose 32-cell tiles straddle a cache line more on
+// every row: 301x240x250 48.0 / 52.2, 331x277x201 47.2 / 49.7, 243x251x260 43.6 / 46.2, 289^3
+// 66.0 / 66.8 (309^3 79.7 / 79.0, 349x300x200 56.7 / 54.6; below 12 M cells 217x219x221 28.9 /
+// 28.4, 151x149x147 8.0 / 7.2).  MITTET_FDTD_LDS=1 takes it on any grid.
+constexpr long long kLdsMinCells = 12000000;
+// ... and, with MITTET_FDTD_FUSE=1, those of at least so many cells (takes_fused)
+constexpr long long kFuseMinCells = 2500000;
 
-// Launches whose steps touch more bytes than the 256 MB Infinity Cache load
+// Launches whose steps touch more bytes than the Infinity Cache can hold of them load
 // and store their once-touched field values non-temporally (stream_nt).
-constexpr long long kNtMinBytes = 256LL << 20;
+constexpr long long kNtMinBytes = 240LL << 20;
+constexpr long long kWideMinBytes = 200LL << 20;
+
+// Bytes one step of a shot touches: E read, E written (to the next ring slot, or in place
+// with one slot), H, and the two coefficient arrays.
+long long step_bytes(long long cells, long long ring) { return cells * (ring > 1 ? 88 : 64); }
 
 // Whether a C-variant shot takes the LDS family (family 3): size, no z-chunk
 // or x-pair override, and a CPML-free interior to march.
@@ -511,7 +528,8 @@ bool takes_lds(const fwi3d_grid_params &p, int zchunk)
     const long long N = (long long)p.ix * p.iy * p.iz;
     const int xlo = (p.ncpml + 15) / 16 * 16;
     const bool pair = p.ix % 2 == 0 && env_pad("MITTET_FDTD_PAIR", 0);
-    const bool lds_size = N >= kLdsMinCells || env_pad("MITTET_FDTD_LDS", 0);
+    const bool lds_size = (p.ix % 2 && N >= kLdsMinCells) || env_pad("MITTET_FDTD_LDS", 0) ||
+                          (N >= kFuseMinCells && env_pad("MITTET_FDTD_FUSE", 0));
     return zchunk == 0 && !pair && lds_size && p.ncpml >= 2 && xlo < p.ix - p.ncpml &&
            p.ncpml < p.iy - p.ncpml && p.ncpml < p.iz - p.ncpml && !env_pad("MITTET_FDTD_NOLDS", 0);
 }
@@ -1112,11 +1130,14 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.row = 8u * (unsigned)p.ix;
     d.pb = 8u * (unsigned)(p.ix * p.iy);
     cell_tile(p.ix, p.iy, d.tw, d.th);
+    if (step_bytes((long long)N, ring) > kWideMinBytes) {
+        d.tw = mt::ZX;
+        d.th = mt::ZY;
+    }
     d.ttx = tiles(p.ix, d.tw);
     d.tpp = d.ttx * tiles(p.iy, d.th);
     magic_div((unsigned)d.ttx, d.xmul, d.xsh);
     magic_div((unsigned)d.tpp, d.tmul, d.tsh);
-    magic_div((unsigned)tiles(d.tpp, 8), d.emul, d.esh);
     d.opp = tiles(p.ix * p.iy, mt::PT);
     magic_div((unsigned)d.opp, d.omul, d.osh);
     magic_div((unsigned)p.ix, d.imul, d.ish);
@@ -1158,6 +1179,8 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     d.pair = (p.ix % 2 == 0 && env_pad("MITTET_FDTD_PAIR", 0)) ? 1 : 0;
     d.ftx = d.pair ? tiles(p.ix, 32) : tiles(p.ix, mt::ZX);
     d.fty = d.pair ? tiles(p.iy, 16) : tiles(p.iy, mt::ZY);
+    magic_div((unsigned)tiles(d.ftx * d.fty, 8), d.emul, d.esh);
+    magic_div((unsigned)d.ftx, d.fmul, d.fsh);
     d.fb = d.pair ? d.ftx * d.fty * p.iz : d.tpp * p.iz;
     d.fb_pad = tiles(d.fb, 8) * 8;
     d.e = s->d_e;
@@ -1197,8 +1220,7 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
     }
     // family 3: LDS z-marching kernels over the CPML-free interior (rows start
     // 128-byte aligned, at ncpml rounded up to 16 cells), per-cell kernels over
-    // the tiles that hold any other cell.  Below kLdsMinCells the per-cell
-    // family alone (two launches per step instead of four) is faster.
+    // the tiles that hold any other cell (takes_lds)
     d.shell = nullptr;
     const int xlo = (p.ncpml + 15) / 16 * 16;
     if (s->kind == 0 && takes_lds(p, sp->zchunk)) {
@@ -1246,7 +1268,7 @@ int fwi3d_shot_create(fwi3d_model *m, const fwi3d_shot_params *sp, fwi3d_shot **
         }
     }
     s->nblocks = s->kind == 2 ? d.zb_pad : d.fb_pad;
-    s->nlayer = s->kind == 0 ? tiles(d.tpp, 8) * 8 * p.iz : s->nblocks;
+    s->nlayer = s->kind == 0 ? tiles(d.ftx * d.fty, 8) * 8 * p.iz : s->nblocks;
     s->nlayer_l = tiles(d.ltx * d.lty, 8) * 8 * d.lkz;
     s->ncellblocks = tiles((int)N, mt::FLUSH_CELLS);
     if ((rc = upload_desc(s)) || (rc = fwi3d_set_zero_eh(s))) {
@@ -1391,23 +1413,16 @@ int fwi3d_hpml_abcs4(fwi3d_shot *s) { return single_op(s, 3, 1, 0); }
 int fwi3d_read_source_3d(fwi3d_shot *s, int step) { return single_op(s, 4, 1, step); }
 int fwi3d_output(fwi3d_shot *s, int step) { return single_op(s, 5, 1, step); }
 
-// Bytes per cell one step touches: E read, E written (to the next ring slot,
-// or in place with one slot), H, and the two coefficient arrays.
-long long step_touch_bytes(const fwi3d_shot *s)
-{
-    return (long long)s->desc.n * (s->ring > 1 ? 88 : 64);
-}
+long long step_touch_bytes(const fwi3d_shot *s) { return step_bytes(s->desc.n, s->ring); }
 
-// Non-temporal field traffic pays once a launch's fields no longer stay in the
-// Infinity Cache from one half-step to the next: then L2 and that cache keep
-// the stencil neighbours that other tiles still read.  Single shots with a
-// 12-cell CPML and a 4-frequency volume DFT (88 B per cell), Gcell-updates/s
-// without / with: 96^3 17.7 / 15.2, 120^3 19.0 / 15.6, 136^3 (211 MiB) 16.3 /
-// 15.5, 152^3 (295 MiB) 18.4 / 18.8, 184^3 17.9 / 19.0, 216^3 19.3 / 20.6,
-// 280^3 20.2 / 21.4-23.1; 84^3 with a 10-cell CPML 14.8 / 12.9.  Without DFT
-// (one slot, 64 B per cell): 184^3 20.3 / 21.4, 216^3 22.2 / 23.5, 280^3
-// 23.1 / 25.2, while eight 152^3 shots (214 MiB) run their forward in 4.79 s
-// without, 5.23 s with.  MITTET_FDTD_NT=0 or 1 overrides the choice.
+// Non-temporal field traffic and tiles in layers pay once a launch's fields no longer
+// stay in the 256 MB Infinity Cache from one half-step to the next: then L2 and that
+// cache keep the stencil neighbours that other tiles still read.  Single shots with a
+// 12-cell CPML, 64 B per cell, ms per pass without / with: 120^3 13.2 / 16.8, 144^3 (182
+// MiB) 19.9 / 22.4, 152^3 (214 MiB) 24.1 / 29.1, 160^3 (250 MiB) 32.6 / 29.1, 176^3 44.2 /
+// 38.5, 192^3 59.6 / 50.0, 288^3 176 / 155; with a 4-frequency volume DFT, 88 B per cell:
+// 128^3 (176 MiB) 21.6 / 23.5, 144^3 (251 MiB) 31.3 / 32.2, 152^3 39.3 / 37.4, 216^3 236 / 220.
+// Four shots of 84^3 to 120^3 (264 MiB) 40.1 / 33.8.  MITTET_FDTD_NT=0 or 1 overrides.
 bool stream_nt(long long touch_bytes)
 {
     const long long e = env_pad("MITTET_FDTD_NT", -1);

@@ -94,8 +94,8 @@ struct alignas(64) ShotDev {
     double dl[3];
     int lo[3], hi[3];         // LDS-kernel region [lo, hi) per axis (inside the CPML-free interior)
     int it;                   // samples; steps 0 .. it-2 exist
-    unsigned emul;            // per-cell tiles in layers (ftile): division by ceil(tpp / 8)
-    int esh;
+    unsigned emul, fmul;      // per-cell tiles in layers (ftile): division by an XCD's tiles of a
+    int esh, fsh;             // plane, ceil(ftx fty / 8), and by ftx
     int opp, osh;             // stand-alone operators: PT-cell runs of a plane, division by it
     unsigned omul, imul;      // ... and by ix
     int ish;

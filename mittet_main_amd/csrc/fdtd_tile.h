@@ -97,25 +97,29 @@ struct FTile {
 template <bool LAYERS, class G> __device__ __forceinline__ bool ftile(const G &S, int b, FTile &T)
 {
     if (!S.shell) {
-        unsigned r;
         if constexpr (LAYERS) {
-            const unsigned m = (unsigned)b >> 3, e = ((unsigned)S.tpp + 7u) >> 3;
+            const unsigned m = (unsigned)b >> 3, tpp = (unsigned)(S.ftx * S.fty), e = (tpp + 7u) >> 3;
             T.k = (int)(((unsigned long long)m * S.emul) >> S.esh);   // m / e
-            r = ((b + (T.k >> 3)) & 7) * e + (m - (unsigned)T.k * e);
-            if (T.k >= S.iz || r >= (unsigned)S.tpp)
+            const unsigned r = ((b + (T.k >> 3)) & 7) * e + (m - (unsigned)T.k * e);
+            if (T.k >= S.iz || r >= tpp)
                 return false;
+            const unsigned ty = (unsigned)(((unsigned long long)r * S.fmul) >> S.fsh);   // r / ftx
+            T.w = ZX;
+            T.h = ZY;
+            T.x0 = (int)(r - ty * S.ftx) * ZX;
+            T.y0 = (int)ty * ZY;
         } else {
             const unsigned q = (b & 7) * (S.fb_pad >> 3) + (b >> 3);
             if (q >= (unsigned)S.fb)
                 return false;
             T.k = (int)(((unsigned long long)q * S.tmul) >> S.tsh);
-            r = q - (unsigned)T.k * S.tpp;
+            const unsigned r = q - (unsigned)T.k * S.tpp;
+            const unsigned ty = (unsigned)(((unsigned long long)r * S.xmul) >> S.xsh);
+            T.w = S.tw;
+            T.h = S.th;
+            T.x0 = (int)(r - ty * S.ttx) * T.w;
+            T.y0 = (int)ty * T.h;
         }
-        const unsigned ty = (unsigned)(((unsigned long long)r * S.xmul) >> S.xsh);
-        T.w = S.tw;
-        T.h = S.th;
-        T.x0 = (int)(r - ty * S.ttx) * T.w;
-        T.y0 = (int)ty * T.h;
         T.yend = S.iy;
         T.region = false;
         return true;
