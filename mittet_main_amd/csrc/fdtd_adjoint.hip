@@ -87,10 +87,9 @@ __global__ void k_adj_inject(AdjArgs A, const double *__restrict__ g, int nrec,
 // stencils are loaded directly.  Bound by memory: 6 weights read and 6 written,
 // lambda, the forward states, the gradient and psi are about 250 B per cell and
 // pass.  152^3 with a 12-cell CPML, per step: 101 and 98 us of events around the two
-// launches, 72 and 44 us around those of the region.  With the step's replay that
-// is 531 us, 574 before each gather shared its launch with a local part (then 8
-// launches a step); at 61 x 50 x 44, where all cells are this kernel's but the
-// innermost, 75 and 89 us.
+// launches, 72 and 44 us around those of the region.  With the step's replay a step
+// takes 512 us there, 574 before each gather shared its launch with a local part (then
+// 8 launches a step); 45 us at 61 x 50 x 44, where every cell is this kernel's, 89 then.
 template <bool EP>
 __global__ __launch_bounds__(PT) void k_adj_cell(AdjArgs A, int gather, int local)
 {

@@ -2406,12 +2406,20 @@ static bool kappa_is_one(const fwi3d_shot *s)
 // LDS region of the adjoint: [ncpml + 1, n - ncpml - 1) on each axis (x start
 // rounded up to 8 cells), where the update is CPML-free and no transposed psi
 // stencil (offsets -2..+2 from a CPML face cell) reaches; empty without
-// kappa = 1 or when the LDS kernels are switched off
+// kappa = 1, when the LDS kernels are switched off, or on grids below
+// kAdjRegionMin cells.  A region cell moves 216 B a step instead of 360, but the
+// region costs two more launches and z-chunks too short for its kernels on small
+// grids.  Adjoint and replay us per step with a region / without: 61x50x44 69.6 / 45.1,
+// 70^3 107 / 82, 90^3 152 / 136, 104^3 208 / 190, 120^3 293 / 285, 136^3 398 / 386, 152^3
+// 515 / 525.  MITTET_FDTD_LDS=1 takes it on any grid.
+constexpr long long kAdjRegionMin = 3000000;
+
 static bool adj_region(const fwi3d_shot *s, int lo[3], int hi[3])
 {
     const ShotDev &d = s->desc;
     const int n[3] = {d.ix, d.iy, d.iz};
-    bool ok = d.nc >= 2 && kappa_is_one(s) && !env_pad("MITTET_FDTD_NOLDS", 0);
+    bool ok = d.nc >= 2 && kappa_is_one(s) && !env_pad("MITTET_FDTD_NOLDS", 0) &&
+              (d.n >= kAdjRegionMin || env_pad("MITTET_FDTD_LDS", 0));
     for (int a = 0; a < 3; ++a) {
         lo[a] = a == 0 ? (d.nc + 1 + 7) / 8 * 8 : d.nc + 1;
         hi[a] = n[a] - d.nc - 1;
@@ -2423,11 +2431,16 @@ static bool adj_region(const fwi3d_shot *s, int lo[3], int hi[3])
     return ok;
 }
 
-// per-cell tiles of the adjoint: around its LDS region, or none (every tile)
+// Per-cell tiles of the adjoint: around its LDS region, or every 32 x 8 tile (the
+// empty region's complement), dealt to the XCDs as complement_tiles has it; none on
+// small grids, whose launches take the shot's tiles in contiguous runs.  Adjoint and
+// replay us per step in runs / from the list: 61x50x44 45.1 / 46.2, 70^3 82 / 86, 90^3 149 /
+// 136, 104^3 215 / 190, 131x97x75 184 / 177, 152^3 559 / 525.
+constexpr long long kAdjListMin = 500000;
 static std::vector<int4> adj_tiles(const fwi3d_shot *s)
 {
     int lo[3], hi[3];
-    if (!adj_region(s, lo, hi))
+    if (!adj_region(s, lo, hi) && s->desc.n < kAdjListMin)
         return {};
     return complement_tiles(s->desc.ix, s->desc.iy, s->desc.iz, lo, hi);
 }

@@ -109,6 +109,24 @@ def test_lds_adjoint_at_region_edges(ix, iy, iz, nc, monkeypatch):
     assert np.abs(g1 - g0).max() <= 1e-12 * np.abs(g0).max()
 
 
+def test_listed_adjoint_tiles_without_a_region(monkeypatch):
+    """From half a million cells without an LDS region the adjoint takes its tiles
+    from a list (97 x 83 x 67, tiles cut on both axes): the gradient with a region
+    up to rounding, as above."""
+    def run():
+        P, sig0, _ = problem(seed=9, ix=97, iy=83, iz=67, nc=6, it=40)
+        _, g = P.value_and_grad(np.log(sig0))
+        P.close()
+        return g
+
+    print("adjoint tiles from a list: 97 x 83 x 67", flush=True)
+    g1 = run()
+    monkeypatch.setenv("MITTET_FDTD_NOLDS", "1")
+    g0 = run()
+    assert np.all(np.isfinite(g0)) and np.abs(g1).max() > 0
+    assert np.abs(g1 - g0).max() <= 1e-12 * np.abs(g1).max()
+
+
 def test_segment_length_does_not_change_gradient():
     P1, sig0, _ = problem(seed=3, segment=7)
     P2, _, _ = problem(seed=3, segment=64)
