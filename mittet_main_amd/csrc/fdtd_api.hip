@@ -2207,10 +2207,11 @@ struct fwi3d_grad {
     int seg = 0, nseg = 0, nt = 0;    // top segment length and count
     int leaf = 0;                     // steps replayed with every state kept
     size_t state = 0;                 // doubles per stored state
+    size_t lstate = 0;                // ... of a replayed segment (E and H alone)
     size_t off_h = 0, off_psi[3] = {0, 0, 0};
     double *ckpt = nullptr;           // nseg states
     std::vector<double *> inner;      // depth l >= 1: slots for the starts of a segment's pieces
-    double *buf = nullptr;            // leaf + 1 states
+    double *buf = nullptr;            // leaf + 1 states of a replayed segment
     double *adj = nullptr;            // adjoint state (one state)
     double *tmp = nullptr;            // weights of the per-cell passes (2 x 6N)
     double *grad = nullptr;           // N
@@ -2245,6 +2246,7 @@ static void state_layout(fwi3d_grad *g)
         o += mt::PSI_N * (size_t)d.slab[a];
     }
     g->state = state_pad(o);
+    g->lstate = state_pad(g->off_psi[0]);
 }
 
 // the shot's live state (E slot 0 -- ring 1 -- H, the psi slabs) in the
@@ -2263,20 +2265,6 @@ static mt::StateSegs state_segs(const fwi3d_grad *g)
         v.count[2 + a] = mt::PSI_N * (size_t)s->desc.slab[a];
     }
     v.nseg = 5;
-    return v;
-}
-
-// the segments from `first` on (1: H and the psi slabs, stored from offset
-// off_h of a state; 2: the psi slabs, from off_psi[0])
-static mt::StateSegs state_segs_from(const fwi3d_grad *g, int first)
-{
-    const mt::StateSegs all = state_segs(g);
-    mt::StateSegs v{};
-    for (int k = first; k < all.nseg; ++k) {
-        v.live[k - first] = all.live[k];
-        v.count[k - first] = all.count[k];
-    }
-    v.nseg = all.nseg - first;
     return v;
 }
 
@@ -2302,12 +2290,12 @@ static int set_step(fwi3d_shot *s, int n)
 // slots than a leaf has steps): step t reads E of slot t and writes E of slot
 // t + 1 in place of the shot's E, and each step's receiver gather rides on the
 // next step's E launch as in a ring shot's chunk.  For the per-cell and LDS
-// kernel families H and the psi slabs go the same way (rings over the states'
-// H and psi parts, see hsel and ShotDev::pstride), so the steps write every
-// stored state themselves and nothing is copied; the other families update H
-// and psi in place and copy them into each slot.  The last slot is copied back
-// to the shot afterwards (E, or the whole state with the rings), which leaves
-// the shot's state at the segment's end as an in-place replay would.
+// kernel families H goes the same way (a ring over the states' H parts, see
+// hsel), so the steps write every stored state themselves and nothing is copied;
+// the other families update H in place and copy it into each slot.  psi, which the
+// adjoint does not read, stays in the shot.  The last slot is copied back to the
+// shot afterwards (E, with the ring H too), which leaves the shot's state at the
+// segment's end as an in-place replay would.
 static int replay_segment(fwi3d_grad *g, int L)
 {
     fwi3d_shot *s = g->s;
@@ -2320,28 +2308,28 @@ static int replay_segment(fwi3d_grad *g, int L)
     const bool hring = (f0.kind == 0 || f0.kind == 3) && !f0.fused;
     g->rdesc = s->desc;
     g->rdesc.e = g->buf;
-    g->rdesc.sstride = (long long)g->state;
+    g->rdesc.sstride = (long long)g->lstate;
     g->rdesc.ring = g->leaf + 1;
     g->rdesc.cur = 0;
     if (hring) {
         g->rdesc.h = g->buf + g->off_h;
-        g->rdesc.hstride = (long long)g->state;
-        for (int a = 0; a < 3; ++a)
-            g->rdesc.psi[a] = g->buf + g->off_psi[a];
-        g->rdesc.pstride = (long long)g->state;
+        g->rdesc.hstride = (long long)g->lstate;
     }
     HIP_TRY(hipMemcpyAsync(g->d_rdesc, &g->rdesc, sizeof(ShotDev), hipMemcpyHostToDevice, s->st));
     if (!g->replay[slot]) {
         Fam f = f0;
         f.rings = true;   // the stored states: an E ring of leaf + 1 slots
-        // a replay step reads one stored state and writes the next: E and H
-        // (and psi) both ways plus the coefficients, 112 B per cell (88 where H
-        // is updated in place and copied)
+        // a replay step reads one stored state and writes the next: E and H both
+        // ways plus the coefficients, 112 B per cell (88 where H is updated in
+        // place and copied)
         f.nt = stream_nt((long long)s->desc.n * (hring ? 112 : 88));
         f.nblocks = cell_blocks(s, f.nt);
         f.nblocks_l = lds_blocks(s, f.nt, f.fused);
         const bool fold = s->nrec && rec_folds(f);
-        const mt::StateSegs segs = state_segs_from(g, 1);   // H and psi, without the rings
+        mt::StateSegs segs{};   // H, without the ring
+        segs.live[0] = state_segs(g).live[1];
+        segs.count[0] = state_segs(g).count[1];
+        segs.nseg = 1;
         hipGraph_t graph = nullptr;
         std::lock_guard<std::recursive_mutex> lk(g_rt_mu);
         HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
@@ -2353,7 +2341,7 @@ static int replay_segment(fwi3d_grad *g, int L)
             if (s->nrec && !(fold && j + 1 < L) &&
                 mt::launch_receivers(g->d_rdesc, 1, j, -1, 0, s->st) != hipSuccess)
                 rc = fail(FWI3D_EDEVICE, "receiver launch");
-            else if (!hring && mt::launch_state_copy(segs, g->buf + g->state * (j + 1) + g->off_h,
+            else if (!hring && mt::launch_state_copy(segs, g->buf + g->lstate * (j + 1) + g->off_h,
                                                      true, s->st) != hipSuccess)
                 rc = fail(FWI3D_EDEVICE, "state copy launch");
         }
@@ -2371,10 +2359,9 @@ static int replay_segment(fwi3d_grad *g, int L)
         g->replay_len[slot] = L;
     }
     HIP_TRY(hipGraphLaunch(g->replay[slot], s->st));
-    mt::StateSegs back = state_segs(g);   // the whole state with the rings, else E
-    if (!hring)
-        back.nseg = 1;
-    HIP_TRY(mt::launch_state_copy(back, g->buf + g->state * L, false, s->st));
+    mt::StateSegs back = state_segs(g);   // E, with the ring H too
+    back.nseg = hring ? 2 : 1;
+    HIP_TRY(mt::launch_state_copy(back, g->buf + g->lstate * L, false, s->st));
     s->step += L;
     return FWI3D_OK;
 }
@@ -2455,7 +2442,8 @@ static long long grad_plan_bytes(const fwi3d_shot *s, const GradPlan &P)
     const size_t other = tmp + N + 1 + std::max<size_t>(1, 3 * (size_t)s->nrec * s->it) +
                          2 * ((size_t)s->desc.ix + s->desc.iy + s->desc.iz) +
                          2 * adj_tiles(s).size();
-    return 8LL * (long long)(P.states * state_pad(st) + other);
+    const size_t leaf = (size_t)P.seglen.back() + 1;   // states of a replayed segment: E and H
+    return 8LL * (long long)((P.states - leaf) * state_pad(st) + leaf * state_pad(6 * N) + other);
 }
 
 static int grad_new(fwi3d_shot *s, int levels, int segment, fwi3d_grad **out)
@@ -2490,7 +2478,7 @@ static int grad_new(fwi3d_shot *s, int levels, int segment, fwi3d_grad **out)
         ok = dalloc(&p, g->state * pieces) == hipSuccess;
         g->inner.push_back(p);
     }
-    if (!ok || dalloc(&g->buf, g->state * (g->leaf + 1)) != hipSuccess ||
+    if (!ok || dalloc(&g->buf, g->lstate * (g->leaf + 1)) != hipSuccess ||
         dalloc(&g->adj, g->state) != hipSuccess || dalloc(&g->tmp, tmp) != hipSuccess ||
         dalloc(&g->grad, N) != hipSuccess || dalloc(&g->grad_src, 1) != hipSuccess ||
         dalloc(&g->g, std::max<size_t>(1, 3 * (size_t)s->nrec * s->it)) != hipSuccess ||
@@ -2614,11 +2602,14 @@ static int adj_range(fwi3d_grad *g, int depth, int n0, int L, double *start, mt:
         return rc;
     if (depth == g->plan.levels - 1) {
         // replay the segment keeping every state, then step the adjoint back
-        if ((rc = state_copy(g, g->buf, true)) || (rc = replay_segment(g, L)))
+        mt::StateSegs eh = state_segs(g);
+        eh.nseg = 2;
+        HIP_TRY(mt::launch_state_copy(eh, g->buf, true, s->st));
+        if ((rc = replay_segment(g, L)))
             return rc;
         // the H local part of step t runs with step t + 1 (both states at hand),
         // that of the segment's last step on its own
-        auto state = [&](int t) { return g->buf + g->state * t; };
+        auto state = [&](int t) { return g->buf + g->lstate * t; };
         A.H0 = state(L - 1) + g->off_h;
         A.H1 = state(L) + g->off_h;
         HIP_TRY(mt::launch_adjoint_local(A, s->st));

@@ -79,9 +79,6 @@ struct alignas(64) ShotDev {
     const double *eps;        // eps' = sigma/2/omega0 per cell
     const double *cbi;        // dt/eps' per cell (cb where the CPML sigma is zero)
     double *psi[3];           // [PSI_N][slab[a]]
-    long long pstride;        // nonzero: psi in ring slots like E (slot q at psi[a] + q*pstride;
-                              // a gradient replay's stored states), read and written by the
-                              // per-cell code only
     int *step;                // absolute step of local index j = 0 of the current chunk
     int src_k;                // plane of the source cell (-1: no source) ...
     unsigned src_o;           // ... and its byte offset there

@@ -105,10 +105,6 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
     const double eps2 = at(cb(S.eps) + kp, q.o);
     const Quad X = quad<false>(S.prof[0], S.ix, i), Y = quad<false>(S.prof[1], S.iy, jj);
     const Quad Z = uquad<false>(S.cq[2], k);
-    // psi in place, or (pstride set) read from ring slot si and written to
-    // slot so like E
-    const size_t pr = S.pstride ? (size_t)si * S.pstride : 0;
-    const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
     const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
     const size_t b0 = (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
     const size_t b1 = (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
@@ -117,17 +113,17 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
     double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, az0 = 0.0, az1 = 0.0;
     if (fx) {
         q0 = (unsigned)(jj * (2 * nc) + slab_pos(i, S.ix, nc)) * 8u;
-        ax0 = at(cb(S.psi[0] + pr) + b0, q0);
-        ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
+        ax0 = at(cb(S.psi[0]) + b0, q0);
+        ax1 = at(cb(S.psi[0]) + L0 + b0, q0);
     }
     if (fy) {
         q1 = (unsigned)(slab_pos(jj, S.iy, nc) * S.ix + i) * 8u;
-        ay0 = at(cb(S.psi[1] + pr) + b1, q1);
-        ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
+        ay0 = at(cb(S.psi[1]) + b1, q1);
+        ay1 = at(cb(S.psi[1]) + L1 + b1, q1);
     }
     if (fz) {
-        az0 = at(cb(S.psi[2] + pr) + b2, q.o);
-        az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
+        az0 = at(cb(S.psi[2]) + b2, q.o);
+        az1 = at(cb(S.psi[2]) + L2 + b2, q.o);
     }
 
     // ---- arithmetic
@@ -203,16 +199,16 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
             ez -= amp;
     }
     if (fx) {
-        put_s<NT>(mb(S.psi[0] + pw) + b0, q0, px0);
-        put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, px1);
+        put_s<NT>(mb(S.psi[0]) + b0, q0, px0);
+        put_s<NT>(mb(S.psi[0]) + L0 + b0, q0, px1);
     }
     if (fy) {
-        put_s<NT>(mb(S.psi[1] + pw) + b1, q1, py0);
-        put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, py1);
+        put_s<NT>(mb(S.psi[1]) + b1, q1, py0);
+        put_s<NT>(mb(S.psi[1]) + L1 + b1, q1, py1);
     }
     if (fz) {
-        put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, pz0);
-        put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, pz1);
+        put_s<NT>(mb(S.psi[2]) + b2, q.o, pz0);
+        put_s<NT>(mb(S.psi[2]) + L2 + b2, q.o, pz1);
     }
     put_s<NT>(Eout, q.o, ex);
     put_s<NT>(Eout + nb, q.o, ey);
@@ -254,10 +250,6 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
     const double eps2 = at(cb(S.eps) + kp, q.o);
     const Quad X = quad<true>(S.prof[0], S.ix, i), Y = quad<true>(S.prof[1], S.iy, jj);
     const Quad Z = uquad<true>(S.cq[2], k);
-    // psi in place, or (pstride set) read from the ring slot before so and
-    // written to slot so like H
-    const size_t pr = S.pstride ? (size_t)(so == 0 ? S.ring - 1 : so - 1) * S.pstride : 0;
-    const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
     const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
     const size_t b0 = 2 * L0 + (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
     const size_t b1 = 2 * L1 + (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
@@ -266,17 +258,17 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
     double ax0 = 0.0, ax1 = 0.0, ay0 = 0.0, ay1 = 0.0, az0 = 0.0, az1 = 0.0;
     if (gx) {
         q0 = (unsigned)(jj * (2 * nc) + slab_pos(i, S.ix, nc)) * 8u;
-        ax0 = at(cb(S.psi[0] + pr) + b0, q0);
-        ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
+        ax0 = at(cb(S.psi[0]) + b0, q0);
+        ax1 = at(cb(S.psi[0]) + L0 + b0, q0);
     }
     if (gy) {
         q1 = (unsigned)(slab_pos(jj, S.iy, nc) * S.ix + i) * 8u;
-        ay0 = at(cb(S.psi[1] + pr) + b1, q1);
-        ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
+        ay0 = at(cb(S.psi[1]) + b1, q1);
+        ay1 = at(cb(S.psi[1]) + L1 + b1, q1);
     }
     if (gz) {
-        az0 = at(cb(S.psi[2] + pr) + b2, q.o);
-        az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
+        az0 = at(cb(S.psi[2]) + b2, q.o);
+        az1 = at(cb(S.psi[2]) + L2 + b2, q.o);
     }
 
     // ---- arithmetic
@@ -340,16 +332,16 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
         hy -= dby * pz1;
     }
     if (gx) {
-        put_s<NT>(mb(S.psi[0] + pw) + b0, q0, px0);
-        put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, px1);
+        put_s<NT>(mb(S.psi[0]) + b0, q0, px0);
+        put_s<NT>(mb(S.psi[0]) + L0 + b0, q0, px1);
     }
     if (gy) {
-        put_s<NT>(mb(S.psi[1] + pw) + b1, q1, py0);
-        put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, py1);
+        put_s<NT>(mb(S.psi[1]) + b1, q1, py0);
+        put_s<NT>(mb(S.psi[1]) + L1 + b1, q1, py1);
     }
     if (gz) {
-        put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, pz0);
-        put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, pz1);
+        put_s<NT>(mb(S.psi[2]) + b2, q.o, pz0);
+        put_s<NT>(mb(S.psi[2]) + L2 + b2, q.o, pz1);
     }
     const gmp Ho = mb(Hout) + kp;
     put_s<NT>(Ho, q.o, hx);
@@ -1238,8 +1230,6 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     const double mat = shell ? at(cb(S.eps) + kp, q.o) : at_s<NT>(cb(S.cbi) + kp, q.o);
     Quad X{0.0, 0.0, 0.0, 0.0}, Y = X, Z = X;
     int fl = 0;
-    const size_t pr = S.pstride ? (size_t)si * S.pstride : 0;
-    const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
     const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
     const size_t b0 = (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
     const size_t b1 = (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
@@ -1256,8 +1246,8 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
             fl &= *(const GLOBAL int *)(cb(S.fl[0]) + (unsigned)(ci * 4));
             if (in_face(ci, 2, nc - 1, S.ix - nc + 1, S.ix - 2)) {
                 q0 = (unsigned)(cj * (2 * nc) + slab_pos(ci, S.ix, nc)) * 8u;
-                ax0 = at(cb(S.psi[0] + pr) + b0, q0);
-                ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
+                ax0 = at(cb(S.psi[0]) + b0, q0);
+                ax1 = at(cb(S.psi[0]) + L0 + b0, q0);
             }
         } else {
             X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_E + 1);
@@ -1268,16 +1258,16 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
             fl &= *(const GLOBAL int *)(cb(S.fl[1]) + (unsigned)(cj * 4));
             if (in_face(cj, 2, nc, S.iy - nc + 1, S.iy - 2)) {
                 q1 = (unsigned)(slab_pos(cj, S.iy, nc) * S.ix + ci) * 8u;
-                ay0 = at(cb(S.psi[1] + pr) + b1, q1);
-                ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
+                ay0 = at(cb(S.psi[1]) + b1, q1);
+                ay1 = at(cb(S.psi[1]) + L1 + b1, q1);
             }
         } else {
             Y.k = uload(S.cq[1] + (size_t)T.y0 * CQ_N + CQ_E + 1);
             fl &= uload(S.fl[1] + T.y0);
         }
         if (in_face(k, 2, nc, S.iz - nc + 1, S.iz - 2)) {
-            az0 = at(cb(S.psi[2] + pr) + b2, q.o);
-            az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
+            az0 = at(cb(S.psi[2]) + b2, q.o);
+            az1 = at(cb(S.psi[2]) + L2 + b2, q.o);
         }
     } else {
         X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_E + 1);
@@ -1373,16 +1363,16 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
             ez -= amp;
     }
     if (ax && (fl & FL_PEX)) {
-        put_s<NT>(mb(S.psi[0] + pw) + b0, q0, ax0);
-        put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, ax1);
+        put_s<NT>(mb(S.psi[0]) + b0, q0, ax0);
+        put_s<NT>(mb(S.psi[0]) + L0 + b0, q0, ax1);
     }
     if (ay && (fl & FL_PEY)) {
-        put_s<NT>(mb(S.psi[1] + pw) + b1, q1, ay0);
-        put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, ay1);
+        put_s<NT>(mb(S.psi[1]) + b1, q1, ay0);
+        put_s<NT>(mb(S.psi[1]) + L1 + b1, q1, ay1);
     }
     if (az && (fl & FL_PEZ)) {
-        put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, az0);
-        put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, az1);
+        put_s<NT>(mb(S.psi[2]) + b2, q.o, az0);
+        put_s<NT>(mb(S.psi[2]) + L2 + b2, q.o, az1);
     }
     put_s<NT>(Eout, q.o, ex);
     put_s<NT>(Eout + nb, q.o, ey);
@@ -1432,8 +1422,6 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     Quad X{0.0, 0.0, 0.0, 0.0}, Y = X, Z = X;
     double mat = 1.0;
     int fl = 0;
-    const size_t pr = S.pstride ? (size_t)(so == 0 ? S.ring - 1 : so - 1) * S.pstride : 0;
-    const size_t pw = S.pstride ? (size_t)so * S.pstride : 0;
     const size_t L0 = (size_t)S.slab[0] * 8, L1 = (size_t)S.slab[1] * 8, L2 = (size_t)S.slab[2] * 8;
     const size_t b0 = 2 * L0 + (size_t)(unsigned)k * (unsigned)(S.iy * nc * 16);
     const size_t b1 = 2 * L1 + (size_t)(unsigned)k * (unsigned)(S.ix * nc * 16);
@@ -1451,8 +1439,8 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
             fl &= *(const GLOBAL int *)(cb(S.fl[0]) + (unsigned)(ci * 4));
             if (in_face(ci, 1, nc - 1, S.ix - nc, S.ix - 2)) {
                 q0 = (unsigned)(cj * (2 * nc) + slab_pos(ci, S.ix, nc)) * 8u;
-                ax0 = at(cb(S.psi[0] + pr) + b0, q0);
-                ax1 = at(cb(S.psi[0] + pr) + L0 + b0, q0);
+                ax0 = at(cb(S.psi[0]) + b0, q0);
+                ax1 = at(cb(S.psi[0]) + L0 + b0, q0);
             }
         } else {
             X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_H + 1);
@@ -1463,16 +1451,16 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
             fl &= *(const GLOBAL int *)(cb(S.fl[1]) + (unsigned)(cj * 4));
             if (in_face(cj, 1, nc - 1, S.iy - nc, S.iy - 2)) {
                 q1 = (unsigned)(slab_pos(cj, S.iy, nc) * S.ix + ci) * 8u;
-                ay0 = at(cb(S.psi[1] + pr) + b1, q1);
-                ay1 = at(cb(S.psi[1] + pr) + L1 + b1, q1);
+                ay0 = at(cb(S.psi[1]) + b1, q1);
+                ay1 = at(cb(S.psi[1]) + L1 + b1, q1);
             }
         } else {
             Y.k = uload(S.cq[1] + (size_t)T.y0 * CQ_N + CQ_H + 1);
             fl &= uload(S.fl[1] + T.y0);
         }
         if (in_face(k, 1, nc - 1, S.iz - nc, S.iz - 2)) {
-            az0 = at(cb(S.psi[2] + pr) + b2, q.o);
-            az1 = at(cb(S.psi[2] + pr) + L2 + b2, q.o);
+            az0 = at(cb(S.psi[2]) + b2, q.o);
+            az1 = at(cb(S.psi[2]) + L2 + b2, q.o);
         }
     } else {
         X.k = uload(S.cq[0] + (size_t)T.x0 * CQ_N + CQ_H + 1);
@@ -1560,16 +1548,16 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
             hy -= dby * az1;
         }
         if (ax && (fl & FL_PHX)) {
-            put_s<NT>(mb(S.psi[0] + pw) + b0, q0, ax0);
-            put_s<NT>(mb(S.psi[0] + pw) + L0 + b0, q0, ax1);
+            put_s<NT>(mb(S.psi[0]) + b0, q0, ax0);
+            put_s<NT>(mb(S.psi[0]) + L0 + b0, q0, ax1);
         }
         if (ay && (fl & FL_PHY)) {
-            put_s<NT>(mb(S.psi[1] + pw) + b1, q1, ay0);
-            put_s<NT>(mb(S.psi[1] + pw) + L1 + b1, q1, ay1);
+            put_s<NT>(mb(S.psi[1]) + b1, q1, ay0);
+            put_s<NT>(mb(S.psi[1]) + L1 + b1, q1, ay1);
         }
         if (az && (fl & FL_PHZ)) {
-            put_s<NT>(mb(S.psi[2] + pw) + b2, q.o, az0);
-            put_s<NT>(mb(S.psi[2] + pw) + L2 + b2, q.o, az1);
+            put_s<NT>(mb(S.psi[2]) + b2, q.o, az0);
+            put_s<NT>(mb(S.psi[2]) + L2 + b2, q.o, az1);
         }
     }
     const gmp Hout = mb(hsel(S, j + 1, hf)) + kp;

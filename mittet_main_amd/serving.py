@@ -191,31 +191,34 @@ def gradient_bytes(req: Request, budget: float):
 
 
 def _adjoint_tile_doubles(grid: Grid) -> int:
-    """Doubles held by the adjoint's per-cell tile list: 16-byte entries for
-    the 32 x 8 tiles (16 x 16 over the x edges) around its LDS region
-    [ncpml + 1, n - ncpml - 1) (x start rounded up to 8); none without that
-    region (kappa != 1, ncpml < 2, LDS kernels switched off)."""
+    """Doubles held by the adjoint's per-cell tile list: 16-byte entries, a
+    multiple of 8 per plane, for the 32 x 8 tiles (16 x 16 over the x edges)
+    around its LDS region [ncpml + 1, n - ncpml - 1) (x start rounded up to 8),
+    or all 32 x 8 tiles without that region (below 3 M cells, kappa != 1,
+    ncpml < 2, LDS kernels switched off); no list then below 0.5 M cells."""
     nc = grid.ncpml
     n = (grid.ix, grid.iy, grid.iz)
-    if nc < 2 or grid.kappa_max != 1.0 or int(os.environ.get("MITTET_FDTD_NOLDS", "0") or 0):
-        return 0
     lo = [(nc + 1 + 7) // 8 * 8, nc + 1, nc + 1]
     hi = [v - nc - 1 for v in n]
-    if any(a >= b for a, b in zip(lo, hi)):
-        return 0
+    if nc < 2 or grid.kappa_max != 1.0 or int(os.environ.get("MITTET_FDTD_NOLDS", "0") or 0) or \
+            not (grid.ncells >= 3_000_000 or int(os.environ.get("MITTET_FDTD_LDS", "0") or 0)) or \
+            any(a >= b for a, b in zip(lo, hi)):
+        if grid.ncells < 500_000:
+            return 0
+        lo = hi = [0, 0, 0]
     ftx, fty = -(-grid.ix // 32), -(-grid.iy // 8)
     ya, yb = -(-lo[1] // 8), hi[1] // 8
     inside = max(0, yb - ya)
     edge = -(-lo[0] // 16) + -(-(grid.ix - hi[0]) // 16)
     per_in = (fty - inside) * ftx + (-(-inside * 8 // 16) * edge if inside else 0)
-    count = (hi[2] - lo[2]) * per_in + (grid.iz - (hi[2] - lo[2])) * fty * ftx
-    return 2 * (-(-count // 8) * 8)
+    return 16 * ((hi[2] - lo[2]) * -(-per_in // 8) + (grid.iz - (hi[2] - lo[2])) * -(-fty * ftx // 8))
 
 
 def plan_bytes(grid: Grid, nt: int, nrec: int, levels: int) -> int:
     """Device bytes of a gradient's checkpoint storage (host-side mirror of
-    fwi3d_grad_plan_bytes: states of 6 fields + shell psi, each padded to
-    256 bytes, scratch, gradient, the adjoint's tile list)."""
+    fwi3d_grad_plan_bytes: states of 6 fields + shell psi and the replayed
+    segment's of 6 fields, each padded to 256 bytes, scratch, gradient, the
+    adjoint's tile list)."""
     import ctypes as C
     sl = (C.c_int * levels)()
     ns, st = C.c_int(0), C.c_longlong(0)
@@ -223,9 +226,10 @@ def plan_bytes(grid: Grid, nt: int, nrec: int, levels: int) -> int:
     n, nc = grid.ncells, grid.ncpml
     psi = 4 * 2 * nc * (grid.iy * grid.iz + grid.ix * grid.iz + grid.ix * grid.iy)
     state = 6 * n + psi
-    other = ((state - 3 * n) + n + 1 + max(1, 3 * nrec * (nt + 1)) +
+    leaf = sl[levels - 1] + 1
+    other = (12 * n + n + 1 + max(1, 3 * nrec * (nt + 1)) +
              2 * (grid.ix + grid.iy + grid.iz) + _adjoint_tile_doubles(grid))
-    return 8 * (st.value * ((state + 31) // 32 * 32) + other)
+    return 8 * ((st.value - leaf) * ((state + 31) // 32 * 32) + leaf * ((6 * n + 31) // 32 * 32) + other)
 
 
 def run_gradient(req: Request, budget: float) -> Result:
