@@ -74,8 +74,8 @@ struct alignas(64) ShotDev {
                               // a gradient replay's stored states), see hsel
     const int4 *shell;        // tiles of the per-cell kernels when the LDS kernels cover the
                               // interior: {x0, y0, k, yend} (yend 0: a 32 x 8 tile; else a
-                              // 16 x 16 tile with rows below yend), fb entries then k = -1
-                              // padding; null: every tw x th tile of every plane
+                              // 16 x 16 tile with rows below yend), fb entries, k = -1 in
+                              // those that hold none; null: every tile of every plane
     const double *eps;        // eps' = sigma/2/omega0 per cell
     const double *cbi;        // dt/eps' per cell (cb where the CPML sigma is zero)
     double *psi[3];           // [PSI_N][slab[a]]
@@ -100,7 +100,8 @@ struct alignas(64) ShotDev {
     int kb;                   // z-chunk length of the z-marching kernels
     int ztx, zty, nkz;        // z-marching tiles along x, y and z-chunks
     int zb, zb_pad;           // z-marching blocks, padded to a multiple of 8
-    int ftx, fty;             // 32 x 8 (pair: 32 x 16) tiles along x and y of the pair kernels
+    int ftx, fty;             // 32 x 8 tiles along x and y, of the per-cell tiles in layers
+                              // (pair kernels: 32 x 16)
     int pair;                 // 1: fused kernels update x-pairs of cells (even ix)
     int ltx, lty, lkz;        // LDS-kernel tiles along x, y and z-chunks
     int lkb;                  // LDS-kernel z-chunk length (planes)
