@@ -63,20 +63,24 @@ __device__ __forceinline__ bool in_region(const AdjArgs &A, int i, int j, int k)
 
 }  // namespace
 
-// adjoint receiver source: lE[comp][rec] += g[comp][rec] (state after step n);
-// receivers on one cell add up
+// adjoint receiver source: lE[comp][rec] += g[comp][rec] (state after step n).  At most
+// one receiver of a cell has a sensitivity that is not zero (the host sums those on one
+// cell), and only that lane touches the cell: each lane loads, adds and stores by itself.
 __global__ void k_adj_inject(AdjArgs A, const double *__restrict__ g, int nrec,
                              const int *__restrict__ rec)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= 3 * nrec)
         return;
+    const double gq = g[q];
+    if (gq == 0.0)
+        return;
     const int comp = q / nrec, r = q - comp * nrec, c = rec[r];
     const int i = c % A.ix, t = c / A.ix, j = t % A.iy, k = t / A.iy;
     if (in_region(A, i, j, k))
-        A.lE[(size_t)comp * A.n + c] += A.cbi[c] * g[q];
+        A.lE[(size_t)comp * A.n + c] += A.cbi[c] * gq;
     else
-        A.lE[(size_t)comp * A.n + c] += g[q];
+        A.lE[(size_t)comp * A.n + c] += gq;
 }
 
 // Per-cell pass over the tiles outside the LDS region (every tile without one).

@@ -2641,6 +2641,18 @@ static int adj_range(fwi3d_grad *g, int depth, int n0, int L, double *start, mt:
     return FWI3D_OK;
 }
 
+// for each receiver the first one on its cell
+static std::vector<int> first_on_cell(const std::vector<int> &cell)
+{
+    std::vector<int> order(cell.size()), first(cell.size());
+    for (size_t r = 0; r < order.size(); ++r)
+        order[r] = (int)r;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cell[a] < cell[b]; });
+    for (size_t q = 0; q < order.size(); ++q)
+        first[order[q]] = q && cell[order[q]] == cell[order[q - 1]] ? first[order[q - 1]] : order[q];
+    return first;
+}
+
 int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
 {
     if (!g || !djdt || !djds)
@@ -2652,12 +2664,14 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
         return rc;
     const int nrec = s->nrec, it = s->it;
     const size_t N = (size_t)s->desc.n;
-    // sensitivities regrouped per step: g[n][comp][rec]
+    // sensitivities regrouped per step: g[n][comp][rec]; those of receivers on one cell
+    // are summed at the first of them, in receiver order, and zero at the others
+    const std::vector<int> first = first_on_cell(s->rec);
     std::vector<double> gt(std::max<size_t>(1, 3 * (size_t)nrec * it));
     for (int c = 0; c < 3; ++c)
         for (int r = 0; r < nrec; ++r)
             for (int n = 0; n < it; ++n)
-                gt[((size_t)n * 3 + c) * nrec + r] = djdt[((size_t)c * nrec + r) * it + n];
+                gt[((size_t)n * 3 + c) * nrec + first[r]] += djdt[((size_t)c * nrec + r) * it + n];
     HIP_TRY(hipMemcpyAsync(g->g, gt.data(), sizeof(double) * gt.size(), hipMemcpyHostToDevice, s->st));
     HIP_TRY(mt::launch_fill(g->adj, g->state, 0.0, s->st));
     HIP_TRY(mt::launch_fill(g->tmp, 6 * N, 0.0, s->st));   // uh
