@@ -626,8 +626,32 @@ __global__ __launch_bounds__(ANT) void k_adj_el(AdjArgs A)
     }
 }
 
+// rim weights of the H update from the region's lH: they do not outlive a replayed
+// segment in uh
+__global__ __launch_bounds__(256) void k_adj_rim(AdjArgs A)
+{
+    const unsigned w = (unsigned)(A.hi[0] - A.lo[0]), h = (unsigned)(A.hi[1] - A.lo[1]);
+    const unsigned q = blockIdx.x * 256u + threadIdx.x, t = q / w;
+    const int i = A.lo[0] + (int)(q - t * w), j = A.lo[1] + (int)(t % h), k = A.lo[2] + (int)(t / h);
+    if (k >= A.hi[2])
+        return;
+    const bool inner = i >= A.lo[0] + 2 && i < A.hi[0] - 2 && j >= A.lo[1] + 2 && j < A.hi[1] - 2 &&
+                       k >= A.lo[2] + 2 && k < A.hi[2] - 2;
+    if (inner)
+        return;
+    const size_t nb = (size_t)A.n * 8;
+    const gcp lH = cb(A.lH) + (size_t)k * A.pb;
+    const unsigned o = (unsigned)j * A.row + (unsigned)i * 8u;
+    rim(A, A.uh, i, j, k, o, at(lH, o), at(lH + nb, o), at(lH + 2 * nb, o));
+}
+
 hipError_t launch_adjoint_local(const AdjArgs &A, hipStream_t st)
 {
+    if (A.lb_pad > 0) {
+        const unsigned cells = (unsigned)(A.hi[0] - A.lo[0]) * (unsigned)(A.hi[1] - A.lo[1]) *
+                               (unsigned)(A.hi[2] - A.lo[2]);
+        hipLaunchKernelGGL(k_adj_rim, dim3((cells + 255) / 256), dim3(256), 0, st, A);
+    }
     hipLaunchKernelGGL(k_adj_cell<true>, dim3(A.fb_pad), dim3(PT), 0, st, A, 0, 1);
     return hipGetLastError();
 }

@@ -2211,9 +2211,8 @@ struct fwi3d_grad {
     size_t off_h = 0, off_psi[3] = {0, 0, 0};
     double *ckpt = nullptr;           // nseg states
     std::vector<double *> inner;      // depth l >= 1: slots for the starts of a segment's pieces
-    double *buf = nullptr;            // leaf + 1 states of a replayed segment
+    double *buf = nullptr;            // leaf + 1 states of a replayed segment, then 3N (see adj_range)
     double *adj = nullptr;            // adjoint state (one state)
-    double *tmp = nullptr;            // weights of the per-cell passes (2 x 6N)
     double *grad = nullptr;           // N
     double *grad_src = nullptr;       // 1
     double *g = nullptr;              // [it][3][nrec] trace sensitivities
@@ -2268,6 +2267,30 @@ static mt::StateSegs state_segs(const fwi3d_grad *g)
     return v;
 }
 
+// the segments [first, last) of it, stored from the offset of `first` on
+static mt::StateSegs state_segs(const fwi3d_grad *g, int first, int last)
+{
+    const mt::StateSegs all = state_segs(g);
+    mt::StateSegs v{};
+    for (int k = first; k < last; ++k) {
+        v.live[k - first] = all.live[k];
+        v.count[k - first] = all.count[k];
+    }
+    v.nseg = last - first;
+    return v;
+}
+
+// copy E and H of one stored state to another
+static int state_move(const fwi3d_grad *g, double *from, double *to)
+{
+    mt::StateSegs v{};
+    v.live[0] = from;
+    v.count[0] = g->off_psi[0];
+    v.nseg = 1;
+    HIP_TRY(mt::launch_state_copy(v, to, true, g->s->st));
+    return FWI3D_OK;
+}
+
 // copy the shot's live state to / from a stored state (one launch)
 static int state_copy(fwi3d_grad *g, double *dst_state, bool save)
 {
@@ -2280,6 +2303,22 @@ static int set_step(fwi3d_shot *s, int n)
     HIP_TRY(hipMemcpyAsync(s->d_step, &n, sizeof(int), hipMemcpyHostToDevice, s->st));
     HIP_TRY(hipStreamSynchronize(s->st));
     s->step = n;
+    return FWI3D_OK;
+}
+
+// whether a replay keeps H in a ring over the stored states too
+static bool replay_hring(const Fam &f) { return (f.kind == 0 || f.kind == 3) && !f.fused; }
+
+// The state at the start of a segment into buffer slot 0 (E and H) and the shot
+// (psi, and where the replay updates H in place E and H too)
+static int replay_start(fwi3d_grad *g, double *start)
+{
+    mt::StateSegs v = state_segs(g);
+    v.live[0] = g->buf;
+    v.live[1] = g->buf + g->off_h;
+    HIP_TRY(mt::launch_state_copy(v, start, false, g->s->st));
+    if (!replay_hring(shot_fam(g->s)))
+        HIP_TRY(mt::launch_state_copy(state_segs(g, 0, 2), start, false, g->s->st));
     return FWI3D_OK;
 }
 
@@ -2305,7 +2344,7 @@ static int replay_segment(fwi3d_grad *g, int L)
         g->replay[slot] = nullptr;
     }
     const Fam f0 = shot_fam(s);
-    const bool hring = (f0.kind == 0 || f0.kind == 3) && !f0.fused;
+    const bool hring = replay_hring(f0);
     g->rdesc = s->desc;
     g->rdesc.e = g->buf;
     g->rdesc.sstride = (long long)g->lstate;
@@ -2326,10 +2365,7 @@ static int replay_segment(fwi3d_grad *g, int L)
         f.nblocks = cell_blocks(s, f.nt);
         f.nblocks_l = lds_blocks(s, f.nt, f.fused);
         const bool fold = s->nrec && rec_folds(f);
-        mt::StateSegs segs{};   // H, without the ring
-        segs.live[0] = state_segs(g).live[1];
-        segs.count[0] = state_segs(g).count[1];
-        segs.nseg = 1;
+        const mt::StateSegs segs = state_segs(g, 1, 2);   // H, without the ring
         hipGraph_t graph = nullptr;
         std::lock_guard<std::recursive_mutex> lk(g_rt_mu);
         HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
@@ -2359,9 +2395,8 @@ static int replay_segment(fwi3d_grad *g, int L)
         g->replay_len[slot] = L;
     }
     HIP_TRY(hipGraphLaunch(g->replay[slot], s->st));
-    mt::StateSegs back = state_segs(g);   // E, with the ring H too
-    back.nseg = hring ? 2 : 1;
-    HIP_TRY(mt::launch_state_copy(back, g->buf + g->lstate * L, false, s->st));
+    // E, with the ring H too
+    HIP_TRY(mt::launch_state_copy(state_segs(g, 0, hring ? 2 : 1), g->buf + g->lstate * L, false, s->st));
     s->step += L;
     return FWI3D_OK;
 }
@@ -2432,14 +2467,14 @@ static std::vector<int4> adj_tiles(const fwi3d_shot *s)
     return complement_tiles(s->desc.ix, s->desc.iy, s->desc.iz, lo, hi);
 }
 
-// device bytes a gradient with this plan allocates (states, scratch, gradient,
-// trace sensitivities, profile reciprocals, per-cell tile list; the replay's
-// copy of the shot descriptor, under 1 KB, is not counted)
+// device bytes a gradient with this plan allocates (states, 3 values per cell
+// behind the replayed ones, gradient, trace sensitivities, profile reciprocals,
+// per-cell tile list; the replay's copy of the shot descriptor, under 1 KB, is
+// not counted)
 static long long grad_plan_bytes(const fwi3d_shot *s, const GradPlan &P)
 {
     const size_t N = (size_t)s->desc.n, st = state_doubles(s);
-    const size_t tmp = 12 * N;
-    const size_t other = tmp + N + 1 + std::max<size_t>(1, 3 * (size_t)s->nrec * s->it) +
+    const size_t other = 3 * N + N + 1 + std::max<size_t>(1, 3 * (size_t)s->nrec * s->it) +
                          2 * ((size_t)s->desc.ix + s->desc.iy + s->desc.iz) +
                          2 * adj_tiles(s).size();
     const size_t leaf = (size_t)P.seglen.back() + 1;   // states of a replayed segment: E and H
@@ -2469,7 +2504,6 @@ static int grad_new(fwi3d_shot *s, int levels, int segment, fwi3d_grad **out)
     g->leaf = g->plan.seglen[levels - 1];
     state_layout(g);
     const size_t N = (size_t)s->desc.n;
-    const size_t tmp = 12 * N;
     bool ok = dalloc(&g->ckpt, g->state * g->nseg) == hipSuccess;
     for (int l = 1; l < levels && ok; ++l) {
         const size_t pieces =
@@ -2478,8 +2512,8 @@ static int grad_new(fwi3d_shot *s, int levels, int segment, fwi3d_grad **out)
         ok = dalloc(&p, g->state * pieces) == hipSuccess;
         g->inner.push_back(p);
     }
-    if (!ok || dalloc(&g->buf, g->lstate * (g->leaf + 1)) != hipSuccess ||
-        dalloc(&g->adj, g->state) != hipSuccess || dalloc(&g->tmp, tmp) != hipSuccess ||
+    if (!ok || dalloc(&g->buf, g->lstate * (g->leaf + 1) + 3 * N) != hipSuccess ||
+        dalloc(&g->adj, g->state) != hipSuccess ||
         dalloc(&g->grad, N) != hipSuccess || dalloc(&g->grad_src, 1) != hipSuccess ||
         dalloc(&g->g, std::max<size_t>(1, 3 * (size_t)s->nrec * s->it)) != hipSuccess ||
         dalloc(&g->rp, 2 * ((size_t)s->desc.ix + s->desc.iy + s->desc.iz)) != hipSuccess ||
@@ -2553,7 +2587,6 @@ int fwi3d_grad_destroy(fwi3d_grad *g)
         dfree(p);
     dfree(g->buf);
     dfree(g->adj);
-    dfree(g->tmp);
     dfree(g->grad);
     dfree(g->grad_src);
     dfree(g->g);
@@ -2592,26 +2625,30 @@ int fwi3d_grad_forward(fwi3d_grad *g)
 
 // Adjoint steps over [n0, n0 + L) in reverse, at recursion depth `depth` of
 // the checkpoint plan; the stored state `start` is the forward state at n0.
+//
+// The per-cell passes' weights (12 values per cell) live in states that are idle
+// while a segment's adjoint steps run.  uh: H of the segment's last state, which only
+// the H local part of its last step reads (each cell its own values before it writes
+// its weights), and the 3N values behind it, the next slot or the end of buf.  ue: E
+// and H of the start, of which slot 0 is a copy.  At depth 0 a second backward sweep
+// needs the start again, so it gets E and H back from there.
 static int adj_range(fwi3d_grad *g, int depth, int n0, int L, double *start, mt::AdjArgs &A,
                      const std::vector<double> &amp)
 {
     fwi3d_shot *s = g->s;
     const int nrec = s->nrec;
     int rc;
-    if ((rc = state_copy(g, start, false)) || (rc = set_step(s, n0)))
-        return rc;
     if (depth == g->plan.levels - 1) {
         // replay the segment keeping every state, then step the adjoint back
-        mt::StateSegs eh = state_segs(g);
-        eh.nseg = 2;
-        HIP_TRY(mt::launch_state_copy(eh, g->buf, true, s->st));
-        if ((rc = replay_segment(g, L)))
+        if ((rc = replay_start(g, start)) || (rc = set_step(s, n0)) || (rc = replay_segment(g, L)))
             return rc;
         // the H local part of step t runs with step t + 1 (both states at hand),
         // that of the segment's last step on its own
         auto state = [&](int t) { return g->buf + g->lstate * t; };
         A.H0 = state(L - 1) + g->off_h;
         A.H1 = state(L) + g->off_h;
+        A.uh = state(L) + g->off_h;
+        A.ue = start;
         HIP_TRY(mt::launch_adjoint_local(A, s->st));
         for (int t = L - 1; t >= 0; --t) {
             const int n = n0 + t;
@@ -2622,8 +2659,10 @@ static int adj_range(fwi3d_grad *g, int depth, int n0, int L, double *start, mt:
             A.amp_n = amp[n];
             HIP_TRY(mt::launch_adjoint_step(A, g->g + (size_t)n * 3 * nrec, nrec, s->d_rec, t > 0, s->st));
         }
-        return FWI3D_OK;
+        return depth == 0 ? state_move(g, state(0), start) : FWI3D_OK;
     }
+    if ((rc = state_copy(g, start, false)) || (rc = set_step(s, n0)))
+        return rc;
     // one forward pass over the segment storing the start of each piece
     const int P = g->plan.seglen[depth + 1];
     const int np = (L + P - 1) / P;
@@ -2674,7 +2713,6 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
                 gt[((size_t)n * 3 + c) * nrec + first[r]] += djdt[((size_t)c * nrec + r) * it + n];
     HIP_TRY(hipMemcpyAsync(g->g, gt.data(), sizeof(double) * gt.size(), hipMemcpyHostToDevice, s->st));
     HIP_TRY(mt::launch_fill(g->adj, g->state, 0.0, s->st));
-    HIP_TRY(mt::launch_fill(g->tmp, 6 * N, 0.0, s->st));   // uh
     HIP_TRY(mt::launch_fill(g->grad, N, 0.0, s->st));
     HIP_TRY(mt::launch_fill(g->grad_src, 1, 0.0, s->st));
     std::vector<double> amp(it, 0.0);
@@ -2741,8 +2779,6 @@ int fwi3d_grad_backward(fwi3d_grad *g, const double *djdt, double *djds)
     A.cbi = d.cbi;
     A.lE = g->adj;
     A.lH = g->adj + g->off_h;
-    A.uh = g->tmp;
-    A.ue = g->tmp + 6 * N;
     A.grad = g->grad;
     A.grad_src = g->grad_src;
     A.src_cell = s->src_cell;

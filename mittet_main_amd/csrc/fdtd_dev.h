@@ -182,8 +182,9 @@ struct AdjArgs {
 };
 
 // One adjoint step but for the cell-local H part of its own step, which
-// launch_adjoint_local has done (first step of a replayed segment) or the step
-// before (next_local: this one does that of the next, with H0 and H1 its H).
+// launch_adjoint_local has done (first step of a replayed segment, with the region's
+// rim weights in uh) or the step before (next_local: this one does that of the next,
+// with H0 and H1 its H).
 hipError_t launch_adjoint_local(const AdjArgs &A, hipStream_t st);
 hipError_t launch_adjoint_step(const AdjArgs &A, const double *g, int nrec, const int *rec,
                                bool next_local, hipStream_t st);

@@ -217,8 +217,8 @@ def _adjoint_tile_doubles(grid: Grid) -> int:
 def plan_bytes(grid: Grid, nt: int, nrec: int, levels: int) -> int:
     """Device bytes of a gradient's checkpoint storage (host-side mirror of
     fwi3d_grad_plan_bytes: states of 6 fields + shell psi and the replayed
-    segment's of 6 fields, each padded to 256 bytes, scratch, gradient, the
-    adjoint's tile list)."""
+    segment's of 6 fields, each padded to 256 bytes, 3 values per cell behind
+    them, gradient, the adjoint's tile list)."""
     import ctypes as C
     sl = (C.c_int * levels)()
     ns, st = C.c_int(0), C.c_longlong(0)
@@ -227,7 +227,7 @@ def plan_bytes(grid: Grid, nt: int, nrec: int, levels: int) -> int:
     psi = 4 * 2 * nc * (grid.iy * grid.iz + grid.ix * grid.iz + grid.ix * grid.iy)
     state = 6 * n + psi
     leaf = sl[levels - 1] + 1
-    other = (12 * n + n + 1 + max(1, 3 * nrec * (nt + 1)) +
+    other = (3 * n + n + 1 + max(1, 3 * nrec * (nt + 1)) +
              2 * (grid.ix + grid.iy + grid.iz) + _adjoint_tile_doubles(grid))
     return 8 * ((st.value - leaf) * ((state + 31) // 32 * 32) + leaf * ((6 * n + 31) // 32 * 32) + other)
 
