@@ -439,6 +439,9 @@ std::vector<int4> complement_tiles(int ix, int iy, int iz, const int lo[3], cons
     std::vector<int4> shell;
     const int ftx = tiles(ix, mt::ZX), fty = tiles(iy, mt::ZY);
     const int ya = tiles(lo[1], mt::ZY), yb = hi[1] / mt::ZY;   // tile rows inside [lo_y, hi_y)
+    // where the second x-edge segment starts: a tile of the first one reaches past hi_x in
+    // a narrow region that starts inside it, and no cell may be in two tiles
+    const int x1 = std::max(hi[0], tiles(lo[0], 16) * 16);
     std::vector<int4> plane;
     auto deal = [&](int k) {
         const int P = (int)plane.size(), e = tiles(P, 8);
@@ -460,7 +463,7 @@ std::vector<int4> complement_tiles(int ix, int iy, int iz, const int lo[3], cons
         for (int y0 = ya * mt::ZY; inz && y0 < yend; y0 += 16) {
             for (int x0 = 0; x0 < lo[0]; x0 += 16)
                 plane.push_back(int4{x0, y0, k, yend});
-            for (int x0 = hi[0]; x0 < ix; x0 += 16)
+            for (int x0 = x1; x0 < ix; x0 += 16)
                 plane.push_back(int4{x0, y0, k, yend});
         }
         deal(k);

@@ -209,7 +209,8 @@ def _adjoint_tile_doubles(grid: Grid) -> int:
     ftx, fty = -(-grid.ix // 32), -(-grid.iy // 8)
     ya, yb = -(-lo[1] // 8), hi[1] // 8
     inside = max(0, yb - ya)
-    edge = -(-lo[0] // 16) + -(-(grid.ix - hi[0]) // 16)
+    edge = -(-lo[0] // 16)
+    edge += -(-(grid.ix - max(hi[0], 16 * edge)) // 16)
     per_in = (fty - inside) * ftx + (-(-inside * 8 // 16) * edge if inside else 0)
     return 16 * ((hi[2] - lo[2]) * -(-per_in // 8) + (grid.iz - (hi[2] - lo[2])) * -(-fty * ftx // 8))
 
