@@ -617,6 +617,7 @@ struct fwi3d_batch {
     int *d_pre = nullptr, *d_pre_l = nullptr, *d_pre_cells = nullptr;
     int nblocks = 0, nblocks_l = 0, ncellblocks = 0;
     bool rings = false, fused = false, nt = false;   // the members' Fam
+    std::vector<char> done;   // members that had finished at the last upload: they get no blocks
     int kind = 0;         // fused kernel family of the members (all equal)
     bool dirty = true;
     hipGraphExec_t graph = nullptr;
@@ -3239,6 +3240,17 @@ int fwi3d_batch_remove(fwi3d_batch *b, fwi3d_shot *s)
 
 int fwi3d_batch_size(const fwi3d_batch *b) { return b ? (int)b->shots.size() : -1; }
 
+static bool finished(const fwi3d_shot *s) { return s->step >= s->it - 1; }
+
+// whether a member has finished since the last upload
+static bool batch_changed(const fwi3d_batch *b)
+{
+    for (size_t q = 0; q < b->shots.size(); ++q)
+        if (finished(b->shots[q]) != (bool)b->done[q])
+            return true;
+    return false;
+}
+
 static int batch_upload(fwi3d_batch *b)
 {
     const int ns = (int)b->shots.size();
@@ -3253,12 +3265,14 @@ static int batch_upload(fwi3d_batch *b)
         touch += step_touch_bytes(s);
     }
     b->nt = stream_nt(touch);
+    b->done.assign(ns, 0);
     for (int q = 0; q < ns; ++q) {
         const fwi3d_shot *s = b->shots[q];
         descs[q] = s->desc;
-        pre[q + 1] = pre[q] + cell_blocks(s, b->nt);
-        prel[q + 1] = prel[q] + lds_blocks(s, b->nt, b->fused);
-        prec[q + 1] = prec[q] + b->shots[q]->ncellblocks;
+        b->done[q] = finished(s);
+        pre[q + 1] = pre[q] + (b->done[q] ? 0 : cell_blocks(s, b->nt));
+        prel[q + 1] = prel[q] + (b->done[q] ? 0 : lds_blocks(s, b->nt, b->fused));
+        prec[q + 1] = prec[q] + (b->done[q] ? 0 : s->ncellblocks);
     }
     b->nblocks = pre[ns];
     b->nblocks_l = prel[ns];
@@ -3307,6 +3321,8 @@ int fwi3d_batch_step(fwi3d_batch *b, int nsteps)
     }
     while (left > 0) {
         const int L = std::min(b->chunk, left);
+        if (batch_changed(b) && (rc = batch_upload(b)))
+            return rc;
         if (L == b->chunk) {
             if (!b->graph && (rc = capture_chunk(&b->graph, b->d_desc, ns, batch_fam(b),
                                                  b->d_pre_cells, b->ncellblocks, L, dft, rec,

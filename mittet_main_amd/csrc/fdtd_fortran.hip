@@ -113,6 +113,8 @@ __global__ __launch_bounds__(PT) void k_efield_v(const ShotDev *__restrict__ D, 
     FTile T;
     if (!ftile<false>(S, ns > 1 ? b - pre[s] : b, T))
         return;   // uniform over the block
+    if (ns > 1 && chunk_step(S) + j >= S.it - 1)
+        return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc, ix = S.ix, iy = S.iy, iz = S.iz;
     const bool ax = T.x0 < nc || T.x0 + T.w > ix - nc, ay = T.y0 < nc || T.y0 + T.h > iy - nc;
     const bool az = k < nc || k >= iz - nc, shell = ax || ay || az;
@@ -270,6 +272,8 @@ __global__ __launch_bounds__(PT) void k_hfield_v(const ShotDev *__restrict__ D, 
     FTile T;
     if (!ftile<false>(S, ns > 1 ? b - pre[s] : b, T))
         return;   // uniform over the block
+    if (ns > 1 && chunk_step(S) + j >= S.it - 1)
+        return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc, ix = S.ix, iy = S.iy, iz = S.iz;
     const bool ax = T.x0 < nc || T.x0 + T.w > ix - nc, ay = T.y0 < nc || T.y0 + T.h > iy - nc;
     const bool az = k < nc || k >= iz - nc, shell = ax || ay || az;

@@ -1207,6 +1207,8 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     FTile T;
     if (!ftile<NT>(S, ns > 1 ? b - pre[s] : b, T))
         return;   // uniform over the block
+    if (ns > 1 && chunk_step(S) + j >= S.it - 1)
+        return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
     const bool az = k < nc || k >= S.iz - nc;
@@ -1281,8 +1283,8 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     if (q.halo)
         lds_put(sh, q.ha + (unsigned)hc * (PT_TILE * 8u), hv);
     __syncthreads();
-    // the step is looked up behind the loads (it costs two dependent scalar
-    // loads): a shot that has finished its time loop stores nothing
+    // a lone shot's step is looked up behind the loads (it costs two dependent
+    // scalar loads), only for the source: its launches end with its time loop
     const int n = chunk_step(S) + j;
     if (n >= S.it - 1 || !q.own || q.i >= S.ix || q.jj >= T.yend)
         return;
@@ -1399,6 +1401,8 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     FTile T;
     if (!ftile<NT>(S, ns > 1 ? b - pre[s] : b, T))
         return;   // uniform over the block
+    if (ns > 1 && chunk_step(S) + j >= S.it - 1)
+        return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
     const bool az = k < nc || k >= S.iz - nc;
@@ -1474,8 +1478,8 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     if (q.halo)
         lds_put(sh, q.ha + (unsigned)hc * (PT_TILE * 8u), hv);
     __syncthreads();
-    // the step is looked up behind the loads (it costs two dependent scalar
-    // loads): a shot that has finished its time loop stores nothing
+    // a lone shot's step is looked up behind the loads: its launches end with its
+    // time loop
     const int n = chunk_step(S) + j;
     if (n >= S.it - 1 || !q.own || q.i >= S.ix || q.jj >= T.yend)
         return;
