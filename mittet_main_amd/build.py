@@ -17,7 +17,7 @@ SOURCES = [os.path.join(HERE, "csrc", f)
            for f in ("fdtd_kernels.hip", "fdtd_adjoint.hip", "fdtd_compat.hip", "fdtd_transform.hip",
                      "fdtd_fortran.hip", "fdtd_api.hip")]
 HEADERS = [os.path.join(HERE, "csrc", "fdtd_dev.h"), os.path.join(HERE, "csrc", "fdtd_tile.h"),
-           os.path.join(HERE, "csrc", "fdtd_transform.h"),
+           os.path.join(HERE, "csrc", "fdtd_transform.h"), os.path.join(HERE, "csrc", "host_threads.h"),
            os.path.join(ROOT, "include", "mittet_fdtd.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

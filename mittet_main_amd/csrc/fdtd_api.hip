@@ -13,13 +13,12 @@
 #include <cstring>
 #include <string>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "../../include/mittet_fdtd.h"
 #include "fdtd_dev.h"
 #include "fdtd_transform.h"
+#include "host_threads.h"
 
 using mt::ShotDev;
 
@@ -180,19 +179,7 @@ hipError_t read_back(Staging &sg, void *dst, const void *src, size_t width, size
             (void)hipEventDestroy(ev);
         err[t] = q;
     };
-    std::thread th[kStageThreads];
-    int t0 = 1;
-    for (; t0 < kStageThreads; ++t0)
-        try {
-            th[t0] = std::thread(work, t0);
-        } catch (const std::system_error &) {
-            break;   // no thread to be had: this one does the rest
-        }
-    work(0);
-    for (int t = t0; t < kStageThreads; ++t)
-        work(t);
-    for (int t = 1; t < t0; ++t)
-        th[t].join();
+    mt::on_threads<kStageThreads>(kStageThreads, work);
     // a failed piece may have left its copy into the staging memory under way
     e = hipStreamSynchronize(st);
     for (hipError_t q : err)
