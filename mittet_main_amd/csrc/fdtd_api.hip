@@ -138,7 +138,8 @@ hipError_t read_back(Staging &sg, void *dst, const void *src, size_t width, size
         hipError_t e = hipMemcpy2DAsync(dst, width, src, pitch, width, rows, hipMemcpyDeviceToHost, st);
         return e != hipSuccess ? e : hipStreamSynchronize(st);
     };
-    if (width * rows < kStageMin)
+    // (the per-thread stream's handle names another stream in each of the threads)
+    if (width * rows < kStageMin || st == hipStreamPerThread)
         return direct();
     // memory that the runtime knows (pinned, device, managed) needs no staging
     hipPointerAttribute_t at{};
@@ -153,8 +154,11 @@ hipError_t read_back(Staging &sg, void *dst, const void *src, size_t width, size
     const size_t piece = std::min(kStagePiece, (width * rows / 64 + 65535) & ~(size_t)65535);
     if (!sg.grow(kStageThreads * piece))
         return direct();
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    // the threads work on the stream's device, which need not be the caller's current one
+    int dev = 0, cur = 0;
+    hipError_t e = hipStreamGetDevice(st, &dev);
+    if (e == hipSuccess)
+        e = hipGetDevice(&cur);
     if (e != hipSuccess)
         return e;
     const size_t per = (width + piece - 1) / piece, pieces = per * rows;
@@ -180,6 +184,8 @@ hipError_t read_back(Staging &sg, void *dst, const void *src, size_t width, size
         err[t] = q;
     };
     mt::on_threads<kStageThreads>(kStageThreads, work);
+    if (cur != dev)
+        (void)hipSetDevice(cur);
     // a failed piece may have left its copy into the staging memory under way
     e = hipStreamSynchronize(st);
     for (hipError_t q : err)
