@@ -1,7 +1,8 @@
-"""Tiles of the per-cell forward kernels: every tile shape the host picks (16
-to 38 columns), rows and columns cut by the grid's edges, planes of less than
-one tile, and the thinnest CPML, against the oracle bit for bit: all six fields
-and the traces, in place and with E in ring slots, per operator and fused."""
+"""Tiles of the per-cell forward kernels: rows and columns cut by the grid's
+edges, planes of less than one tile, and the thinnest CPML, against the oracle
+bit for bit: all six fields and the traces, in place and with E in ring slots,
+per operator and fused (with the LDS family over the interior where it has one;
+the per-cell kernels alone: test_gpu_tile_shapes.py)."""
 import numpy as np
 import pytest
 
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 OM0 = 2 * np.pi
 # ix, iy, iz, ncpml: a plane below one tile; one cell more or less than a
-# tile's columns or rows; sizes with tiles of 16, 21, 28, 32, 36 columns
+# tile's columns or rows
 GRIDS = [(8, 8, 8, 2), (9, 31, 8, 2), (17, 13, 9, 2), (21, 12, 11, 3), (22, 37, 13, 3),
          (33, 24, 14, 5), (43, 25, 12, 4), (71, 20, 15, 5), (96, 19, 12, 4), (131, 11, 12, 3)]
 
