@@ -370,8 +370,6 @@ int axis_flags(int a, int r, int n, int nc)
         if (own ? (r >= 1 && r < nc - 1) || (r >= n - nc && r < n - 2) : r < n - 1)
             f |= mt::FL_PHX << d;
     }
-    if (r >= nc && r < n - nc)
-        f |= mt::FL_IN;
     return f;
 }
 

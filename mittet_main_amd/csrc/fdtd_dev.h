@@ -20,8 +20,7 @@ enum {
     FL_UEX = 1, FL_UEY = 2, FL_UEZ = 4,          // E updates
     FL_PEX = 8, FL_PEY = 16, FL_PEZ = 32,        // CPML-E faces of the x, y, z axis
     FL_UHX = 64, FL_UHY = 128, FL_UHZ = 256,     // H updates
-    FL_PHX = 512, FL_PHY = 1024, FL_PHZ = 2048,  // CPML-H faces
-    FL_IN = 4096                                 // outside every CPML shell
+    FL_PHX = 512, FL_PHY = 1024, FL_PHZ = 2048   // CPML-H faces
 };
 
 // psi arrays per axis: slab arrays of [0,nc) U [n-nc,n) along the axis.
@@ -126,8 +125,7 @@ struct alignas(64) ShotDev {
     const double *mu;         // variant 1: per-cell permeability
 };
 
-// M_NT: once-touched field values are loaded and stored non-temporally
-enum { M_UPD = 1, M_PSI = 2, M_SRC = 4, M_INPLACE = 8, M_NT = 16 };
+enum { M_UPD = 1, M_PSI = 2, M_SRC = 4, M_INPLACE = 8 };
 
 // H before local step j of a chunk.  In a launch sequence that updates H in
 // place (hf = 0) that is always the current buffer.  The fused E+H launches
@@ -203,7 +201,7 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // they gather E of step j itself (shots that update E in place).
 // hf: part of a fused E+H step (H read from hsel(S, j, 1), written to
 // hsel(S, j + 1, 1)); 0: H updated in place.  nt (also for the _l launches):
-// the once-touched field values go non-temporal (M_NT).
+// the once-touched field values go non-temporal (ld_s, st_s).
 hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks, int j,
                            hipStream_t st, bool rec_prev = false, bool rec_e = true, int hf = 0,
                            bool nt = false);
@@ -244,8 +242,6 @@ hipError_t launch_receiver_dft(const double *traces, int ncomp_rows, int it, dou
                                double *out, hipStream_t st);
 // bins k0 .. k0 + nbins - 1 of sum_n x[n] exp(2 pi i n k / it), complex
 hipError_t launch_bin_dft(const double *x, int it, int k0, int nbins, double *out, hipStream_t st);
-hipError_t launch_bin_dft(const double *traces, int nrows, int it, double dt, double omega0,
-                          int nbins, double *out, hipStream_t st);
 hipError_t launch_fill(double *p, size_t count, double v, hipStream_t st);
 hipError_t launch_copy(const double *src, double *dst, size_t count, hipStream_t st);
 // one launch that gathers up to 5 segments into a contiguous buffer (save) or

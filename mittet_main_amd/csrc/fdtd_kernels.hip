@@ -78,7 +78,7 @@ template <int MODE>
 __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, int i, int jj, int k,
                                             unsigned oc, int fl, int n, int si, int so, int sign)
 {
-    constexpr bool NT = (MODE & M_NT) != 0, UPD = (MODE & M_UPD) != 0, PSI = (MODE & M_PSI) != 0;
+    constexpr bool UPD = (MODE & M_UPD) != 0, PSI = (MODE & M_PSI) != 0;
     const bool upx = UPD && (fl & FL_UEX), upy = UPD && (fl & FL_UEY), upz = UPD && (fl & FL_UEZ);
     const bool fx = PSI && (fl & FL_PEX), fy = PSI && (fl & FL_PEY), fz = PSI && (fl & FL_PEZ);
     if (!UPD && !(fx || fy || fz))
@@ -101,7 +101,7 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
     const double x0 = at(Hx, q.o), xzm1 = at(Hb + zm1, q.o), xzp1 = at(Hb + zp1, q.o),
                  xzm2 = at(Hb + zm2, q.o);
     const double xym1 = at(Hx, q.ym1), xyp1 = at(Hx, q.yp1), xym2 = at(Hx, q.ym2);
-    double ex = at_s<NT>(Ein, q.o), ey = at_s<NT>(Ein + nb, q.o), ez = at_s<NT>(Ein + 2 * nb, q.o);
+    double ex = at(Ein, q.o), ey = at(Ein + nb, q.o), ez = at(Ein + 2 * nb, q.o);
     const double eps2 = at(cb(S.eps) + kp, q.o);
     const Quad X = quad<false>(S.prof[0], S.ix, i), Y = quad<false>(S.prof[1], S.iy, jj);
     const Quad Z = uquad<false>(S.cq[2], k);
@@ -199,29 +199,28 @@ __device__ __forceinline__ void efield_cell(const ShotDev &S, const double *H, i
             ez -= amp;
     }
     if (fx) {
-        put_s<NT>(mb(S.psi[0]) + b0, q0, px0);
-        put_s<NT>(mb(S.psi[0]) + L0 + b0, q0, px1);
+        put_s<false>(mb(S.psi[0]) + b0, q0, px0);
+        put_s<false>(mb(S.psi[0]) + L0 + b0, q0, px1);
     }
     if (fy) {
-        put_s<NT>(mb(S.psi[1]) + b1, q1, py0);
-        put_s<NT>(mb(S.psi[1]) + L1 + b1, q1, py1);
+        put_s<false>(mb(S.psi[1]) + b1, q1, py0);
+        put_s<false>(mb(S.psi[1]) + L1 + b1, q1, py1);
     }
     if (fz) {
-        put_s<NT>(mb(S.psi[2]) + b2, q.o, pz0);
-        put_s<NT>(mb(S.psi[2]) + L2 + b2, q.o, pz1);
+        put_s<false>(mb(S.psi[2]) + b2, q.o, pz0);
+        put_s<false>(mb(S.psi[2]) + L2 + b2, q.o, pz1);
     }
-    put_s<NT>(Eout, q.o, ex);
-    put_s<NT>(Eout + nb, q.o, ey);
-    put_s<NT>(Eout + 2 * nb, q.o, ez);
+    put_s<false>(Eout, q.o, ex);
+    put_s<false>(Eout + nb, q.o, ey);
+    put_s<false>(Eout + 2 * nb, q.o, ez);
 }
 
 // One cell of the H update + CPML-H corrections, general path, as efield_cell.
-// H is read from Hin and written to Hout (the same buffer when updated in place).
 template <int MODE>
-__device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin, double *Hout, int i,
-                                            int jj, int k, unsigned oc, int fl, int so, int sign)
+__device__ __forceinline__ void hfield_cell(const ShotDev &S, double *H, int i, int jj, int k,
+                                            unsigned oc, int fl, int so, int sign)
 {
-    constexpr bool NT = (MODE & M_NT) != 0, UPD = (MODE & M_UPD) != 0, PSI = (MODE & M_PSI) != 0;
+    constexpr bool UPD = (MODE & M_UPD) != 0, PSI = (MODE & M_PSI) != 0;
     const bool upx = UPD && (fl & FL_UHX), upy = UPD && (fl & FL_UHY), upz = UPD && (fl & FL_UHZ);
     const bool gx = PSI && (fl & FL_PHX), gy = PSI && (fl & FL_PHY), gz = PSI && (fl & FL_PHZ);
     if (!(upx || upy || upz || gx || gy || gz))
@@ -235,7 +234,7 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
     const size_t zp1 = k + 1 < S.iz ? kp + pb : kp, zp2 = k + 2 < S.iz ? kp + 2 * pb : kp;
     const gcp Eb = cb(S.e + (size_t)so * S.sstride), Ex = Eb + kp, Ey = Eb + nb + kp,
               Ez = Eb + 2 * nb + kp;
-    const gcp Hi = cb(Hin) + kp;
+    const gcp Hi = cb(H) + kp;
     const double z0 = at(Ez, q.o), zyp1 = at(Ez, q.yp1), zyp2 = at(Ez, q.yp2), zym1 = at(Ez, q.ym1);
     const double zxp1 = at(Ez, q.x, 8), zxp2 = at(Ez, q.x, 16), zxm1 = at(Ez, q.x, -8);
     const double y0 = at(Ey, q.o), yzp1 = at(Eb + nb + zp1, q.o), yzp2 = at(Eb + nb + zp2, q.o),
@@ -244,7 +243,7 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
     const double x0 = at(Ex, q.o), xzp1 = at(Eb + zp1, q.o), xzp2 = at(Eb + zp2, q.o),
                  xzm1 = at(Eb + zm1, q.o);
     const double xyp1 = at(Ex, q.yp1), xyp2 = at(Ex, q.yp2), xym1 = at(Ex, q.ym1);
-    double hx = at_s<NT>(Hi, q.o), hy = at_s<NT>(Hi + nb, q.o), hz = at_s<NT>(Hi + 2 * nb, q.o);
+    double hx = at(Hi, q.o), hy = at(Hi + nb, q.o), hz = at(Hi + 2 * nb, q.o);
     // eps' is only used where a magnetic CPML conductivity is nonzero; loading
     // it beside the conductivities rather than after them saves a round trip
     const double eps2 = at(cb(S.eps) + kp, q.o);
@@ -332,21 +331,21 @@ __device__ __forceinline__ void hfield_cell(const ShotDev &S, const double *Hin,
         hy -= dby * pz1;
     }
     if (gx) {
-        put_s<NT>(mb(S.psi[0]) + b0, q0, px0);
-        put_s<NT>(mb(S.psi[0]) + L0 + b0, q0, px1);
+        put_s<false>(mb(S.psi[0]) + b0, q0, px0);
+        put_s<false>(mb(S.psi[0]) + L0 + b0, q0, px1);
     }
     if (gy) {
-        put_s<NT>(mb(S.psi[1]) + b1, q1, py0);
-        put_s<NT>(mb(S.psi[1]) + L1 + b1, q1, py1);
+        put_s<false>(mb(S.psi[1]) + b1, q1, py0);
+        put_s<false>(mb(S.psi[1]) + L1 + b1, q1, py1);
     }
     if (gz) {
-        put_s<NT>(mb(S.psi[2]) + b2, q.o, pz0);
-        put_s<NT>(mb(S.psi[2]) + L2 + b2, q.o, pz1);
+        put_s<false>(mb(S.psi[2]) + b2, q.o, pz0);
+        put_s<false>(mb(S.psi[2]) + L2 + b2, q.o, pz1);
     }
-    const gmp Ho = mb(Hout) + kp;
-    put_s<NT>(Ho, q.o, hx);
-    put_s<NT>(Ho + nb, q.o, hy);
-    put_s<NT>(Ho + 2 * nb, q.o, hz);
+    const gmp Ho = mb(H) + kp;
+    put_s<false>(Ho, q.o, hx);
+    put_s<false>(Ho + nb, q.o, hy);
+    put_s<false>(Ho + 2 * nb, q.o, hz);
 }
 
 // Cell of this lane in the single operators: PT consecutive cells of a plane
@@ -385,7 +384,7 @@ __global__ __launch_bounds__(PT) void k_hfield(const ShotDev *__restrict__ D, in
     if (!plane_cell(S, blockIdx.x, i, jj, k, o))
         return;
     double *H = hsel(S, 0, 0);
-    hfield_cell<MODE>(S, H, H, i, jj, k, o, flags(S, i, jj, k), S.cur, sign);
+    hfield_cell<MODE>(S, H, i, jj, k, o, flags(S, i, jj, k), S.cur, sign);
 }
 
 // read_source_3d as a stand-alone operator (in place on the current slot)
@@ -2405,7 +2404,7 @@ __global__ __launch_bounds__(256) void k_hfield_p(const ShotDev *__restrict__ D,
     if (!__all(inner)) {
         double *H = hsel(S, 0, 0);
         for (int d = 0; d < 2; ++d)
-            hfield_cell<M_UPD | M_PSI>(S, H, H, i + d, jj, k, (unsigned)(jj * ix + i + d) * 8u,
+            hfield_cell<M_UPD | M_PSI>(S, H, i + d, jj, k, (unsigned)(jj * ix + i + d) * 8u,
                                        flags(S, i + d, jj, k), so, sign);
         return;
     }
