@@ -27,9 +27,9 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Gcell-updates/s + % HBM peak (256³ fp64); served shots/s, p50/p99 latency"
 HBM_PEAK_GBS = 8000.0
-# the launches that make up each timed half-step: the LDS family on large grids with
-# an odd row or with MITTET_FDTD_LDS=1 (takes_lds in fdtd_api.hip), else the per-cell
-# family alone
+# the launches that make up each timed half-step: the LDS family on large grids whose
+# rows 8 does not divide (and fill its columns) or with MITTET_FDTD_LDS=1 (takes_lds in
+# fdtd_api.hip), else the per-cell family alone
 LDS_MIN_CELLS = 12_000_000
 HALF_STEP_KERNELS = {
     "efield": "E half-step: k_efield_f (CPML-shell tiles) + k_efield_l (interior, LDS z-march)",
@@ -532,7 +532,7 @@ def main():
                    "sigma_sha256_16": configs.sigma_digest(wl.sigma)},
         "roofline": {"bound": "hbm",
                      "kernel": (FUSED_KERNELS if fused else
-                                HALF_STEP_KERNELS if g.ix % 2 and g.ncells >= LDS_MIN_CELLS
+                                HALF_STEP_KERNELS if g.ix % 8 and g.ncells >= LDS_MIN_CELLS
                                 or os.environ.get("MITTET_FDTD_LDS", "0") != "0"
                                 else HALF_STEP_KERNELS_PER_CELL).get(dom, dom),
                      "achieved": round(achieved, 1),

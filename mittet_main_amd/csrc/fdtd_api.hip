@@ -393,7 +393,10 @@ int tiles(int n, int t) { return (n + t - 1) / t; }
 // 216 / 155 ms per pass, 216^3 with a volume DFT 241 / 262 / 231 / 256 / 219), and so they are
 // in runs of launches that all but fill the Infinity Cache (kWideMinBytes: 152^3 25.4 /
 // 27.2 / 26.5 / 25.7 / 24.1); below, lanes count more (120^3 13.6 / 13.2 / 13.1 / 14.5 / 13.6,
-// 131 x 97 x 75 11.8 / 11.6 / 11.5 / 11.1 / 12.2).
+// 131 x 97 x 75 11.8 / 11.6 / 11.5 / 11.1 / 12.2).  Between 200 and 240 MiB, us a step with the
+// fewest idle lanes / 32 x 8: 152^3 140 / 124, 156^3 164 / 154, 154^3 148 / 142, 147x160x150 131 / 129,
+// 192x144x128 124 / 125, 176x152x140 139 / 140, 125x170x170 149 / 154, 240x128x120 132 / 143; with E in a
+// ring 134^3 137 / 128, 140^3 140 / 131, 160x128x125 110 / 110; at 182 MiB 144^3 98 / 105.
 void cell_tile(int ix, int iy, int &w, int &h)
 {
     double best = 0.0;
@@ -494,15 +497,23 @@ int lds_chunk(int ltx, int lty, int nz)
 }
 
 // Shots that take the LDS family (two interior and two shell launches a step instead of
-// two over whole planes).  Since the per-cell launches take their tiles in layers
-// (ftile) they are the faster ones, ms per pass LDS / per-cell: 136^3 23.4 / 18.1, 160^3
-// 36.1 / 29.1, 176^3 48.2 / 38.5, 240^3 32.6 / 29.6, 288^3 157.2 / 156.3, 400^3 128 / 125,
-// 216^3 with a volume DFT 222 / 220, 600x500x60 42.0 / 41.7, 60x500x600 65 / 51.  Left
-// are large grids with an odd row, whose 32-cell tiles straddle a cache line more on
-// every row: 301x240x250 48.0 / 52.2, 331x277x201 47.2 / 49.7, 243x251x260 43.6 / 46.2, 289^3
-// 66.0 / 66.8 (309^3 79.7 / 79.0, 349x300x200 56.7 / 54.6; below 12 M cells 217x219x221 28.9 /
-// 28.4, 151x149x147 8.0 / 7.2).  MITTET_FDTD_LDS=1 takes it on any grid.
+// two over whole planes): large grids whose rows 8 does not divide and whose interior
+// fills the 64-cell columns about as well as the rows fill 32-cell tiles.  Where rows
+// are whole half cache lines the per-cell launches with their tiles in layers (ftile) are
+// the faster ones, us a step LDS / per-cell: 256^3 630 / 590, 272^3 734 / 691, 304x240x250 669 /
+// 630, 320x320x160 601 / 563, 312x260x260 817 / 790, 296x260x260 799 / 816.  Where they are not,
+// the rows of a 32 x 8 tile start anywhere in a line and touch one more each, and the
+// LDS kernels, whose columns are wider and read a plane once, gain: 302x240x250 776 / 843,
+// 301x240x250 793 / 861, 330x277x201 767 / 807, 243x251x260 723 / 765, 250^3 690 / 721, 300x300x200
+// 762 / 791, 274^3 888 / 916, 401x301x151 760 / 816, 289^3 1097 / 1100, 310^3 1305 / 1275; not so with
+// idle lanes in the columns (kLdsFill): 350x300x200 926 / 885, 187x306x331 946 / 888.  On 28
+// grids of 12 to 40 M cells drawn to check this rule, CPMLs of 6 to 16 cells, the LDS family
+// takes 0.915 to 1.034 (mean 0.966) of the other's time where the rule takes it, and 0.95 to
+// 1.09 (mean 1.008) where it does not.  Below 12 M cells both signs: 210^3 418 / 439, 227x222x226
+// 539 / 596, but 201x200x200 389 / 379, 300x180x180 423 / 410, 180^3 278 / 256, 166^3 241 / 234.
+// MITTET_FDTD_LDS=1 takes it on any grid.
 constexpr long long kLdsMinCells = 12000000;
+constexpr double kLdsFill = 0.88;
 // ... and, with MITTET_FDTD_FUSE=1, those of at least so many cells (takes_fused)
 constexpr long long kFuseMinCells = 2500000;
 
@@ -515,6 +526,13 @@ constexpr long long kWideMinBytes = 200LL << 20;
 // with one slot), H, and the two coefficient arrays.
 long long step_bytes(long long cells, long long ring) { return cells * (ring > 1 ? 88 : 64); }
 
+// Lanes in use of the LDS kernels' 64-cell columns over those of 32-cell tiles
+double lds_fill(int ix, int xlo, int xhi)
+{
+    const double cols = (double)(xhi - xlo) / (mt::LX * tiles(xhi - xlo, mt::LX));
+    return cols / ((double)ix / (mt::ZX * tiles(ix, mt::ZX)));
+}
+
 // Whether a C-variant shot takes the LDS family (family 3): size, no z-chunk
 // or x-pair override, and a CPML-free interior to march.
 bool takes_lds(const fwi3d_grid_params &p, int zchunk)
@@ -522,7 +540,8 @@ bool takes_lds(const fwi3d_grid_params &p, int zchunk)
     const long long N = (long long)p.ix * p.iy * p.iz;
     const int xlo = (p.ncpml + 15) / 16 * 16;
     const bool pair = p.ix % 2 == 0 && env_pad("MITTET_FDTD_PAIR", 0);
-    const bool lds_size = (p.ix % 2 && N >= kLdsMinCells) || env_pad("MITTET_FDTD_LDS", 0) ||
+    const bool lds_size = (p.ix % 8 && N >= kLdsMinCells && xlo < p.ix - p.ncpml &&
+                           lds_fill(p.ix, xlo, p.ix - p.ncpml) >= kLdsFill) || env_pad("MITTET_FDTD_LDS", 0) ||
                           (N >= kFuseMinCells && env_pad("MITTET_FDTD_FUSE", 0));
     return zchunk == 0 && !pair && lds_size && p.ncpml >= 2 && xlo < p.ix - p.ncpml &&
            p.ncpml < p.iy - p.ncpml && p.ncpml < p.iz - p.ncpml && !env_pad("MITTET_FDTD_NOLDS", 0);
@@ -1413,11 +1432,14 @@ long long step_touch_bytes(const fwi3d_shot *s) { return step_bytes(s->desc.n, s
 // Non-temporal field traffic and tiles in layers pay once a launch's fields no longer
 // stay in the 256 MB Infinity Cache from one half-step to the next: then L2 and that
 // cache keep the stencil neighbours that other tiles still read.  Single shots with a
-// 12-cell CPML, 64 B per cell, ms per pass without / with: 120^3 13.2 / 16.8, 144^3 (182
-// MiB) 19.9 / 22.4, 152^3 (214 MiB) 24.1 / 29.1, 160^3 (250 MiB) 32.6 / 29.1, 176^3 44.2 /
-// 38.5, 192^3 59.6 / 50.0, 288^3 176 / 155; with a 4-frequency volume DFT, 88 B per cell:
-// 128^3 (176 MiB) 21.6 / 23.5, 144^3 (251 MiB) 31.3 / 32.2, 152^3 39.3 / 37.4, 216^3 236 / 220.
-// Four shots of 84^3 to 120^3 (264 MiB) 40.1 / 33.8.  MITTET_FDTD_NT=0 or 1 overrides.
+// 12-cell CPML, us a step without / with, 64 B per cell: 148^3 (198 MiB) 117 / 144, 154^3 (223)
+// 139 / 159, 156^3 (232) 156 / 159, 158^3 (241) 170 / 170, 176x152x150 (245) 158 / 148, 125x180x180
+// (247) 189 / 193, 160^3 (250) 162 / 148, 168^3 (289) 244 / 212; with a 4-frequency volume DFT, 88 B
+// per cell: 140^3 (230) 135 / 148, 142^3 (240) 148 / 157, 96x192x160 (248) 140 / 137, 144^3 (251) 145 /
+// 141, 160x140x135 (254) 142 / 135, 146^3 (261) 161 / 161, 152^3 (295) 181 / 165.  288^3 176 / 155 ms per
+// pass, 216^3 with the DFT 236 / 220.  Four shots of 84^3 to 120^3 (264 MiB) 40.1 / 33.8 ms.
+// MITTET_FDTD_NT=0 or 1 overrides (read where launches are captured into a graph, per
+// call for the others).
 bool stream_nt(long long touch_bytes)
 {
     const long long e = env_pad("MITTET_FDTD_NT", -1);

@@ -1159,9 +1159,8 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // values), so a cell costs 4 loads there instead of 15, and its values wait in
 // LDS instead of registers; the z neighbours, which no other lane of the block
 // needs, are loaded directly.  All loads of a block are issued before its one
-// barrier.  What bounds them: above 2.5 M cells, where they take the CPML
-// shells, and for batches beyond the Infinity Cache, memory (5 TB/s on their own
-// bytes at 288^3); on grids that fit that cache a plain copy of the same bytes
+// barrier.  What bounds them: on grids and batches beyond the Infinity Cache (and as
+// the LDS family's CPML shells) memory (5.8 TB/s on their own bytes at 288^3); on grids that fit that cache a plain copy of the same bytes
 // reaches 6.5 TB/s plus 3 us a launch, and these kernels 60-75 % of that, held
 // back by the instructions a wave issues around its one round trip.  Against
 // the same per-cell code with every stencil value loaded by its own lane

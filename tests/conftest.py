@@ -30,7 +30,8 @@ def hip_lib():
 
 @pytest.fixture(autouse=True)
 def _lds_family_on_small_grids(monkeypatch):
-    """The library takes the LDS kernel family only from 2.5 M cells up; the
-    parity tests run on small grids, so they force it there (tests of the
-    size-based choice itself remove the variable)."""
+    """The library takes the LDS kernel family only from 12 M cells up, on rows that
+    8 does not divide (the adjoint's from 3 M); the parity tests run on small
+    grids, so they force it there (tests of the size-based choice itself remove
+    the variable)."""
     monkeypatch.setenv("MITTET_FDTD_LDS", "1")

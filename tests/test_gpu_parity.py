@@ -162,8 +162,8 @@ def test_laplace_to_freq_vs_oracle():
 def test_batch_mixed_sizes_equal_alone(families, monkeypatch):
     """Shots of different grid sizes in one persistent launch give the same
     bits as each run alone; one joins mid-way (continuous batching).  "mixed":
-    the second shot runs the per-cell family alone (as grids below 2.5 M cells
-    do), the others the LDS family, in the same launches.  "lds-nt": the
+    the second shot runs the per-cell family alone (as most grids do by
+    default), the others the LDS family, in the same launches.  "lds-nt": the
     batch launches load and store non-temporally (MITTET_FDTD_NT=1), the
     lone runs do not."""
     monkeypatch.setenv("MITTET_FDTD_NT", "0")
