@@ -444,7 +444,9 @@ __global__ void k_receivers(const ShotDev *__restrict__ D, int j, int nover, int
 // 2.11 ms (5.5), 245 us and 2.34 ms with the components one after the other in a block, four
 // samples loaded and then summed, and weights in LDS (32 KB a block).  Two, four or
 // eight samples ahead: 186, 189, 193 us and 2.23, 2.33, 2.40 ms; with plain loads and
-// stores 221 us; two or three blocks a CU instead of four 272 or 217 us.
+// stores 221 us; two or three blocks a CU instead of four 272 or 217 us.  (The 16 KB of
+// LDS a block that the kernel is compiled with are flush_cell_any's accumulators, which
+// the compiler puts there; at four blocks a CU they cost nothing.)
 constexpr int FLUSH_NF_MAX = 8, FLUSH_G = 2;
 
 template <int V> struct Cells;
@@ -1183,8 +1185,9 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // the slot this step reads.  With one slot, E is overwritten by that launch, so
 // the H launch of the step itself gathers E.  The samples are the ones a
 // receiver launch after the step takes.  hf: the step is a fused E+H launch
-// sequence (H before step j is hsel(S, j, 1)).
-template <bool NT>
+// sequence (H before step j is hsel(S, j, 1)).  MANY: a launch over several shots,
+// whose members may have finished; they look the step up before their loads.
+template <bool NT, bool MANY>
 __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, int ns,
                                                  const int *__restrict__ pre, int j, int recn, int rec_e,
                                                  int hf)
@@ -1200,12 +1203,12 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
         return;
     }
     const int b = blockIdx.x - recn;
-    const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
+    const int s = MANY ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
     FTile T;
-    if (!ftile<NT>(S, ns > 1 ? b - pre[s] : b, T))
+    if (!ftile<NT>(S, MANY ? b - pre[s] : b, T))
         return;   // uniform over the block
-    if (ns > 1 && chunk_step(S) + j >= S.it - 1)
+    if (MANY && chunk_step(S) + j >= S.it - 1)
         return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
@@ -1379,7 +1382,7 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     put_s<NT>(Eout + 2 * nb, q.o, ez);
 }
 
-template <bool NT>
+template <bool NT, bool MANY>
 __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, int ns,
                                                  const int *__restrict__ pre, int j, int recn, int hf)
 {
@@ -1394,12 +1397,12 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
         return;
     }
     const int b = blockIdx.x - recn;
-    const int s = ns > 1 ? find_shot(pre, ns, b) : 0;
+    const int s = MANY ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
     FTile T;
-    if (!ftile<NT>(S, ns > 1 ? b - pre[s] : b, T))
+    if (!ftile<NT>(S, MANY ? b - pre[s] : b, T))
         return;   // uniform over the block
-    if (ns > 1 && chunk_step(S) + j >= S.it - 1)
+    if (MANY && chunk_step(S) + j >= S.it - 1)
         return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
@@ -1576,12 +1579,9 @@ hipError_t launch_efield_f(const ShotDev *d, int ns, const int *pre, int nblocks
     if (nblocks <= 0)
         return rec_prev ? hipErrorInvalidValue : hipSuccess;
     const int recn = rec_blocks(rec_prev && j > 0, ns);
-    if (nt)
-        hipLaunchKernelGGL(k_efield_f<true>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn,
-                           rec_e ? 1 : 0, hf);
-    else
-        hipLaunchKernelGGL(k_efield_f<false>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn,
-                           rec_e ? 1 : 0, hf);
+    const auto k = ns > 1 ? (nt ? k_efield_f<true, true> : k_efield_f<false, true>)
+                          : (nt ? k_efield_f<true, false> : k_efield_f<false, false>);
+    hipLaunchKernelGGL(k, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, rec_e ? 1 : 0, hf);
     return hipGetLastError();
 }
 
@@ -1591,10 +1591,9 @@ hipError_t launch_hfield_f(const ShotDev *d, int ns, const int *pre, int nblocks
     if (nblocks <= 0)
         return rec_e ? hipErrorInvalidValue : hipSuccess;
     const int recn = rec_blocks(rec_e, ns);
-    if (nt)
-        hipLaunchKernelGGL(k_hfield_f<true>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
-    else
-        hipLaunchKernelGGL(k_hfield_f<false>, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
+    const auto k = ns > 1 ? (nt ? k_hfield_f<true, true> : k_hfield_f<false, true>)
+                          : (nt ? k_hfield_f<true, false> : k_hfield_f<false, false>);
+    hipLaunchKernelGGL(k, dim3(recn + nblocks), dim3(PT), 0, st, d, ns, pre, j, recn, hf);
     return hipGetLastError();
 }
 
