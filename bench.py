@@ -67,7 +67,7 @@ def measured_traffic(workload, ring, kernel):
     with open(path) as f:
         rec = json.load(f)
     src = b"".join(open(os.path.join(ROOT, "mittet_main_amd", "csrc", n), "rb").read()
-                   for n in ("fdtd_kernels.hip", "fdtd_dev.h"))
+                   for n in ("fdtd_kernels.hip", "fdtd_dev.h", "fdtd_tile.h"))
     if rec.get("ring") != ring or rec.get("sources_sha256_16") != hashlib.sha256(src).hexdigest()[:16]:
         return None
     k = rec["kernels"].get(kernel)

@@ -156,7 +156,11 @@ int fwi3d_shot_destroy(fwi3d_shot *s);
 /* Fortran variant: one more Hz source point with the shot's waveform (the
  * second transmitter of ver0040/cpu_waveform.f90:49-51); at most 4 points. */
 int fwi3d_shot_add_source(fwi3d_shot *s, int i, int j, int k);
-/* device bytes this shot would allocate (admission control) */
+/* device bytes this shot would allocate (admission control).  Not counted: the
+ * memory of its spectrum requests (fwi3d_receiver_dft, fwi3d_laplace_to_freq,
+ * fwi3d_laplace_fft), which the shot keeps from the first to its end where a
+ * request needs up to 4 MiB (8 bytes times nfreq + 12 nrec nfreq, for
+ * laplace_to_freq also the two waveforms), and else frees after the call. */
 long long fwi3d_shot_bytes(const fwi3d_grid_params *p, const fwi3d_shot_params *sp);
 
 /* satan_i/fwi3d_cpu_function_v1.4.c:964-986 (+ traces, DFT accumulators, step counter) */
@@ -209,7 +213,10 @@ int fwi3d_get_field(fwi3d_shot *s, int which, double *out);
 int fwi3d_set_field(fwi3d_shot *s, int which, const double *in);
 /* traces: [6][nrec][it] doubles, E then H, sample n = after step n */
 int fwi3d_get_traces(fwi3d_shot *s, double *out);
-/* volume E spectra: complex [3][nf_vol][ix*iy*iz] = sum_n E[n]*w_n(omega) */
+/* volume E spectra: complex [3][nf_vol][ix*iy*iz] = sum_n E[n]*w_n(omega).  From
+ * 32 MiB up into pageable memory, through pinned pieces and up to 8 host threads
+ * for the length of the call; the model keeps the pinned memory (at most 32 MiB
+ * of host memory) until it is destroyed. */
 int fwi3d_get_volume_dft(fwi3d_shot *s, double *out);
 /* Volume H spectra at the shot's nf_vol frequencies, sum_n H[n]*w_n(omega)
  * with H after step n (the sample of the H traces).  The reference transforms

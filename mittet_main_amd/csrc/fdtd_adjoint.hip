@@ -49,6 +49,11 @@
 // for cells that only a psi correction changes (ca = 1) as well, and with
 // Km = msig dt/2, r = 1/(e + Km)
 //   dda/de H - ddb/de X = (Km r/e) (H' + H)   (H' - H where only psi acts).
+// E' - E cancels where the field changes little in a step.  Its rounding is that of E, as
+// large as that of the curl it stands for while the field is a wave (cb |H| / dl is about
+// |E| / 2).  Against 64-bit values the gradient's relative error is 6.4e-15 at 152^3 with 200
+// steps (5.8e-15 with the stencils) and 1.3e-15 at 61 x 50 x 44 with 160 (1.4e-15), and in one
+// dimension 2.9e-15 after 16 000 steps (2.2e-15).
 #include "fdtd_tile.h"
 
 namespace mt {
