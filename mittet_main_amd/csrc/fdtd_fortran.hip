@@ -113,10 +113,11 @@ __global__ __launch_bounds__(PT) void k_efield_v(const ShotDev *__restrict__ D, 
     const int b = blockIdx.x - recn;
     const int s = MANY ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
+    const int nm = MANY ? chunk_step(S) + j : 0;
     FTile T;
     if (!ftile<false>(S, MANY ? b - pre[s] : b, T))
         return;   // uniform over the block
-    if (MANY && chunk_step(S) + j >= S.it - 1)
+    if (MANY && nm >= S.it - 1)
         return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc, ix = S.ix, iy = S.iy, iz = S.iz;
     const bool ax = T.x0 < nc || T.x0 + T.w > ix - nc, ay = T.y0 < nc || T.y0 + T.h > iy - nc;
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(PT) void k_efield_v(const ShotDev *__restrict__ D, 
         az0 = at(P2, q.o);
         az1 = at(P2 + L2, q.o);
     }
-    const int n = chunk_step(S) + j;
+    const int n = MANY ? nm : chunk_step(S) + j;
     if (!MANY && n >= S.it - 1)
         return;   // uniform over the block
     if (hz_plane(S, k)) {
@@ -273,10 +274,11 @@ __global__ __launch_bounds__(PT) void k_hfield_v(const ShotDev *__restrict__ D, 
     const int b = blockIdx.x - recn;
     const int s = MANY ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
+    const int nm = MANY ? chunk_step(S) + j : 0;
     FTile T;
     if (!ftile<false>(S, MANY ? b - pre[s] : b, T))
         return;   // uniform over the block
-    if (MANY && chunk_step(S) + j >= S.it - 1)
+    if (MANY && nm >= S.it - 1)
         return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc, ix = S.ix, iy = S.iy, iz = S.iz;
     const bool ax = T.x0 < nc || T.x0 + T.w > ix - nc, ay = T.y0 < nc || T.y0 + T.h > iy - nc;
@@ -341,7 +343,7 @@ __global__ __launch_bounds__(PT) void k_hfield_v(const ShotDev *__restrict__ D, 
         lds_put(sh, q.ha + (unsigned)hc * (PT_TILE * 8u), hv);
     __syncthreads();
     // the step is looked up behind the loads
-    const int n = chunk_step(S) + j;
+    const int n = MANY ? nm : chunk_step(S) + j;
     if (n >= S.it - 1 || !q.own || q.i >= ix || q.jj >= iy)
         return;
     if (hz_plane(S, k))

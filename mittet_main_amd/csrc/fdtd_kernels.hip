@@ -1205,10 +1205,11 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     const int b = blockIdx.x - recn;
     const int s = MANY ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
+    const int nm = MANY ? chunk_step(S) + j : 0;
     FTile T;
     if (!ftile<NT>(S, MANY ? b - pre[s] : b, T))
         return;   // uniform over the block
-    if (MANY && chunk_step(S) + j >= S.it - 1)
+    if (MANY && nm >= S.it - 1)
         return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
@@ -1286,7 +1287,7 @@ __global__ __launch_bounds__(PT) void k_efield_f(const ShotDev *__restrict__ D, 
     __syncthreads();
     // a lone shot's step is looked up behind the loads (it costs two dependent
     // scalar loads), only for the source: its launches end with its time loop
-    const int n = chunk_step(S) + j;
+    const int n = MANY ? nm : chunk_step(S) + j;
     if (n >= S.it - 1 || !q.own || q.i >= S.ix || q.jj >= T.yend)
         return;
     if (T.region && q.i >= S.lo[0] && q.i < S.hi[0] && q.jj >= S.lo[1] && q.jj < S.hi[1])
@@ -1399,10 +1400,11 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     const int b = blockIdx.x - recn;
     const int s = MANY ? find_shot(pre, ns, b) : 0;
     const ShotDev &S = D[s];
+    const int nm = MANY ? chunk_step(S) + j : 0;
     FTile T;
     if (!ftile<NT>(S, MANY ? b - pre[s] : b, T))
         return;   // uniform over the block
-    if (MANY && chunk_step(S) + j >= S.it - 1)
+    if (MANY && nm >= S.it - 1)
         return;   // a member of a batch that has finished its time loop loads nothing
     const int k = T.k, nc = S.nc;
     const bool ax = T.x0 < nc || T.x0 + T.w > S.ix - nc, ay = T.y0 < nc || T.y0 + T.h > S.iy - nc;
@@ -1481,7 +1483,7 @@ __global__ __launch_bounds__(PT) void k_hfield_f(const ShotDev *__restrict__ D, 
     __syncthreads();
     // a lone shot's step is looked up behind the loads: its launches end with its
     // time loop
-    const int n = chunk_step(S) + j;
+    const int n = MANY ? nm : chunk_step(S) + j;
     if (n >= S.it - 1 || !q.own || q.i >= S.ix || q.jj >= T.yend)
         return;
     if (T.region && q.i >= S.lo[0] && q.i < S.hi[0] && q.jj >= S.lo[1] && q.jj < S.hi[1])
