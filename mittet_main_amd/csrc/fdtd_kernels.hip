@@ -1162,7 +1162,8 @@ hipError_t launch_hfield_z(const ShotDev *d, int ns, const int *pre, int nblocks
 // LDS instead of registers; the z neighbours, which no other lane of the block
 // needs, are loaded directly.  All loads of a block are issued before its one
 // barrier.  What bounds them: on grids and batches beyond the Infinity Cache (and as
-// the LDS family's CPML shells) memory (5.8 TB/s on their own bytes at 288^3); on grids that fit that cache a plain copy of the same bytes
+// the LDS family's CPML shells) memory (288^3: 5.6 to 5.9 TB/s at the L2's memory side,
+// 1.07 times their own bytes); on grids that fit that cache a plain copy of the same bytes
 // reaches 6.5 TB/s plus 3 us a launch, and these kernels 60-75 % of that, held
 // back by the instructions a wave issues around its one round trip.  Against
 // the same per-cell code with every stencil value loaded by its own lane
