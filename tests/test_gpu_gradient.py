@@ -171,9 +171,9 @@ def test_odd_cell_count_gradient():
 
 
 def test_gradient_with_the_x_pair_forward_family(monkeypatch):
-    """The replays of the LDS and per-cell forward families write E, H and
-    psi straight into the stored states; other families update H and psi in
-    place and copy them into each state.  With the x-pair family
+    """The replays of the LDS and per-cell forward families write E and H
+    straight into the stored states (psi stays in the shot); other families
+    update H in place and copy it into each state.  With the x-pair family
     (MITTET_FDTD_PAIR=1) the gradient is bitwise that of the default family:
     the forward is bitwise the same and the adjoint kernels are shared."""
     print("gradient: x-pair forward family vs default, 26 x 24 x 22", flush=True)
